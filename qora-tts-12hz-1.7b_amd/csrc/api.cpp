@@ -371,23 +371,75 @@ void mfma_plan(int K, int *sw, int *kc) {
     *kc = (Ks + 4 * s - 1) / (4 * s);
 }
 
+// Rows past kMfmaPassRows run in row blocks (k_gemm_mfma_tile), at most
+// kTileMaxRows rows per launch (which bounds the split rows' scratch).
+constexpr int kMfmaPassRows = 64;
+constexpr int kTileMaxRows = 4096;
+
+// The block shape and K chunks of a product of M rows: the least estimated
+// time over 32-row tiles (mt) x panels (nw) per block and K chunks.  Measured
+// per 32-row K stage: `alone`, one block on a CU (issue and latency), and
+// `loaded`, each block of a CU that has several (operand reads through the
+// L2).  A block of 4 x 8 reads the rows half as often as 4 x 4: 1064 rows,
+// 2048 -> 12288, 180 against 192 us.  Few row and column blocks take K
+// chunks, each a partial written and read once: 1000 rows, 6144 -> 2048,
+// 161 us with one chunk, 113 with four.
+GemmTilePlan tile_plan(int M, int K, int N) {
+    struct Shape {
+        int mt, nw;
+        double alone, loaded;  // us per stage
+    };
+    constexpr Shape shapes[] = {{1, 4, 0.35, 0.28}, {2, 4, 0.42, 0.43}, {3, 4, 0.47, 0.63}, {4, 4, 0.55, 0.83},
+                                {4, 8, 1.00, 1.30}};
+    const int tiles = (M + 31) / 32, Ks = K / 16;
+    GemmTilePlan best{};
+    double best_us = 0.0;
+    for (const Shape &h : shapes)
+        for (int kc = 1; kc <= 16; kc++) {
+            GemmTilePlan t{};
+            t.mt = h.mt;
+            t.nw = h.nw;
+            t.mb = (tiles + h.mt - 1) / h.mt;
+            t.nb = (N / 32 + h.nw - 1) / h.nw;
+            t.cs = ((Ks + kc - 1) / kc + 1) / 2 * 2;
+            t.kc = (Ks + t.cs - 1) / t.cs;
+            if (t.kc != kc || (kc > 1 && t.cs < 8)) continue;
+            const long long blocks = (long long)t.mb * t.nb * t.kc;
+            if (kc > 1 && (blocks > 1024 || t.mb * t.nb > kCounters)) break;
+            const double x = (double)blocks / 256.0, deep = x <= 2.0 ? ceil(x) : x + 0.35;
+            const double mb = (double)blocks * h.mt * h.nw * 4096e-6;
+            const double us = t.cs / 2 * std::max(h.alone, h.loaded * deep) + (kc > 1 ? 5.0 + 0.4 * mb : 0.0);
+            if (best_us == 0.0 || us < best_us) best_us = us, best = t;
+        }
+    return best;
+}
+
+size_t tile_part_floats(const GemmTilePlan &t) {
+    return t.kc > 1 ? (size_t)t.mb * t.nb * t.kc * (size_t)(t.nw * t.mt * 1024) : 0;
+}
+
 // Grows the MFMA GEMM scratch for a K x N weight at up to M rows, so that a
 // later call allocates nothing (e.g. under stream capture).
 qtts_status mfma_reserve(qtts_ctx *c, int K, int N, int M) {
     int sw, kc;
     mfma_plan(K, &sw, &kc);
-    const int Mpad = M > 32 ? 64 : 32;
-    QTTS_TRY(grow(c, &c->mfma_x, &c->mfma_x_cap, (size_t)2 * 64 * K + 2 * 64));
-    if (kc > 1) QTTS_TRY(grow(c, &c->mfma_part, &c->mfma_part_cap, (size_t)kc * Mpad * N));
-    return QTTS_OK;
+    size_t rows = 64, part = kc > 1 ? (size_t)kc * (M > 32 ? 64 : 32) * N : 0;
+    if (M > kMfmaPassRows) {
+        const GemmTilePlan t = tile_plan(M < kTileMaxRows ? M : kTileMaxRows, K, N);
+        rows = std::max(rows, (size_t)32 * t.mt * t.mb);
+        part = std::max(part, tile_part_floats(t));
+    }
+    QTTS_TRY(grow(c, &c->mfma_x, &c->mfma_x_cap, 2 * rows * K + 2 * rows));
+    return grow(c, &c->mfma_part, &c->mfma_part_cap, part);
 }
 
 // y[m] (+)= f(x[m]) . W (+ bias) for M rows on the matrix cores
-// (csrc/mfma.hip), f the row prologue (MfmaRowsMode), 64 rows per pass: the
-// prologue and binary16 split, then one block per (panel, K chunk) of
-// 4 * sw 16-row steps, and the last block of a panel sums its chunks.  sw is
-// 8 (each wave keeps 8 steps of operand loads in flight; measured fastest at
-// every talker shape, 64 rows) unless K is short.
+// (csrc/mfma.hip), f the row prologue (MfmaRowsMode): the prologue and
+// binary16 split, then the product.  Up to kMfmaPassRows rows: one block per
+// (panel, K chunk) of 4 * sw 16-row steps, and the last block of a panel sums
+// its chunks; sw is 8 (each wave keeps 8 steps of operand loads in flight;
+// measured fastest at every talker shape, 64 rows) unless K is short.  More
+// rows: row blocks by tile_plan.
 qtts_status run_gemm_mfma(qtts_ctx *c, const DevQ4Mfma &w, const float *x, int M, int ldx, int mode,
                           const uint16_t *gamma, float *y, int ldy, const float *bias, bool accumulate,
                           float *norm_out = nullptr, int ldn = 0) {
@@ -395,13 +447,17 @@ qtts_status run_gemm_mfma(qtts_ctx *c, const DevQ4Mfma &w, const float *x, int M
     if (K % 16 || N % 32 || K > kMfmaRowsMaxK || ldx % 4 || ((uintptr_t)x & 15))
         return fail(c, QTTS_ESHAPE, "MFMA GEMM: unsupported shape or unaligned rows");
     if (panels > kCounters) return fail(c, QTTS_ESHAPE, "MFMA GEMM: more panels than counters");
-    int sw, kc;
-    mfma_plan(K, &sw, &kc);
-    for (int r0 = 0; r0 < M; r0 += 64) {
-        const int Mc = M - r0 < 64 ? M - r0 : 64;
-        const int mt = Mc > 32 ? 2 : 1, Mpad = 32 * mt;
-        QTTS_TRY(grow(c, &c->mfma_x, &c->mfma_x_cap, (size_t)2 * 64 * K + 2 * 64));
-        if (kc > 1) QTTS_TRY(grow(c, &c->mfma_part, &c->mfma_part_cap, (size_t)kc * Mpad * N));
+    for (int r0 = 0; r0 < M; r0 += kTileMaxRows) {
+        const int Mc = M - r0 < kTileMaxRows ? M - r0 : kTileMaxRows;
+        const bool tiled = Mc > kMfmaPassRows;
+        GemmTilePlan t{};
+        int sw = 0, kc = 0;
+        if (tiled)
+            t = tile_plan(Mc, K, N);
+        else
+            mfma_plan(K, &sw, &kc);
+        const int mt = Mc > 32 ? 2 : 1, Mpad = tiled ? 32 * t.mt * t.mb : 32 * mt;
+        QTTS_TRY(mfma_reserve(c, K, N, Mc));
         MfmaRowsParams r{};
         r.x = x + (size_t)r0 * ldx;
         r.ldx = ldx;
@@ -412,7 +468,7 @@ qtts_status run_gemm_mfma(qtts_ctx *c, const DevQ4Mfma &w, const float *x, int M
         r.gamma = gamma;
         r.xh = c->mfma_x;
         r.xl = c->mfma_x + (size_t)Mpad * K;
-        r.rexp = reinterpret_cast<int *>(c->mfma_x + (size_t)2 * 64 * K);
+        r.rexp = reinterpret_cast<int *>(c->mfma_x + (size_t)2 * Mpad * K);
         r.norm_out = norm_out ? norm_out + (size_t)r0 * ldn : nullptr;
         r.ldn = ldn;
         launch_mfma_rows(c->stream, r);
@@ -429,7 +485,10 @@ qtts_status run_gemm_mfma(qtts_ctx *c, const DevQ4Mfma &w, const float *x, int M
         p.y = y + (size_t)r0 * ldy;
         p.ldy = ldy;
         p.accumulate = accumulate ? 1 : 0;
-        launch_gemm_mfma(c->stream, p, mt, sw, kc);
+        if (tiled)
+            launch_gemm_mfma_tile(c->stream, p, t);
+        else
+            launch_gemm_mfma(c->stream, p, mt, sw, kc);
         QTTS_TRY(check_launch(c, "k_gemm_mfma"));
     }
     return QTTS_OK;

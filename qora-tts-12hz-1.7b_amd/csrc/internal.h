@@ -32,7 +32,8 @@ struct DevQ4 {
 //     4*(i/2) + 16*(i%2) -- rows 2j and 2j+1 are the two halves of
 //     (word >> 4j) & 0x000F000F;
 //   sa[p*K + k], sb[p*K + k]: the row's binary16 scale split exactly into
-//     its top 7 and low 4 significand bits (s = sa + sb).
+//     itself rounded to 7 significand bits (truncated where 8 * sa would pass
+//     binary16) and the rest, at most 4 bits (s = sa + sb).
 struct DevQ4Mfma {
     const uint32_t *wm;
     const uint16_t *sa, *sb;
@@ -149,6 +150,17 @@ struct GemmMfmaParams {
     const float *bias;        // optional
     float *y;                 // y[m * ldy + n] (+)= result
     int ldy, accumulate;
+};
+
+// The same product in row blocks of 32 * mt rows (k_gemm_mfma_tile), for
+// more rows than one pass of k_gemm_mfma takes.
+struct GemmTilePlan {
+    int mt;  // 32-row tiles per block
+    int mb;  // row blocks; xh / xl / rexp hold 32 * mt * mb rows (zero past M)
+    int nw;  // panels (waves) per block: 4 or 8
+    int nb;  // blocks of nw panels
+    int kc;  // K chunks, each of cs 16-row steps (an even number)
+    int cs;
 };
 
 constexpr int kGemvThreads = 256;
@@ -348,6 +360,8 @@ void launch_dec_conv_repack(hipStream_t st, const float *w, long long sm, long l
                             int taps, int cin16, int mtiles, int ksteps, int ew, _Float16 *wh, _Float16 *wl);
 void launch_dec_conv_mfma(hipStream_t st, const DecConvMfmaParams &p);
 void launch_gemm_mfma(hipStream_t st, const GemmMfmaParams &p, int mt, int sw, int kc);
+// part: [mb * nb * kc][32 * mt * 32 * nw] when kc > 1; counters: mb * nb, zero between launches
+void launch_gemm_mfma_tile(hipStream_t st, const GemmMfmaParams &p, const GemmTilePlan &t);
 void launch_embed_sum(hipStream_t st, const EmbSumParams &p);
 void launch_advance(hipStream_t st, LoopState *s, int frame_step, int batch = 1);
 // Prompt rows of prefill_custom_voice: out[r] = a[r] (+ b[r] when b[r] is

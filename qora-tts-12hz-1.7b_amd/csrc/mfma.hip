@@ -6,13 +6,13 @@
 // Exactness.  The reference forms every term as f32(f32(s)*x)*(nib-8) and
 // sums in f32.  Here each term is (xh + xl) * (sa*q + sb*q) with
 //   q = nib - 8 in [-8, 7], exact in binary16;
-//   s = sa + sb, sa keeping the top 7 significand bits of the binary16 scale
-//     and sb the low 4, so sa*q and sb*q are exact binary16 products
+//   s = sa + sb, sa the binary16 scale rounded to 7 significand bits and sb
+//     the rest (at most 4 bits), so sa*q and sb*q are exact binary16 products
 //     (formed with v_pk_mul_f16);
 //   x = xh + xl, xh = f16(x), xl = f16(x - xh): |x - xh - xl| <= 2^-22 |x|.
 // Products of binary16 values are exact in the f32 accumulator, and the
-// xl*sb*q term (relative size 2^-18) is dropped, so every term carries a
-// relative error of ~2^-18 or less before the f32 sums -- the f32 level the
+// xl*sb*q term (relative size 2^-19) is dropped, so every term carries a
+// relative error of ~2^-19 or less before the f32 sums -- the f32 level the
 // parity tolerance is set for.
 #include <hip/hip_runtime.h>
 
@@ -56,7 +56,10 @@ __global__ void k_repack_mfma(DevQ4 w, uint32_t *wm, uint16_t *sa, uint16_t *sb,
     if (idx < nrows) {
         const uint16_t s = w.ws[idx];
         if (fabsf((float)__builtin_bit_cast(_Float16, s)) > 8188.0f) atomicOr(too_large, 1);
-        const uint16_t hi = s & 0xFFF0u;  // top 7 significand bits (sign and exponent kept)
+        // top 7 significand bits, rounded to nearest unless that could
+        // overflow sa * q (then truncated)
+        uint16_t hi = (uint16_t)(s + 8u) & 0xFFF0u;
+        if (fabsf((float)__builtin_bit_cast(_Float16, hi)) > 8128.0f) hi = s & 0xFFF0u;
         sa[idx] = hi;
         const float d = (float)__builtin_bit_cast(_Float16, s) - (float)__builtin_bit_cast(_Float16, hi);
         sb[idx] = __builtin_bit_cast(uint16_t, (_Float16)d);  // exact
@@ -322,6 +325,210 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     }
 }
 
+// The same product for many rows.  A block of NW waves owns 32 * MT rows x NW
+// panels: wave w takes panel NW * n + w and all MT row tiles, so the nibbles
+// become B operands once per wave and are used by 3 * MT MFMAs, and the
+// block's A operands go through LDS once for its NW panels (two 16-row steps
+// per stage, double buffered).  Loads run two stages ahead, and everything
+// that is not an MFMA is issued between MFMAs.  Bound by the rows' operands
+// from the L2: 1064 rows, 2048 -> 12288, take 180 us, 297 TFLOP/s (892 of
+// binary16 MFMAs issued; a library binary16 product with as many MFMAs takes
+// 181), where 17 passes of k_gemm_mfma took 410; 1000 rows, 6144 -> 2048, 342
+// -> 113 us.
+template <int MT, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void k_gemm_mfma_tile(GemmMfmaParams P, GemmTilePlan T) {
+    constexpr int SS = 2;  // 16-row steps per stage
+    constexpr int U = SS * MT * 2;  // 1 KiB operand units per stage
+    constexpr int UW = U / NW;
+    __shared__ __align__(16) half8 abuf[2][U][64];
+    __shared__ int s_last;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int half = lane >> 5, col = lane & 31;
+    // Blocks of one XCD (every 8th) take a contiguous run of (column block,
+    // chunk, row block), row blocks innermost: the XCD's L2 then holds its
+    // weights while the rows stream past them.
+    const int total = T.mb * T.nb * T.kc, per = (int)(gridDim.x >> 3);
+    const int L = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if (L >= total) return;
+    const int m_blk = L % T.mb, nc = L / T.mb;
+    const int ch = nc % T.kc, n_blk = nc / T.kc;
+    const int K = P.w.K, N = P.w.N, Ks = K / 16, panels = N / 32;
+    const int pw = NW * n_blk + wave, p = min(pw, panels - 1);
+    const int sb = ch * T.cs, se = min(Ks, sb + T.cs);
+    const int nst = (se - sb + SS - 1) / SS;
+
+    const uint32_t *wm = P.w.wm + (size_t)p * Ks * 64 + lane;
+    const uint16_t *sa = P.w.sa + (size_t)p * K + 8 * half, *sc = P.w.sb + (size_t)p * K + 8 * half;
+    // this wave's units of a stage's A operands: u = wave * MT + j ->
+    // (step u / (2 MT), tile, hi / lo)
+    const half8 *asrc[UW];
+    int astep[UW];
+#pragma unroll
+    for (int j = 0; j < UW; j++) {
+        const int u = wave * UW + j, rem = u % (2 * MT);
+        astep[j] = u / (2 * MT);
+        asrc[j] = reinterpret_cast<const half8 *>((rem & 1) ? P.xl : P.xh) +
+                  (size_t)(m_blk * MT + (rem >> 1)) * Ks * 64 + lane;
+    }
+    half8 ra[2][UW];
+    uint32_t wq[2][SS];
+    u32x4v va[2][SS], vb[2][SS];
+    auto load = [&](int st, int b) {
+#pragma unroll
+        for (int i = 0; i < SS; i++) {
+            const int s = min(sb + SS * st + i, Ks - 1);
+            wq[b][i] = wm[(size_t)s * 64];
+            va[b][i] = *reinterpret_cast<const u32x4v *>(sa + 16 * s);
+            vb[b][i] = *reinterpret_cast<const u32x4v *>(sc + 16 * s);
+        }
+#pragma unroll
+        for (int j = 0; j < UW; j++) ra[b][j] = asrc[j][(size_t)min(sb + SS * st + astep[j], Ks - 1) * 64];
+    };
+    auto put = [&](int b) {
+#pragma unroll
+        for (int j = 0; j < UW; j++) abuf[b][wave * UW + j][lane] = ra[b][j];
+    };
+    f32x16 acc[MT];
+#pragma unroll
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[t][r] = 0.0f;
+
+    // The B operands of one step: q as binary16 1024 + nib (magic exponent)
+    // minus 1032, times sa and sb.  A step past the end has nibbles of 8, q = 0.
+    half8 ba[SS], bb[SS];
+    auto form = [&](int st, int b, int i) {
+        const uint32_t w = sb + SS * st + i < se ? wq[b][i] : 0x88888888u;  // uniform
+        const uint32_t sap[4] = {va[b][i].x, va[b][i].y, va[b][i].z, va[b][i].w};
+        const uint32_t sbp[4] = {vb[b][i].x, vb[b][i].y, vb[b][i].z, vb[b][i].w};
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+            const uint32_t bits = ((w >> (4 * j)) & 0x000F000Fu) | 0x64006400u;
+            const half2v q = __builtin_bit_cast(half2v, bits) - (half2v){(_Float16)1032.0f, (_Float16)1032.0f};
+            const half2v a = q * __builtin_bit_cast(half2v, sap[j]);
+            const half2v c = q * __builtin_bit_cast(half2v, sbp[j]);
+            ba[i][2 * j] = a.x;
+            ba[i][2 * j + 1] = a.y;
+            bb[i][2 * j] = c.x;
+            bb[i][2 * j + 1] = c.y;
+        }
+    };
+    half8 xh[SS][MT], xl[SS][MT];
+    auto get = [&](int b, int i) {
+#pragma unroll
+        for (int t = 0; t < MT; t++) {
+            xh[i][t] = abuf[b][(i * MT + t) * 2][lane];
+            xl[i][t] = abuf[b][(i * MT + t) * 2 + 1][lane];
+        }
+    };
+    auto mma = [&](int i) {
+#pragma unroll
+        for (int t = 0; t < MT; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh[i][t], ba[i], acc[t], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < MT; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh[i][t], bb[i], acc[t], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < MT; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl[i][t], ba[i], acc[t], 0, 0, 0);
+    };
+    // Stage st from buffer b = st % 2, its first step's B operands formed: the
+    // second step's operands under the first step's, the next stage's LDS writes and
+    // first B operands and the loads of stage st + 2 under the second's.
+    auto stage = [&](int st, int b) {
+        get(b, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        get(b, 1);
+        form(st, b, 1);
+        mma(0);
+#pragma unroll
+        for (int u = 0; u < 3 * MT; u++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 12 / MT, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        put(b ^ 1);  // stage st + 1
+        form(min(st + 1, nst - 1), b ^ 1, 0);
+        load(min(st + 2, nst - 1), b);
+        mma(1);
+#pragma unroll
+        for (int u = 0; u < 3 * MT; u++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 16 / MT, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+    };
+
+    load(0, 0);
+    put(0);
+    load(min(1, nst - 1), 1);
+    form(0, 0, 0);
+    __syncthreads();
+    for (int st = 0; st < nst; st += 2) {
+        stage(st, 0);
+        if (st + 1 < nst) stage(st + 1, 1);  // uniform
+    }
+
+    const int m0 = m_blk * MT * 32, n = 32 * p + col;
+    const int tile = n_blk * T.mb + m_blk;
+    if (T.kc > 1) {
+        // partials in accumulator order: [chunk][wave][tile][register][lane]
+        float *mine = P.part + ((size_t)tile * T.kc + ch) * (size_t)(NW * MT * 1024) + wave * (MT * 1024) + lane;
+#pragma unroll
+        for (int t = 0; t < MT; t++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) st_dev(mine + (t * 16 + r) * 64, acc[t][r]);
+        wait_stores();
+        __syncthreads();
+        if (tid == 0) s_last = arrive_dev(&P.counters[tile]) == (unsigned)(T.kc - 1);
+        __syncthreads();
+        if (!s_last) return;
+        if (tid == 0) reset_dev(&P.counters[tile]);
+        // the last chunk to arrive adds all of them in chunk order
+        const float *all = P.part + (size_t)tile * T.kc * (size_t)(NW * MT * 1024) + wave * (MT * 1024) + lane;
+#pragma unroll
+        for (int t = 0; t < MT; t++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[t][r] = 0.0f;
+        for (int c = 0; c < T.kc; c++) {
+            const float *pc = all + (size_t)c * (NW * MT * 1024);
+            float v[MT][16];
+#pragma unroll
+            for (int t = 0; t < MT; t++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) v[t][r] = ld_dev(pc + (t * 16 + r) * 64);
+#pragma unroll
+            for (int t = 0; t < MT; t++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[t][r] += v[t][r];
+        }
+    }
+    if (pw >= panels) return;
+    const float bias = P.bias ? P.bias[n] : 0.0f;
+#pragma unroll
+    for (int t = 0; t < MT; t++) {
+        float old[16];
+        int e[16];
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int m = m0 + 32 * t + (r >> 2) * 8 + half * 4 + (r & 3);
+            e[r] = P.rexp[m];
+            old[r] = P.accumulate ? P.y[(size_t)min(m, P.M - 1) * P.ldy + n] : 0.0f;
+        }
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int m = m0 + 32 * t + (r >> 2) * 8 + half * 4 + (r & 3);
+            if (m >= P.M) continue;
+            float v = ldexpf(acc[t][r], -e[r]);
+            if (P.bias) v += bias;
+            P.y[(size_t)m * P.ldy + n] = P.accumulate ? old[r] + v : v;
+        }
+    }
+}
+
 }  // namespace
 
 void launch_repack_mfma(hipStream_t st, const DevQ4 &w, uint32_t *wm, uint16_t *sa, uint16_t *sb, int *too_large) {
@@ -357,6 +564,21 @@ void launch_gemm_mfma(hipStream_t st, const GemmMfmaParams &p, int mt, int sw, i
         launch_gemm_mfma_mt<1>(st, p, sw, kc);
     else
         launch_gemm_mfma_mt<2>(st, p, sw, kc);
+}
+
+void launch_gemm_mfma_tile(hipStream_t st, const GemmMfmaParams &p, const GemmTilePlan &t) {
+    const int total = t.mb * t.nb * t.kc;
+    const dim3 grid((unsigned)((total + 7) / 8 * 8)), block(64 * t.nw);
+    if (t.nw == 8) {
+        hipLaunchKernelGGL((k_gemm_mfma_tile<4, 8>), grid, block, 0, st, p, t);
+        return;
+    }
+    switch (t.mt) {
+        case 4: hipLaunchKernelGGL((k_gemm_mfma_tile<4, 4>), grid, block, 0, st, p, t); break;
+        case 3: hipLaunchKernelGGL((k_gemm_mfma_tile<3, 4>), grid, block, 0, st, p, t); break;
+        case 2: hipLaunchKernelGGL((k_gemm_mfma_tile<2, 4>), grid, block, 0, st, p, t); break;
+        default: hipLaunchKernelGGL((k_gemm_mfma_tile<1, 4>), grid, block, 0, st, p, t); break;
+    }
 }
 
 }  // namespace qtts

@@ -1,0 +1,47 @@
+"""The Q4 product in row blocks (more than 64 rows) against float64, at the
+edges of its tiles: one row past a pass, rows off the 32- and 128-row tiles,
+an odd number of 16-row K steps, panel counts off a block's 4 or 8, one and
+several K chunks; and the scale split's last accepted scales."""
+import numpy as np
+import pytest
+
+import qtts
+
+pytestmark = pytest.mark.gpu
+
+
+def _bound(x, w, K):
+    """Per output: the terms' dropped part (|xl| <= 2^-12 |x| times |sb| <=
+    2^-8 s, one bit spare) and one f32 rounding per 16-row product of each of
+    the three partial products, on the sum of magnitudes."""
+    return (2.0 ** -19 + (3 * K / 16 + 32) * 2.0 ** -24) * (np.abs(x.astype(np.float64)) @ np.abs(w))
+
+
+@pytest.mark.parametrize("rows,K,N", [(65, 1040, 160), (96, 2048, 2048), (97, 16, 32), (128, 48, 288), (129, 6144, 96),
+                                      (300, 1024, 1056), (1000, 272, 2048), (1064, 2048, 4096), (4097, 32, 64)])
+def test_gemm_row_blocks(ctx, rows, K, N):
+    w = qtts.Q4Weight.synthetic(21, f"tiles.{K}.{N}", K, N)
+    x = qtts.synth_normal_f32(21, f"tiles.x.{rows}.{K}", rows * K).reshape(rows, K)
+    x[rows // 2] *= 1e4
+    x[rows - 1] *= 1e-6
+    d = qtts.DeviceQ4(ctx, w)
+    y = d.gemm(x, rows).reshape(rows, N)
+    wd = w.dequantize().astype(np.float64)
+    err = np.abs(y - x.astype(np.float64) @ wd)
+    assert np.all(err <= _bound(x, wd, K) + 1e-38), float(np.max(err / (_bound(x, wd, K) + 1e-38)))
+    assert np.array_equal(y, d.gemm(x, rows).reshape(rows, N))
+
+
+@pytest.mark.parametrize("rows", [16, 80])
+@pytest.mark.parametrize("scale", [8188.0, 8160.0, 8128.0, 4100.0, 6e-8, 6.1e-5])
+def test_gemm_scale_split_is_exact(ctx, rows, scale):
+    """One-hot rows give the dequantized rows bit for bit: s = sa + sb exactly,
+    also where rounding sa up would pass binary16."""
+    K, N = 96, 64
+    w = qtts.Q4Weight.synthetic(22, "split", K, N)
+    w.scales[:] = np.float16(scale).view(np.uint16)
+    w.scales[1::2] += np.arange(K // 2, dtype=np.uint16)[:, None] if scale < 8000 else 0
+    x = np.zeros((rows, K), dtype=np.float32)
+    x[np.arange(rows), np.arange(rows) * 7 % K] = 1.0
+    y = qtts.DeviceQ4(ctx, w).gemm(x, rows).reshape(rows, N)
+    assert np.array_equal(y, w.dequantize()[np.arange(rows) * 7 % K])
