@@ -415,52 +415,69 @@ __global__ __launch_bounds__(64 * NW, 2) void k_gemm_mfma_tile(GemmMfmaParams P,
             bb[i][2 * j + 1] = c.y;
         }
     };
-    half8 xh[SS][MT], xl[SS][MT];
-    auto get = [&](int b, int i) {
+    // Tiles two at a time: the operands of the next two come from LDS under
+    // the MFMAs of these two.
+    constexpr int NG = (MT + 1) / 2;
+    half8 xh[2][2], xl[2][2];
+    auto get = [&](int b, int g) {  // group g = step g / NG, tiles 2 (g % NG) and the next
 #pragma unroll
-        for (int t = 0; t < MT; t++) {
-            xh[i][t] = abuf[b][(i * MT + t) * 2][lane];
-            xl[i][t] = abuf[b][(i * MT + t) * 2 + 1][lane];
+        for (int u = 0; u < 2; u++) {
+            const int t = 2 * (g % NG) + u;
+            if (t < MT) {
+                xh[g & 1][u] = abuf[b][((g / NG) * MT + t) * 2][lane];
+                xl[g & 1][u] = abuf[b][((g / NG) * MT + t) * 2 + 1][lane];
+            }
         }
     };
-    auto mma = [&](int i) {
+    auto mma = [&](int g) {
+        const int i = g / NG, t0 = 2 * (g % NG), n = t0 + 1 < MT ? 2 : 1;
 #pragma unroll
-        for (int t = 0; t < MT; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh[i][t], ba[i], acc[t], 0, 0, 0);
+        for (int u = 0; u < n; u++)
+            acc[t0 + u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh[g & 1][u], ba[i], acc[t0 + u], 0, 0, 0);
 #pragma unroll
-        for (int t = 0; t < MT; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh[i][t], bb[i], acc[t], 0, 0, 0);
+        for (int u = 0; u < n; u++)
+            acc[t0 + u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh[g & 1][u], bb[i], acc[t0 + u], 0, 0, 0);
 #pragma unroll
-        for (int t = 0; t < MT; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl[i][t], ba[i], acc[t], 0, 0, 0);
+        for (int u = 0; u < n; u++)
+            acc[t0 + u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl[g & 1][u], ba[i], acc[t0 + u], 0, 0, 0);
     };
     // Stage st from buffer b = st % 2, its first step's B operands formed: the
-    // second step's operands under the first step's, the next stage's LDS writes and
-    // first B operands and the loads of stage st + 2 under the second's.
+    // second step's under the first step's MFMAs, the next stage's LDS writes
+    // and first B operands and the loads of stage st + 2 under the second's.
     auto stage = [&](int st, int b) {
         get(b, 0);
         __builtin_amdgcn_sched_barrier(0);
-        get(b, 1);
-        form(st, b, 1);
-        mma(0);
 #pragma unroll
-        for (int u = 0; u < 3 * MT; u++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x002, 12 / MT, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        put(b ^ 1);  // stage st + 1
-        form(min(st + 1, nst - 1), b ^ 1, 0);
-        load(min(st + 2, nst - 1), b);
-        mma(1);
+        for (int g = 0; g < SS * NG; g++) {
+            if (g + 1 < SS * NG) get(b, g + 1);
+            if (g == 0) form(st, b, 1);
+            if (g == NG) {
+                put(b ^ 1);  // stage st + 1
+                form(min(st + 1, nst - 1), b ^ 1, 0);
+            }
+            if (g == SS * NG - 1) load(min(st + 2, nst - 1), b);
+            mma(g);
 #pragma unroll
-        for (int u = 0; u < 3 * MT; u++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x002, 16 / MT, 0);
+            for (int u = 0; u < 6; u++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
         }
-        __builtin_amdgcn_sched_barrier(0);
         __syncthreads();
     };
+    // Every 16 steps the accumulators move to a second level, so that a sum
+    // over K = 2048 rounds as often as one over 16 steps and one over 8 such
+    // sums: with one chain of 384 MFMAs its rounding (4.1e-7 of an
+    // all-positive sum) was five times k_gemm_mfma's.
+    f32x16 top[MT];
+#pragma unroll
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) top[t][r] = 0.0f;
 
     load(0, 0);
     put(0);
@@ -470,7 +487,18 @@ __global__ __launch_bounds__(64 * NW, 2) void k_gemm_mfma_tile(GemmMfmaParams P,
     for (int st = 0; st < nst; st += 2) {
         stage(st, 0);
         if (st + 1 < nst) stage(st + 1, 1);  // uniform
+        if ((st & 6) == 6 || st + 2 >= nst) {
+#pragma unroll
+            for (int t = 0; t < MT; t++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    top[t][r] += acc[t][r];
+                    acc[t][r] = 0.0f;
+                }
+        }
     }
+#pragma unroll
+    for (int t = 0; t < MT; t++) acc[t] = top[t];
 
     const int m0 = m_blk * MT * 32, n = 32 * p + col;
     const int tile = n_blk * T.mb + m_blk;
