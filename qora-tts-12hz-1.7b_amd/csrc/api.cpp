@@ -1953,16 +1953,17 @@ static qtts_status make_talker_mfma(qtts_talker *t) {
 // layer: QKV (RMSNorm prologue) -> QK-norm, RoPE, KV append -> causal
 // attention (row r sees positions 0..r) -> O (+residual) -> gate|up (RMSNorm
 // prologue) -> down (SiLU*up prologue, +residual); src/talker.rs:364-462.
+// Up to kAttnPrefillRows rows, one block per row and kv head (k_attn: 6.8 us
+// at 10 rows, 8.0 at 64, 12.7 at 96) has the shorter chain; past them the
+// row-tiled kernel (k_attn_prefill: 9.4, 10.0 and 9.7 us) wins, 78 against
+// 620 us at 1064.
+constexpr int kAttnPrefillRows = 64;
+static_assert(kAttnPrefillRows <= kAttnMaxChunk, "one split holds every row's cache");
+
 static qtts_status prefill_layers_mfma(qtts_talker *t, qtts_kv *kv, int seq_len) {
     qtts_ctx *c = t->ctx;
     const Stack &st = t->st;
     const int hidden = st.hidden, qd = st.nq * st.hd, nqkv = qd + 2 * st.nkv * st.hd;
-    // one attention split per kAttnMaxChunk positions of the prefill (the
-    // decode-sized split count would give thousands of tiny blocks)
-    const int nsplit = attn_nsplit(seq_len, 1);
-    int attn_rows = (int)(kAttnPartFloats / ((size_t)st.nq * nsplit * (st.hd + 2)));
-    if (attn_rows > kAttnCounters / st.nkv) attn_rows = kAttnCounters / st.nkv;
-    if (attn_rows < 1) return fail(c, QTTS_ESHAPE, "attention split buffer too small");
     for (int l = 0; l < st.layers; l++) {
         const DevLayer &Ly = st.L[l];
         const DevQ4Mfma *W = &t->mfma[(size_t)4 * l];
@@ -1989,27 +1990,27 @@ static qtts_status prefill_layers_mfma(qtts_talker *t, qtts_kv *kv, int seq_len)
         q.kv_cap = kv->cap;
         launch_qkv_rows(c->stream, q);
         QTTS_TRY(check_launch(c, "k_qkv_rows"));
-        for (int r0 = 0; r0 < seq_len; r0 += attn_rows) {
-            const int M = seq_len - r0 < attn_rows ? seq_len - r0 : attn_rows;
-            AttnParams a{};
-            a.q = t->qp + (size_t)r0 * qd;
-            a.ldq = qd;
-            a.kcache = kc;
-            a.vcache = vc;
-            a.kv_cap = kv->cap;
-            a.nq = st.nq;
-            a.nkv = st.nkv;
-            a.hd = st.hd;
-            a.kvlen_const = r0;
-            a.nsplit = nsplit;
-            a.scale = 1.0f / sqrtf((float)st.hd);  // src/talker.rs:305
+        AttnParams a{};
+        a.q = t->qp;
+        a.ldq = qd;
+        a.kcache = kc;
+        a.vcache = vc;
+        a.kv_cap = kv->cap;
+        a.nq = st.nq;
+        a.nkv = st.nkv;
+        a.hd = st.hd;
+        a.scale = 1.0f / sqrtf((float)st.hd);  // src/talker.rs:305
+        a.out = t->ap;
+        a.ldo = qd;
+        if (seq_len > kAttnPrefillRows || seq_len * st.nkv > kAttnCounters) {
+            launch_attn_prefill(c->stream, a, seq_len);
+        } else {
+            a.nsplit = 1;
             a.part = c->attn_part;
             a.counters = c->attn_counters;
-            a.out = t->ap + (size_t)r0 * qd;
-            a.ldo = qd;
-            launch_attention(c->stream, a, M);
-            QTTS_TRY(check_launch(c, "k_attn"));
+            launch_attention(c->stream, a, seq_len);
         }
+        QTTS_TRY(check_launch(c, "prefill attention"));
         QTTS_TRY(run_gemm_mfma(c, W[1], t->ap, seq_len, qd, MFMA_ROWS_PLAIN, nullptr, t->xp, hidden, nullptr, true));
         QTTS_TRY(run_gemm_mfma(c, W[2], t->xp, seq_len, hidden, MFMA_ROWS_RMSNORM, Ly.post_g, t->rawp, 2 * st.inter,
                                nullptr, false));

@@ -79,6 +79,11 @@ __device__ __forceinline__ float halves_sum(float v) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+__device__ __forceinline__ float halves_max(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
 // Sum / max over the 64-lane wave; every lane gets the result.
 __device__ __forceinline__ float wave_sum(float v) {
     v = row16_sum(v);

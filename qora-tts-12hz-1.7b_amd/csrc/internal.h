@@ -360,6 +360,8 @@ void launch_dec_conv_repack(hipStream_t st, const float *w, long long sm, long l
                             int taps, int cin16, int mtiles, int ksteps, int ew, _Float16 *wh, _Float16 *wl);
 void launch_dec_conv_mfma(hipStream_t st, const DecConvMfmaParams &p);
 void launch_gemm_mfma(hipStream_t st, const GemmMfmaParams &p, int mt, int sw, int kc);
+// q, kcache, vcache, kv_cap, nq, nkv, scale and out of p; head_dim 128; M rows into an empty cache
+void launch_attn_prefill(hipStream_t st, const AttnParams &p, int M);
 // part: [mb * nb * kc][32 * mt * 32 * nw] when kc > 1; counters: mb * nb, zero between launches
 void launch_gemm_mfma_tile(hipStream_t st, const GemmMfmaParams &p, const GemmTilePlan &t);
 void launch_embed_sum(hipStream_t st, const EmbSumParams &p);

@@ -27,6 +27,7 @@ namespace {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x4v __attribute__((ext_vector_type(4)));
 
 // Repack of one panel-major Q4 weight into the MFMA B-operand order
@@ -557,6 +558,170 @@ __global__ __launch_bounds__(64 * NW, 2) void k_gemm_mfma_tile(GemmMfmaParams P,
     }
 }
 
+// Causal attention of a whole prefill (src/talker.rs:404-441): row i of M
+// sees cache rows 0..i.  A block takes one query head and 32 rows; its 4
+// waves take every 4th run of 32 keys, and their softmax partials are merged
+// in wave order.  The products are f32 MFMAs (32x32x2), so nothing is
+// rounded below f32.
+//   scores: S^T = K Q^T, lane l holding query l % 32 and the keys
+//     key(r) = 8 (r / 4) + 4 (l / 32) + r % 4 in its 16 registers, so the
+//     softmax of a query is a reduction over registers and one lane exchange;
+//   values: O^T += V^T P^T with the registers of P as they are (MFMA r takes
+//     key(r) of both lane halves), the MFMA row m of the t-th product being
+//     dim 4 m + t, so a lane reads V and stores O four dims at a time.
+// K and V are read from the cache straight into operand registers: an f32
+// MFMA takes 64 cycles, 32 keys 8192, and their 32 KiB come from the L2
+// meanwhile.  Longest rows first; the query heads of one kv head (and so its
+// K and V) fall on one XCD where there are 8 kv heads.
+// 1064 rows, 16 heads: 78 us per layer (the f32 MFMAs alone 37), where k_attn
+// (one row per block) took 620.
+__global__ __launch_bounds__(256, 2) void k_attn_prefill(AttnParams P, int M) {
+    constexpr int HD = 128;
+    __shared__ float part[4][16][4][64];  // [wave][register][t][lane]
+    __shared__ float ml[4][2][32];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int half = lane >> 5, col = lane & 31;
+    const int G = P.nq / P.nkv, tiles = (M + 31) / 32;
+    const int hx = blockIdx.x % P.nq, qt = tiles - 1 - blockIdx.x / P.nq;
+    const int kvh = hx % P.nkv, head = kvh * G + hx / P.nkv;
+    const int q = 32 * qt + col;
+    const float *K = P.kcache + (size_t)kvh * P.kv_cap * HD, *V = P.vcache + (size_t)kvh * P.kv_cap * HD;
+    const float *qr = P.q + (size_t)min(q, M - 1) * P.ldq + (size_t)head * HD + 4 * half;
+
+    f32x4 qv[16];  // dims 8 g + 4 half + j
+#pragma unroll
+    for (int g = 0; g < 16; g++) qv[g] = *reinterpret_cast<const f32x4 *>(qr + 8 * g);
+    f32x16 acc[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[t][r] = 0.0f;
+    float mx = -INFINITY, sum = 0.0f;
+    // K and V in batches of 4 registers' worth, one batch ahead of the MFMAs
+    f32x4 kb[2][4], vb[2][4];
+    auto load_k = [&](int kt, int c, int to) {
+        const float *kr = K + (size_t)min(32 * kt + col, M - 1) * HD + 4 * half + 32 * c;
+#pragma unroll
+        for (int g = 0; g < 4; g++) kb[to][g] = *reinterpret_cast<const f32x4 *>(kr + 8 * g);
+    };
+    auto load_v = [&](int kt, int c, int to) {  // keys 32 kt + 8 c + 4 half + r
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            vb[to][r] = *reinterpret_cast<const f32x4 *>(
+                V + (size_t)min(32 * kt + 8 * c + 4 * half + r, M - 1) * HD + 4 * col);
+    };
+    load_k(min(wave, qt), 0, 0);
+    for (int kt = wave; kt <= qt; kt += 4) {
+        const bool diag = kt == qt;
+        f32x16 s;
+#pragma unroll
+        for (int r = 0; r < 16; r++) s[r] = 0.0f;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            if (c < 3)
+                load_k(kt, c + 1, (c + 1) & 1);
+            else
+                load_v(kt, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    s = __builtin_amdgcn_mfma_f32_32x32x2f32(kb[c & 1][g][j], qv[4 * c + g][j], s, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        float m = mx;
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int key = 32 * kt + 8 * (r >> 2) + 4 * half + (r & 3);
+            s[r] = diag && key > q ? -INFINITY : s[r] * P.scale;
+            m = fmaxf(m, s[r]);
+        }
+        m = halves_max(m);
+        const float alpha = expf(mx - m);
+        float l = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            s[r] = expf(s[r] - m);
+            l += s[r];
+        }
+        sum = sum * alpha + halves_sum(l);
+        mx = m;
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[t][r] *= alpha;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            if (c < 3)
+                load_v(kt, c + 1, (c + 1) & 1);
+            else
+                load_k(min(kt + 4, qt), 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int t = 0; t < 4; t++)
+                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(vb[c & 1][r][t], s[4 * c + r], acc[t], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    // merge: weights exp(max of the wave - max of all), sums in wave order
+    if (half == 0) {
+        ml[wave][0][col] = mx;
+        ml[wave][1][col] = sum;
+    }
+    __syncthreads();
+    float m = ml[0][0][col];
+#pragma unroll
+    for (int w = 1; w < 4; w++) m = fmaxf(m, ml[w][0][col]);
+    float l = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 4; w++)
+        if (w <= qt) l += ml[w][1][col] * expf(ml[w][0][col] - m);
+    const float f = wave <= qt ? expf(mx - m) : 0.0f;
+#pragma unroll
+    for (int r = 0; r < 16; r++)
+#pragma unroll
+        for (int t = 0; t < 4; t++) part[wave][r][t][lane] = acc[t][r] * f;
+    __syncthreads();
+    float *o = P.out + (size_t)q * P.ldo + (size_t)head * HD;
+    bool odd = false;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int r = 4 * wave + i;
+        f32x4 v;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            v[t] = ((part[0][r][t][lane] + part[1][r][t][lane]) + (part[2][r][t][lane] + part[3][r][t][lane])) / l;
+            odd |= !(fabsf(v[t]) < INFINITY);
+        }
+        if (q < M) *reinterpret_cast<f32x4 *>(o + 4 * (8 * (r >> 2) + 4 * half + (r & 3))) = v;
+    }
+    if (!__syncthreads_or(odd)) return;
+    // An infinity or NaN: a key that a row does not see meets it with weight
+    // 0 in the last run's MFMAs.  The block's rows again, one at a time over
+    // the keys each sees, lane d holding dims d and d + 64.
+    for (int i = wave; i < 32 && 32 * qt + i < M; i += 4) {
+        const int row = 32 * qt + i;
+        const float *qq = P.q + (size_t)row * P.ldq + (size_t)head * HD;
+        const float q0 = qq[lane], q1 = qq[lane + 64];
+        float top = -INFINITY, den = 0.0f, o0 = 0.0f, o1 = 0.0f;
+        for (int k = 0; k <= row; k++)
+            top = fmaxf(top, wave_sum(q0 * K[(size_t)k * HD + lane] + q1 * K[(size_t)k * HD + lane + 64]) * P.scale);
+        for (int k = 0; k <= row; k++) {
+            const float sc = wave_sum(q0 * K[(size_t)k * HD + lane] + q1 * K[(size_t)k * HD + lane + 64]) * P.scale;
+            const float p = expf(sc - top);
+            den += p;
+            o0 += p * V[(size_t)k * HD + lane];
+            o1 += p * V[(size_t)k * HD + lane + 64];
+        }
+        float *dst = P.out + (size_t)row * P.ldo + (size_t)head * HD;
+        dst[lane] = o0 / den;
+        dst[lane + 64] = o1 / den;
+    }
+}
+
 }  // namespace
 
 void launch_repack_mfma(hipStream_t st, const DevQ4 &w, uint32_t *wm, uint16_t *sa, uint16_t *sb, int *too_large) {
@@ -607,6 +772,10 @@ void launch_gemm_mfma_tile(hipStream_t st, const GemmMfmaParams &p, const GemmTi
         case 2: hipLaunchKernelGGL((k_gemm_mfma_tile<2, 4>), grid, block, 0, st, p, t); break;
         default: hipLaunchKernelGGL((k_gemm_mfma_tile<1, 4>), grid, block, 0, st, p, t); break;
     }
+}
+
+void launch_attn_prefill(hipStream_t st, const AttnParams &p, int M) {
+    hipLaunchKernelGGL(k_attn_prefill, dim3((unsigned)(p.nq * ((M + 31) / 32))), dim3(256), 0, st, p, M);
 }
 
 }  // namespace qtts

@@ -1,0 +1,47 @@
+"""The prefill's attention past 64 rows (32-row tiles, four waves over the
+keys) against the oracle: one row past the limit, whole and ragged tiles, one
+to four query heads per kv head; and a row of NaNs, which the rows before it
+must not see."""
+import numpy as np
+import pytest
+
+import qtts
+from oracle import oracle
+from shapes import within
+
+pytestmark = pytest.mark.gpu
+
+
+def _talker(ctx, heads, kv_heads, seed=31):
+    cfg = qtts.StackConfig(layers=2, hidden=256, heads=heads, kv_heads=kv_heads, head_dim=128, inter=512, vocab=320,
+                           max_position=4096)
+    tw = qtts.TalkerWeights(seed, cfg)
+    return cfg, tw, qtts.Talker(ctx, tw)
+
+
+@pytest.mark.parametrize("heads,kv_heads", [(4, 4), (4, 2), (4, 1), (18, 18)])
+@pytest.mark.parametrize("rows", [64, 65, 96, 129, 257])
+def test_prefill_attention(ctx, rows, heads, kv_heads):
+    cfg, tw, t = _talker(ctx, heads, kv_heads)
+    ot = oracle.Talker(tw)
+    x = qtts.synth_normal_f32(31, f"attn.x.{rows}", rows * cfg.hidden)
+    kv, okv = t.new_kv(rows + 3), ot.new_kv(rows + 3)
+    lh, olh = t.prefill_talker_raw(x, rows, kv), ot.prefill_talker_raw(x, rows, okv)
+    assert within(lh, olh)
+    for got, ref in zip(kv.store(), okv.store()):  # layer 1's rows carry every row's attention
+        assert within(got, ref)
+
+
+@pytest.mark.parametrize("rows,bad", [(96, 95), (100, 70), (129, 128), (200, 3)])
+def test_prefill_rows_before_a_nan_row_are_unchanged(ctx, rows, bad):
+    cfg, tw, t = _talker(ctx, 4, 2)
+    x = qtts.synth_normal_f32(32, f"nan.x.{rows}", rows * cfg.hidden).reshape(rows, -1).copy()
+    kv = t.new_kv(rows)
+    t.prefill_talker_raw(x, rows, kv)
+    clean = kv.store()
+    x[bad, 7] = np.inf  # its normed row is NaN
+    kv.clear()
+    t.prefill_talker_raw(x, rows, kv)
+    for got, ref in zip(kv.store(), clean):
+        assert np.all(np.isfinite(got[:, :bad])) and within(got[:, :bad], ref[:, :bad])
+        assert np.all(np.isnan(got[1, bad:]).any(axis=(1, 2)))
