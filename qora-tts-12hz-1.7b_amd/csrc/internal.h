@@ -41,7 +41,7 @@ struct DevQ4Mfma {
 };
 
 // Row prologues of the MFMA GEMM's input split.
-enum MfmaRowsMode { MFMA_ROWS_PLAIN = 0, MFMA_ROWS_RMSNORM = 1, MFMA_ROWS_SWIGLU = 2 };
+enum MfmaRowsMode { MFMA_ROWS_PLAIN = 0, MFMA_ROWS_RMSNORM = 1, MFMA_ROWS_SWIGLU = 2, MFMA_ROWS_SILU = 3 };
 constexpr int kMfmaRowsMaxK = 8192;
 
 struct MfmaRowsParams {
@@ -150,6 +150,7 @@ struct GemmMfmaParams {
     const float *bias;        // optional
     float *y;                 // y[m * ldy + n] (+)= result
     int ldy, accumulate;
+    int full;                 // 1: all four partial products of a term
 };
 
 // The same product in row blocks of 32 * mt rows (k_gemm_mfma_tile), for

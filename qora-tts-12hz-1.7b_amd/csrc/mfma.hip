@@ -13,7 +13,9 @@
 // Products of binary16 values are exact in the f32 accumulator, and the
 // xl*sb*q term (relative size 2^-19) is dropped, so every term carries a
 // relative error of ~2^-19 or less before the f32 sums -- the f32 level the
-// parity tolerance is set for.
+// parity tolerance is set for.  With GemmMfmaParams::full that term is a
+// fourth MFMA, and a term's error that of x's split, 2^-22 (the text
+// projection, whose other path is the GEMV's f32 products).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -114,6 +116,10 @@ __global__ __launch_bounds__(256) void k_mfma_rows(MfmaRowsParams P) {
                 const uint4 q = *reinterpret_cast<const uint4 *>(P.gamma + 8 * g);
                 gw[j][0] = q.x, gw[j][1] = q.y, gw[j][2] = q.z, gw[j][3] = q.w;
             }
+            if (P.mode == MFMA_ROWS_SILU) {
+#pragma unroll
+                for (int i = 0; i < 8; i++) v[j][i] = v[j][i] / (1.0f + expf(-v[j][i]));
+            }
             if (P.mode == MFMA_ROWS_SWIGLU) {
                 const float4 c = *reinterpret_cast<const float4 *>(src + K + 8 * g);
                 const float4 d = *reinterpret_cast<const float4 *>(src + K + 8 * g + 4);
@@ -198,7 +204,7 @@ __global__ __launch_bounds__(256) void k_mfma_rows(MfmaRowsParams P) {
 // chunks, each block stores its tile to `part` and the last block of a panel
 // to arrive (a counter per panel) adds the chunks in chunk order --
 // deterministic -- and finishes: * 2^-rexp[m], + bias, store or accumulate.
-template <int MT, int SW>
+template <int MT, int SW, bool FULL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_gemm_mfma(GemmMfmaParams P) {
     __shared__ float red[4][MT * 1024];
     __shared__ int s_last;
@@ -257,6 +263,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
             acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh[i][t], ba, acc[t], 0, 0, 0);
             acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh[i][t], bb, acc[t], 0, 0, 0);
             acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl[i][t], ba, acc[t], 0, 0, 0);
+            if constexpr (FULL) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl[i][t], bb, acc[t], 0, 0, 0);
         }
     }
     // 3. the 4 waves through LDS.  D layout: lane l, register r -> row
@@ -336,7 +343,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
 // binary16 MFMAs issued; a library binary16 product with as many MFMAs takes
 // 181), where 17 passes of k_gemm_mfma took 410; 1000 rows, 6144 -> 2048, 342
 // -> 113 us.
-template <int MT, int NW>
+template <int MT, int NW, bool FULL>
 __global__ __launch_bounds__(64 * NW, 2) void k_gemm_mfma_tile(GemmMfmaParams P, GemmTilePlan T) {
     constexpr int SS = 2;  // 16-row steps per stage
     constexpr int U = SS * MT * 2;  // 1 KiB operand units per stage
@@ -441,6 +448,11 @@ __global__ __launch_bounds__(64 * NW, 2) void k_gemm_mfma_tile(GemmMfmaParams P,
 #pragma unroll
         for (int u = 0; u < n; u++)
             acc[t0 + u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl[g & 1][u], ba[i], acc[t0 + u], 0, 0, 0);
+        if constexpr (FULL) {
+#pragma unroll
+            for (int u = 0; u < n; u++)
+                acc[t0 + u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl[g & 1][u], bb[i], acc[t0 + u], 0, 0, 0);
+        }
     };
     // Stage st from buffer b = st % 2, its first step's B operands formed: the
     // second step's under the first step's MFMAs, the next stage's LDS writes
@@ -459,7 +471,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_gemm_mfma_tile(GemmMfmaParams P,
             if (g == SS * NG - 1) load(min(st + 2, nst - 1), b);
             mma(g);
 #pragma unroll
-            for (int u = 0; u < 6; u++) {
+            for (int u = 0; u < (FULL ? 8 : 6); u++) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);
@@ -470,7 +482,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_gemm_mfma_tile(GemmMfmaParams P,
         }
         __syncthreads();
     };
-    // Every 16 steps the accumulators move to a second level, so that a sum
+    // Every 16 steps (8 with FULL) the accumulators move to a second level, so that a sum
     // over K = 2048 rounds as often as one over 16 steps and one over 8 such
     // sums: with one chain of 384 MFMAs its rounding (4.1e-7 of an
     // all-positive sum) was five times k_gemm_mfma's.
@@ -488,7 +500,7 @@ __global__ __launch_bounds__(64 * NW, 2) void k_gemm_mfma_tile(GemmMfmaParams P,
     for (int st = 0; st < nst; st += 2) {
         stage(st, 0);
         if (st + 1 < nst) stage(st + 1, 1);  // uniform
-        if ((st & 6) == 6 || st + 2 >= nst) {
+        if ((st & (FULL ? 2 : 6)) == (FULL ? 2 : 6) || st + 2 >= nst) {
 #pragma unroll
             for (int t = 0; t < MT; t++)
 #pragma unroll
@@ -741,37 +753,42 @@ void launch_mfma_rows(hipStream_t st, const MfmaRowsParams &p) {
         hipLaunchKernelGGL(k_mfma_rows<4>, dim3((unsigned)p.Mpad), dim3(256), 0, st, p);
 }
 
-template <int MT>
+template <int MT, bool FULL>
 static void launch_gemm_mfma_mt(hipStream_t st, const GemmMfmaParams &p, int sw, int kc) {
     const dim3 grid((unsigned)(p.w.N / 32), (unsigned)kc);
     switch (sw) {
-        case 8: hipLaunchKernelGGL((k_gemm_mfma<MT, 8>), grid, dim3(256), 0, st, p); break;
-        case 4: hipLaunchKernelGGL((k_gemm_mfma<MT, 4>), grid, dim3(256), 0, st, p); break;
-        case 2: hipLaunchKernelGGL((k_gemm_mfma<MT, 2>), grid, dim3(256), 0, st, p); break;
-        default: hipLaunchKernelGGL((k_gemm_mfma<MT, 1>), grid, dim3(256), 0, st, p); break;
+        case 8: hipLaunchKernelGGL((k_gemm_mfma<MT, 8, FULL>), grid, dim3(256), 0, st, p); break;
+        case 4: hipLaunchKernelGGL((k_gemm_mfma<MT, 4, FULL>), grid, dim3(256), 0, st, p); break;
+        case 2: hipLaunchKernelGGL((k_gemm_mfma<MT, 2, FULL>), grid, dim3(256), 0, st, p); break;
+        default: hipLaunchKernelGGL((k_gemm_mfma<MT, 1, FULL>), grid, dim3(256), 0, st, p); break;
     }
 }
 
 void launch_gemm_mfma(hipStream_t st, const GemmMfmaParams &p, int mt, int sw, int kc) {
-    if (mt == 1)
-        launch_gemm_mfma_mt<1>(st, p, sw, kc);
+    if (p.full)
+        mt == 1 ? launch_gemm_mfma_mt<1, true>(st, p, sw, kc) : launch_gemm_mfma_mt<2, true>(st, p, sw, kc);
     else
-        launch_gemm_mfma_mt<2>(st, p, sw, kc);
+        mt == 1 ? launch_gemm_mfma_mt<1, false>(st, p, sw, kc) : launch_gemm_mfma_mt<2, false>(st, p, sw, kc);
 }
 
-void launch_gemm_mfma_tile(hipStream_t st, const GemmMfmaParams &p, const GemmTilePlan &t) {
+template <bool FULL>
+static void launch_gemm_mfma_tile_full(hipStream_t st, const GemmMfmaParams &p, const GemmTilePlan &t) {
     const int total = t.mb * t.nb * t.kc;
     const dim3 grid((unsigned)((total + 7) / 8 * 8)), block(64 * t.nw);
     if (t.nw == 8) {
-        hipLaunchKernelGGL((k_gemm_mfma_tile<4, 8>), grid, block, 0, st, p, t);
+        hipLaunchKernelGGL((k_gemm_mfma_tile<4, 8, FULL>), grid, block, 0, st, p, t);
         return;
     }
     switch (t.mt) {
-        case 4: hipLaunchKernelGGL((k_gemm_mfma_tile<4, 4>), grid, block, 0, st, p, t); break;
-        case 3: hipLaunchKernelGGL((k_gemm_mfma_tile<3, 4>), grid, block, 0, st, p, t); break;
-        case 2: hipLaunchKernelGGL((k_gemm_mfma_tile<2, 4>), grid, block, 0, st, p, t); break;
-        default: hipLaunchKernelGGL((k_gemm_mfma_tile<1, 4>), grid, block, 0, st, p, t); break;
+        case 4: hipLaunchKernelGGL((k_gemm_mfma_tile<4, 4, FULL>), grid, block, 0, st, p, t); break;
+        case 3: hipLaunchKernelGGL((k_gemm_mfma_tile<3, 4, FULL>), grid, block, 0, st, p, t); break;
+        case 2: hipLaunchKernelGGL((k_gemm_mfma_tile<2, 4, FULL>), grid, block, 0, st, p, t); break;
+        default: hipLaunchKernelGGL((k_gemm_mfma_tile<1, 4, FULL>), grid, block, 0, st, p, t); break;
     }
+}
+
+void launch_gemm_mfma_tile(hipStream_t st, const GemmMfmaParams &p, const GemmTilePlan &t) {
+    p.full ? launch_gemm_mfma_tile_full<true>(st, p, t) : launch_gemm_mfma_tile_full<false>(st, p, t);
 }
 
 void launch_attn_prefill(hipStream_t st, const AttnParams &p, int M) {
