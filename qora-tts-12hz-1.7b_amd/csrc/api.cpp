@@ -3108,9 +3108,17 @@ struct DecConvMfma {
     int ew = 0, mtiles = 0, ksteps = 0, cin16 = 0;
 };
 
+// A residual unit's SnakeBeta factors, exp(alpha) and exp(-beta), where
+// k_dec_resunit takes the unit (ea1 null otherwise).
+struct DecResUnit {
+    float *ea1 = nullptr, *eb1 = nullptr, *ea2 = nullptr, *eb2 = nullptr;
+    float ebmax = 0.0f;
+};
+
 struct qtts_decoder {
     qtts_ctx *ctx = nullptr;
     Owner own;
+    std::vector<std::vector<DecResUnit>> res_unit;  // [block][unit]
     // the Vocos convolutions on the matrix cores: [block][unit][conv1, conv2]
     // and [block][output phase] of each block's transposed convolution
     std::vector<std::vector<std::array<DecConvMfma, 2>>> res_mfma;
@@ -3592,6 +3600,7 @@ qtts_status dec_decode(qtts_decoder *d, const uint32_t *d_codes, int T, int ld, 
     // that next reads sig adds it and stores the sum (faster than the conv2
     // epilogue reading each residual), the same f32 addition
     float *pend = nullptr;
+    const bool fuse = !std::getenv("QTTS_DEC_CONV");  // set: every layer through the kernel it names
     for (size_t bi = 0; bi < d->blocks.size(); bi++) {
         const qtts_vocos_block_view &b = d->blocks[bi];
         const int cin = b.upsample.in_channels, cout = b.upsample.out_channels;
@@ -3605,9 +3614,43 @@ qtts_status dec_decode(qtts_decoder *d, const uint32_t *d_codes, int T, int ld, 
         L *= b.upsample.stride;
         sig = nxt;
         float *t2 = other(sig, t1);
+        unsigned *msig = nullptr;  // max |sig|, where a fused unit recorded it
         for (int r = 0; r < b.num_residuals; r++) {
             const qtts_vocos_residual_view &rv = b.residuals[r];
             const std::array<DecConvMfma, 2> &mc = d->res_mfma[bi][(size_t)r];
+            const DecResUnit &ru = d->res_unit[bi][(size_t)r];
+            if (ru.ea1 && !pend && fuse) {
+                if (!msig) QTTS_TRY(maxof(sig, (size_t)cout * L, &msig));
+                DecResUnitParams p{};
+                p.x = sig;
+                p.out = t1;
+                p.len = L;
+                p.dilation = rv.conv1.dilation;
+                p.xmax = msig;
+                p.omax = take();
+                if (!p.omax) return fail(c, QTTS_EDEVICE, "decoder: more matrix-core inputs than max slots");
+                p.ea1 = ru.ea1;
+                p.eb1 = ru.eb1;
+                p.ea2 = ru.ea2;
+                p.eb2 = ru.eb2;
+                p.ebmax = ru.ebmax;
+                p.w1h = mc[0].wh;
+                p.w1l = mc[0].wl;
+                p.ew1 = mc[0].ew;
+                p.ksteps1 = mc[0].ksteps;
+                p.w2h = mc[1].wh;
+                p.w2l = mc[1].wl;
+                p.ew2 = mc[1].ew;
+                p.ksteps2 = mc[1].ksteps;
+                p.b1 = rv.conv1.bias;
+                p.b2 = rv.conv2.bias;
+                launch_dec_resunit(st, p, cout);
+                QTTS_TRY(check_launch(c, "k_dec_resunit"));
+                msig = p.omax;
+                std::swap(sig, t1);
+                continue;
+            }
+            msig = nullptr;
             unsigned *m1 = take(), *m2 = take();
             if (!m1 || !m2) return fail(c, QTTS_EDEVICE, "decoder: more matrix-core inputs than max slots");
             launch_dec_snake(st, sig, rv.act1_alpha, rv.act1_beta, cout, L, t1, m1, pend, pend ? sig : nullptr);
@@ -3765,6 +3808,7 @@ qtts_status qtts_decoder_upload(qtts_ctx *c, const qtts_decoder_view *v, qtts_de
     ch = v->vocos_init.out_channels;
     d->residuals.resize((size_t)std::max(v->num_vocos_blocks, 0));
     d->res_mfma.resize(d->residuals.size());
+    d->res_unit.resize(d->residuals.size());
     d->up_mfma.resize(d->residuals.size());
     for (int b = 0; b < v->num_vocos_blocks; b++) {
         const qtts_vocos_block_view &B = v->vocos_blocks[b];
@@ -3795,6 +3839,20 @@ qtts_status qtts_decoder_upload(qtts_ctx *c, const qtts_decoder_view *v, qtts_de
                 (s = dec_conv_mfma(c, o, R.conv2, E.conv2, &mc[1])) != QTTS_OK)
                 return bail(s);
             d->res_mfma[b].push_back(mc);
+            DecResUnit ru{};
+            if (R.conv1.bias && R.conv2.bias &&
+                dec_resunit_fits(ch, R.conv1.kernel_size, R.conv1.dilation, R.conv2.kernel_size)) {
+                float **const dst[4] = {&ru.ea1, &ru.eb1, &ru.ea2, &ru.eb2};
+                const float *const src[4] = {E.act1_alpha, E.act1_beta, E.act2_alpha, E.act2_beta};
+                for (int i = 0; i < 4; i++) {
+                    if ((s = o.alloc(c, dst[i], (size_t)ch)) != QTTS_OK) return bail(s);
+                    launch_dec_exp(c->stream, src[i], i & 1 ? -1.0f : 1.0f, ch, *dst[i]);
+                    if ((s = check_launch(c, "k_dec_exp")) != QTTS_OK) return bail(s);
+                }
+                for (int i = 0; i < ch; i++)  // a few ulps over the device's exp
+                    ru.ebmax = std::max(ru.ebmax, std::exp(-R.act1_beta[i]) * 1.0001f);
+            }
+            d->res_unit[b].push_back(ru);
             d->amax_slots += 2;
             d->residuals[b].push_back(E);
         }

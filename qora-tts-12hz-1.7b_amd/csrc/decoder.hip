@@ -22,6 +22,8 @@
 //                 k_dec_conv_win_tw, one channel tile per wave, at 3 and 4
 //                 tiles),
 //                 k_dec_conv_mfma_ks for launches too small to fill the GPU
+//  k_dec_resunit  a residual unit of 96 or 192 channels (both SnakeBetas,
+//                 both convolutions, the residual) in one launch
 //  k_dec_absmax   max |x| of a layer input (the operand scale)
 #include <hip/hip_runtime.h>
 
@@ -356,6 +358,7 @@ __global__ __launch_bounds__(256) void k_dec_absmax(const float *x, size_t n, un
     }
 }
 
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -888,6 +891,280 @@ __global__ __launch_bounds__(64 * NW) void k_dec_conv_win_tw(DecConvMfmaParams P
     }
 }
 
+// sin(t)^2 of SnakeBeta: t less the nearest multiple of pi (whose sine has
+// the same square), then sin r = r + r^3 p(r^2) on [-pi/2, pi/2], p fitted
+// for the least relative error (6e-9).  rms error 3.7e-8 over N(0, 6)
+// arguments, a correctly rounded sine's square 2.9e-8.  Past |t| = 8192,
+// where k * (pi - float(pi)) loses bits, the library's sinf.
+__device__ __forceinline__ float dec_sin2(float t) {
+    const float k = rintf(t * 0.318309886f);
+    float r = fmaf(-k, 3.14159274f, t);
+    r = fmaf(-k, -8.74227766e-8f, r);
+    const float z = r * r;
+    float p = fmaf(z, 2.60575049e-6f, -1.980959e-4f);
+    p = fmaf(z, p, 8.33306648e-3f);
+    p = fmaf(z, p, -0.166666597f);
+    float s = fmaf(r * z, p, r);
+    if (!(fabsf(t) <= 8192.0f)) s = sinf(t);
+    return s * s;
+}
+
+// A residual unit (src/decoder.rs:462-480) in one launch: out = x + conv2(
+// snake2(conv1(snake1(x)) + b1)) + b2, conv1 of 7 taps, conv2 of one, for C =
+// 32 CT channels.  As five launches it read and wrote the signal nine times;
+// here each block owns all C channels of P = 64 * 12 / CT positions:
+//   conv1: as k_dec_conv_win_tw, the window of 16 channels at a time staged
+//     position-major in LDS as binary16 hi + lo -- but from x, SnakeBeta
+//     applied as it is staged (once per block, since the block has every
+//     channel tile), interleaved with the MFMAs of the block before;
+//   snake2 of the accumulators, split into LDS as conv2's operand, scaled by
+//     the block's own largest value;
+//   conv2 from LDS, and the residual added from x.
+// 12 waves, wave w on channel tile w % CT and positions 64 (w / CT) ..: three
+// waves a SIMD, each A operand used for two 32-position tiles and shared
+// through L1 by the 12 / CT waves of its tile; A operands are loaded three
+// to four taps ahead.  conv1's operand scale bounds SnakeBeta by max |x| +
+// max exp(-beta), and max |out| is recorded for the next unit.
+// C = 96, 960,000 positions: 1130 us as five launches, 624 here; C = 192,
+// 240,000 positions: 1060, 665.  Matrix cores a third busy, vector ALU (the
+// sines and splits) a third, the rest latency: one block a CU.  Blocks of 6
+// waves and half the positions measured slower (C = 96, 805 us: twice the A
+// operands through the L2).
+template <int CT, int NWV>
+__global__ __launch_bounds__(64 * NWV, 3) void k_dec_resunit(DecResUnitParams P) {
+    static_assert(kDecMaxSlots == 64, "one max slot per lane");
+    constexpr int C = 32 * CT, PG = NWV / CT, NP = 64 * PG, TAPS = 7;
+    constexpr int WMAX = NP + 64;                     // window positions: NP + 6 * dilation at most
+    constexpr int SEG = WMAX / 64, ITEMS = 4 * SEG;   // (4 channels, 64 positions) per wave and pass
+    constexpr int PASSES = (ITEMS + NWV - 1) / NWV;
+    constexpr int NCB = C / 16;
+    union Lds {
+        struct {
+            _Float16 h[2][2][WMAX][8], l[2][2][WMAX][8];  // [buffer][8-channel half][position][channel]
+        } win;
+        struct {
+            _Float16 h[NCB][2][NP][8], l[NCB][2][NP][8];  // conv2's operand
+        } act;
+    };
+    __shared__ __align__(16) Lds sm;
+    __shared__ float red[NWV];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 31, half = lane >> 5;
+    const int tile = wave % CT, p0 = 64 * (wave / CT);  // this wave's channels and positions of the block
+    const int n0 = blockIdx.x * NP, len = P.len, dil = P.dilation;
+    const int w0 = n0 - (TAPS - 1) * dil, W = NP + (TAPS - 1) * dil;
+    const int ex = split_exponent(wave_max(__uint_as_float(P.xmax[lane])) + P.ebmax);
+    const float xs = ldexpf(1.0f, ex);
+
+    float v[PASSES][4];
+    auto load_win = [&](int cb) {
+#pragma unroll
+        for (int q = 0; q < PASSES; q++) {
+            const int it = wave + NWV * q;
+            if (it >= ITEMS) continue;  // uniform
+            const int g = it / SEG, pos = w0 + 64 * (it % SEG) + lane;
+            const float *xp = P.x + (size_t)(16 * cb + 4 * g) * len + min(max(pos, 0), len - 1);
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[q][j] = xp[(size_t)j * len];
+        }
+    };
+    auto put_win = [&](int cb, int q, int buf) {
+        const int it = wave + NWV * q;
+        if (it >= ITEMS) return;  // uniform
+        const int g = it / SEG, wp = 64 * (it % SEG) + lane, pos = w0 + wp;
+        const bool in = wp < W && pos >= 0 && pos < len;
+        half4 h, l;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const float x = in ? v[q][j] : 0.0f;
+            const int c = 16 * cb + 4 * g + j;  // uniform
+            const float o = (x + P.eb1[c] * dec_sin2(P.ea1[c] * x)) * xs;
+            h[j] = (_Float16)o;
+            l[j] = (_Float16)(o - (float)h[j]);
+        }
+        *reinterpret_cast<half4 *>(&sm.win.h[buf][g >> 1][wp][4 * (g & 1)]) = h;
+        *reinterpret_cast<half4 *>(&sm.win.l[buf][g >> 1][wp][4 * (g & 1)]) = l;
+    };
+    // A operands in two runs of taps, each loaded while the other is used
+    half8 a0h[4], a0l[4], a1h[3], a1l[3];
+    const half8 *w1h = reinterpret_cast<const half8 *>(P.w1h) + (size_t)tile * P.ksteps1 * 64 + lane;
+    const half8 *w1l = reinterpret_cast<const half8 *>(P.w1l) + (size_t)tile * P.ksteps1 * 64 + lane;
+    auto load_a0 = [&](int cb) {
+#pragma unroll
+        for (int t = 0; t < 4; t++) a0h[t] = w1h[(cb * TAPS + t) * 64], a0l[t] = w1l[(cb * TAPS + t) * 64];
+    };
+    auto load_a1 = [&](int cb) {
+#pragma unroll
+        for (int t = 0; t < 3; t++) a1h[t] = w1h[(cb * TAPS + 4 + t) * 64], a1l[t] = w1l[(cb * TAPS + 4 + t) * 64];
+    };
+    f32x16 acc[2];
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[t][r] = 0.0f;
+    auto mma = [&](int buf, int tap, const half8 &ah, const half8 &al) {
+        half8 bh[2], bl[2];
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const int p = p0 + 32 * t + col + tap * dil;
+            bh[t] = *reinterpret_cast<const half8 *>(&sm.win.h[buf][half][p][0]);
+            bl[t] = *reinterpret_cast<const half8 *>(&sm.win.l[buf][half][p][0]);
+        }
+#pragma unroll
+        for (int t = 0; t < 2; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh[t], acc[t], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < 2; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl[t], acc[t], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < 2; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh[t], acc[t], 0, 0, 0);
+    };
+    load_win(0);
+    load_a0(0);
+#pragma unroll
+    for (int q = 0; q < PASSES; q++) put_win(0, q, 0);
+    __syncthreads();
+    for (int cb = 0; cb < NCB; cb++) {
+        const int buf = cb & 1;
+        const bool more = cb + 1 < NCB;  // uniform
+        if (more) load_win(cb + 1);
+        load_a1(cb);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < 4; t++) mma(buf, t, a0h[t], a0l[t]);
+        __builtin_amdgcn_sched_barrier(0);
+        load_a0(more ? cb + 1 : cb);
+        if (more) put_win(cb + 1, 0, buf ^ 1);  // last read in channel block cb - 1
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int t = 0; t < 3; t++) mma(buf, 4 + t, a1h[t], a1l[t]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (more)
+#pragma unroll
+            for (int q = 1; q < PASSES; q++) put_win(cb + 1, q, buf ^ 1);
+        __syncthreads();
+    }
+
+    // snake2 of this wave's [32 channels][64 positions]; D layout: lane l,
+    // register r -> row (r / 4) * 8 + (l / 32) * 4 + r % 4, column l % 32
+    const int sc1 = -(ex + P.ew1);
+    float m = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int c = 32 * tile + 8 * j + 4 * half;
+        const float4 b = *reinterpret_cast<const float4 *>(P.b1 + c);
+        const float4 a = *reinterpret_cast<const float4 *>(P.ea2 + c), e = *reinterpret_cast<const float4 *>(P.eb2 + c);
+        const float bv[4] = {b.x, b.y, b.z, b.w}, av[4] = {a.x, a.y, a.z, a.w}, ev[4] = {e.x, e.y, e.z, e.w};
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const bool in = n0 + p0 + 32 * t + col < len;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float x = ldexpf(acc[t][4 * j + i], sc1) + bv[i];
+                const float o = x + ev[i] * dec_sin2(av[i] * x);
+                acc[t][4 * j + i] = in ? o : 0.0f;
+                m = fmaxf(m, fabsf(acc[t][4 * j + i]));
+            }
+        }
+    }
+    m = wave_max(m);
+    if (lane == 0) red[wave] = m;
+    __syncthreads();  // also: the last window is read
+    m = red[0];
+#pragma unroll
+    for (int w = 1; w < NWV; w++) m = fmaxf(m, red[w]);
+    const int ex2 = split_exponent(m);
+    const float xs2 = ldexpf(1.0f, ex2);
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            half4 h, l;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float o = acc[t][4 * j + i] * xs2;
+                h[i] = (_Float16)o;
+                l[i] = (_Float16)(o - (float)h[i]);
+            }
+            const int p = p0 + 32 * t + col;
+            *reinterpret_cast<half4 *>(&sm.act.h[2 * tile + (j >> 1)][j & 1][p][4 * half]) = h;
+            *reinterpret_cast<half4 *>(&sm.act.l[2 * tile + (j >> 1)][j & 1][p][4 * half]) = l;
+        }
+    // the residual, under conv2
+    float x[2][16];
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int c = 32 * tile + (r >> 2) * 8 + half * 4 + (r & 3);
+            x[t][r] = P.x[(size_t)c * len + min(n0 + p0 + 32 * t + col, len - 1)];
+        }
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[t][r] = 0.0f;
+    const half8 *w2h = reinterpret_cast<const half8 *>(P.w2h) + (size_t)tile * P.ksteps2 * 64 + lane;
+    const half8 *w2l = reinterpret_cast<const half8 *>(P.w2l) + (size_t)tile * P.ksteps2 * 64 + lane;
+    half8 ch[2][3], cl[2][3];
+    auto load_c = [&](int s, int to) {
+#pragma unroll
+        for (int i = 0; i < 3; i++) ch[to][i] = w2h[(s + i) * 64], cl[to][i] = w2l[(s + i) * 64];
+    };
+    load_c(0, 0);
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < NCB; s += 3) {
+        const int b = (s / 3) & 1;
+        if (s + 3 < NCB) load_c(s + 3, b ^ 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            half8 bh[2], bl[2];
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                bh[t] = *reinterpret_cast<const half8 *>(&sm.act.h[s + i][half][p0 + 32 * t + col][0]);
+                bl[t] = *reinterpret_cast<const half8 *>(&sm.act.l[s + i][half][p0 + 32 * t + col][0]);
+            }
+#pragma unroll
+            for (int t = 0; t < 2; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ch[b][i], bh[t], acc[t], 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < 2; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ch[b][i], bl[t], acc[t], 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < 2; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(cl[b][i], bh[t], acc[t], 0, 0, 0);
+        }
+    }
+    const int sc2 = -(ex2 + P.ew2);
+    m = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int c = 32 * tile + 8 * j + 4 * half;
+        const float4 b = *reinterpret_cast<const float4 *>(P.b2 + c);
+        const float bv[4] = {b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const int n = n0 + p0 + 32 * t + col;
+            if (n >= len) continue;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float o = x[t][4 * j + i] + (ldexpf(acc[t][4 * j + i], sc2) + bv[i]);
+                m = fmaxf(m, fabsf(o));
+                P.out[(size_t)(c + i) * len + n] = o;
+            }
+        }
+    }
+    m = wave_max(m);
+    if (lane == 0) red[wave] = m;  // last read two barriers ago
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < NWV; w++) m = fmaxf(m, red[w]);
+        atomicMax(&P.omax[blockIdx.x % kDecMaxSlots], __float_as_uint(m));
+    }
+}
+
+// out[i] = exp(sign * x[i])
+__global__ void k_dec_exp(const float *x, float sign, int n, float *out) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) out[i] = expf(sign * x[i]);
+}
+
 unsigned blocks_for(size_t n, unsigned per) { return (unsigned)((n + per - 1) / per); }
 
 }  // namespace
@@ -1012,6 +1289,25 @@ void launch_dec_absmax(hipStream_t st, const float *x, size_t n, unsigned *amax)
     // with one atomic, so fewer blocks queue fewer atomics per slot
     const unsigned blocks = std::min<unsigned>(blocks_for((n + 3) / 4, 256), 512u);
     hipLaunchKernelGGL(k_dec_absmax, dim3(blocks), dim3(256), 0, st, x, n, amax);
+}
+
+// 3 or 6 channel tiles (12 waves a block, conv2's operand at most 96 KiB of
+// LDS) and a window of at most 64 positions before the block's.  At 384
+// channels a block would hold 64 positions and read 4.1 MB of weights for
+// them, more than the L2 gives in the time of its MFMAs.
+bool dec_resunit_fits(int channels, int ksize1, int dilation, int ksize2) {
+    return (channels == 96 || channels == 192) && ksize1 == 7 && dilation >= 1 && dilation <= 10 && ksize2 == 1;
+}
+
+void launch_dec_resunit(hipStream_t st, const DecResUnitParams &p, int channels) {
+    if (channels == 96)
+        hipLaunchKernelGGL((k_dec_resunit<3, 12>), dim3(blocks_for((size_t)p.len, 256)), dim3(768), 0, st, p);
+    else
+        hipLaunchKernelGGL((k_dec_resunit<6, 12>), dim3(blocks_for((size_t)p.len, 128)), dim3(768), 0, st, p);
+}
+
+void launch_dec_exp(hipStream_t st, const float *x, float sign, int n, float *out) {
+    hipLaunchKernelGGL(k_dec_exp, dim3(blocks_for((size_t)n, 256)), dim3(256), 0, st, x, sign, n, out);
 }
 
 }  // namespace qtts

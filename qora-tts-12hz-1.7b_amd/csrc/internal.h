@@ -132,6 +132,21 @@ struct DecConvMfmaParams {
     const _Float16 *ph_wh[kDecMaxPhases], *ph_wl[kDecMaxPhases];
 };
 
+// One residual unit (k_dec_resunit): x, out [C][len], distinct buffers; the
+// convolutions' operand copies as in DecConvMfmaParams.
+struct DecResUnitParams {
+    const float *x;
+    float *out;
+    int len, dilation;
+    const unsigned *xmax;  // [kDecMaxSlots]: max |x|
+    unsigned *omax;        // [kDecMaxSlots]: receives max |out|
+    const float *ea1, *eb1, *ea2, *eb2;  // exp(alpha), exp(-beta) of both SnakeBetas
+    float ebmax;                         // at least max eb1
+    const _Float16 *w1h, *w1l, *w2h, *w2l;
+    int ew1, ew2, ksteps1, ksteps2;
+    const float *b1, *b2;
+};
+
 struct DecAttnParams {
     const float *q, *k, *v;  // rows of heads * hd values, ld apart (0: heads * hd)
     int ld;
@@ -360,6 +375,11 @@ void launch_dec_absmax(hipStream_t st, const float *x, size_t n, unsigned *amax)
 void launch_dec_conv_repack(hipStream_t st, const float *w, long long sm, long long sci, int k0, int kd, int M, int cin,
                             int taps, int cin16, int mtiles, int ksteps, int ew, _Float16 *wh, _Float16 *wl);
 void launch_dec_conv_mfma(hipStream_t st, const DecConvMfmaParams &p);
+// Whether k_dec_resunit takes a residual unit of these shapes.
+bool dec_resunit_fits(int channels, int ksize1, int dilation, int ksize2);
+void launch_dec_resunit(hipStream_t st, const DecResUnitParams &p, int channels);
+// out[i] = exp(sign * x[i]) for i < n
+void launch_dec_exp(hipStream_t st, const float *x, float sign, int n, float *out);
 void launch_gemm_mfma(hipStream_t st, const GemmMfmaParams &p, int mt, int sw, int kc);
 // q, kcache, vcache, kv_cap, nq, nkv, scale and out of p; head_dim 128; M rows into an empty cache
 void launch_attn_prefill(hipStream_t st, const AttnParams &p, int M);

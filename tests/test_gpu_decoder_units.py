@@ -1,0 +1,46 @@
+"""Residual units of 96 and 192 channels (one launch each) against the oracle
+and against the same decoder with every layer a launch of its own: lengths off
+the 128- and 256-position blocks and shorter than a window, the largest
+dilation the unit takes and one past it, and SnakeBeta factors up to e^3."""
+import numpy as np
+import pytest
+
+import qtts
+from oracle import oracle
+from shapes import rel_err, within
+
+pytestmark = pytest.mark.gpu
+
+
+def _decoder(ctx, dilations, big=False):
+    cfg = qtts.DecoderConfig(hidden=32, heads=2, head_dim=16, inter=64, window=8, codebook_dim=16, codebook_size=64,
+                             vq_dim=32, latent=32, num_rest=3, layers=1, upsample=(1,), vocos_channels=64,
+                             vocos=((64, 192, 6, 3), (192, 96, 4, 2)), dilations=dilations, rope_rows=64)
+    w = qtts.DecoderWeights(17, cfg)
+    if big:
+        # SnakeBeta at arguments of tens of periods.  Its slope 1 + exp(alpha -
+        # beta) sin(2 t) stays below 2, so that four units' two SnakeBetas
+        # magnify a rounding at most 2^8 times (steeper ones are chaotic and
+        # compare nothing).
+        for b in w.blocks:
+            for r in b["residuals"]:
+                r["act1_alpha"][::5] = r["act1_beta"][::5] = 3.0
+                r["act2_alpha"][::3] = r["act2_beta"][::3] = 4.0
+    return w, qtts.SpeechDecoder(ctx, w)
+
+
+@pytest.mark.parametrize("frames,dilations,big", [(1, (1, 3, 9), False), (43, (1, 3, 9), False), (44, (10,), False),
+                                                  (60, (11, 2), False), (64, (9, 1), True), (128, (3,), True)])
+def test_residual_units(ctx, monkeypatch, frames, dilations, big):
+    w, dec = _decoder(ctx, dilations, big)
+    codes = w.synthetic_codes(18, frames)
+    got = dec.decode_to_audio(codes)
+    ref = oracle.decode_to_audio(w, codes)
+    monkeypatch.setenv("QTTS_DEC_CONV", "tiles")
+    apart = dec.decode_to_audio(codes)
+    print(f"{frames} frames: {got.size} samples, rel err {rel_err(got, ref):.2e}, apart {rel_err(apart, ref):.2e}")
+    assert got.shape == ref.shape
+    # f32 rounding through the same stages as the small decoder's (2e-6 there),
+    # times the magnification above where it applies
+    assert within(got, ref, tight=2.0 ** 8 * 2e-6 if big else 3e-5)
+    assert rel_err(got, ref) <= 3.0 * rel_err(apart, ref) + 1e-6
