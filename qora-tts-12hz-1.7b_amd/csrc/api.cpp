@@ -3476,6 +3476,11 @@ qtts_status dec_decode(qtts_decoder *d, const uint32_t *d_codes, int T, int ld, 
         launch_dec_absmax(st, x, n, *out);
         return check_launch(c, "k_dec_absmax");
     };
+    // the slots of an input whose max |x| its own kernel records
+    auto own = [&](unsigned **out) -> qtts_status {
+        *out = take();
+        return *out ? QTTS_OK : fail(c, QTTS_EDEVICE, "decoder: more matrix-core inputs than max slots");
+    };
     unsigned *mx = nullptr, *mx2 = nullptr;
     // 1. codebook lookup -> S0 [vq][T] (src/decoder.rs:142-189)
     DecGatherParams g{};
@@ -3515,9 +3520,9 @@ qtts_status dec_decode(qtts_decoder *d, const uint32_t *d_codes, int T, int ld, 
     for (size_t li = 0; li < d->layers.size(); li++) {
         const qtts_dec_layer_view &L = d->layers[li];
         const std::array<DecConvMfma, 7> &lm = d->layer_mfma[li];
-        launch_dec_rmsnorm(st, X, L.input_norm, T, hid, 1e-5f, XN);
+        QTTS_TRY(own(&mx));
+        launch_dec_rmsnorm(st, X, L.input_norm, T, hid, 1e-5f, XN, mx);
         QTTS_TRY(check_launch(c, "k_dec_rmsnorm"));
-        QTTS_TRY(maxof(XN, (size_t)T * hid, &mx));
         if (d->cat) {
             // q|k|v in one launch: row t holds q, k, v side by side (3 * ad)
             QTTS_TRY(dec_linear_mfma(d, d->layer_cat[li][0], XN, hid, 1, T, hid, 3 * ad, mx, nullptr, QKV, 3 * ad, 1,
@@ -3534,32 +3539,34 @@ qtts_status dec_decode(qtts_decoder *d, const uint32_t *d_codes, int T, int ld, 
         launch_dec_rope(st, const_cast<float *>(a.q), const_cast<float *>(a.k), T, w.num_heads, w.head_dim, w.rope_cos,
                         w.rope_sin, w.rope_rows, a.ld);
         QTTS_TRY(check_launch(c, "k_dec_rope"));
+        QTTS_TRY(own(&mx));
+        a.amax = mx;
         launch_dec_attn(st, a);
         QTTS_TRY(check_launch(c, "k_dec_attn"));
-        QTTS_TRY(maxof(AO, (size_t)T * ad, &mx));
         QTTS_TRY(dec_linear_mfma(d, lm[3], AO, ad, 1, T, ad, hid, mx, nullptr, X, hid, 1, DEC_EPI_SCALED_RESID,
                                  L.attn_scale));
-        launch_dec_rmsnorm(st, X, L.post_attn_norm, T, hid, 1e-5f, XN);
+        QTTS_TRY(own(&mx));
+        launch_dec_rmsnorm(st, X, L.post_attn_norm, T, hid, 1e-5f, XN, mx);
         QTTS_TRY(check_launch(c, "k_dec_rmsnorm"));
-        QTTS_TRY(maxof(XN, (size_t)T * hid, &mx));
         if (d->cat) {
             // gate|up in one launch (row t: gate then up), SiLU(gate) * up into G
             QTTS_TRY(dec_linear_mfma(d, d->layer_cat[li][1], XN, hid, 1, T, hid, 2 * inter, mx, nullptr, GU, 2 * inter,
                                      1, DEC_EPI_STORE));
-            launch_dec_swiglu(st, GU, GU + inter, T, inter, 2 * inter, G);
+            QTTS_TRY(own(&mx));
+            launch_dec_swiglu(st, GU, GU + inter, T, inter, 2 * inter, G, mx);
         } else {
             QTTS_TRY(dec_linear_mfma(d, lm[4], XN, hid, 1, T, hid, inter, mx, nullptr, G, inter, 1, DEC_EPI_STORE));
             QTTS_TRY(dec_linear_mfma(d, lm[5], XN, hid, 1, T, hid, inter, mx, nullptr, U, inter, 1, DEC_EPI_STORE));
-            launch_dec_swiglu(st, G, U, T, inter, inter, G);
+            QTTS_TRY(own(&mx));
+            launch_dec_swiglu(st, G, U, T, inter, inter, G, mx);
         }
         QTTS_TRY(check_launch(c, "k_dec_swiglu"));
-        QTTS_TRY(maxof(G, (size_t)T * inter, &mx));
         QTTS_TRY(dec_linear_mfma(d, lm[6], G, inter, 1, T, inter, hid, mx, nullptr, X, hid, 1, DEC_EPI_SCALED_RESID,
                                  L.mlp_scale));
     }
-    launch_dec_rmsnorm(st, X, w.tf_norm, T, hid, 1e-5f, XN);
+    QTTS_TRY(own(&mx));
+    launch_dec_rmsnorm(st, X, w.tf_norm, T, hid, 1e-5f, XN, mx);
     QTTS_TRY(check_launch(c, "k_dec_rmsnorm"));
-    QTTS_TRY(maxof(XN, (size_t)T * hid, &mx));
     QTTS_TRY(dec_linear_mfma(d, d->tf_out, XN, hid, 1, T, hid, lat, mx, w.tf_output_b, S0, 1, T, DEC_EPI_STORE));
     // 4. upsample: transposed conv + ConvNeXt (src/decoder.rs:336-388, 424-448)
     float *const pool[4] = {S0, S1, S2, S3};
@@ -3578,9 +3585,9 @@ qtts_status dec_decode(qtts_decoder *d, const uint32_t *d_codes, int T, int ld, 
         L *= u.conv_t.stride;
         launch_dec_dwconv(st, up, u.dw_conv.weight, u.dw_conv.bias, u.channels, L, u.dw_conv.kernel_size, dw);
         QTTS_TRY(check_launch(c, "k_dec_dwconv"));
-        launch_dec_lnorm(st, dw, u.norm_w, u.norm_b, u.channels, L, 1e-5f, nrm);
+        QTTS_TRY(own(&mx));
+        launch_dec_lnorm(st, dw, u.norm_w, u.norm_b, u.channels, L, 1e-5f, nrm, mx);
         QTTS_TRY(check_launch(c, "k_dec_lnorm"));
-        QTTS_TRY(maxof(nrm, (size_t)u.channels * L, &mx));
         QTTS_TRY(dec_linear_mfma(d, d->pw_mfma[ui][0], nrm, 1, L, L, u.channels, u.inner_dim, mx, u.pw1_b, P1,
                                  u.inner_dim, 1, DEC_EPI_STORE, nullptr, nullptr, DEC_ACT_GELU));
         // out = residual + gamma * pw2 (the residual is the stage input `up`)

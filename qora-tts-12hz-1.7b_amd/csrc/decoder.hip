@@ -9,8 +9,8 @@
 //  k_dec_swiglu   silu(gate) * up
 //  k_dec_dwconv   causal depthwise convolution (src/conv.rs:280-345)
 //  k_dec_lnorm    channel-first LayerNorm per time step, channels summed in
-//                 order (src/decoder.rs:580-602); k_dec_lnorm_tile the same
-//                 over an LDS tile of 16 or 8 time steps
+//                 order (src/decoder.rs:580-602); k_dec_lnorm_tile over an
+//                 LDS tile of 16 or 8 time steps, several threads a step
 //  k_dec_snake    SnakeBeta (src/conv.rs:347-400), optionally recording
 //                 max |out| for the convolution that reads it
 //  k_dec_conv_mfma  every projection and convolution on the matrix cores
@@ -71,8 +71,21 @@ __global__ void k_dec_gather(DecGatherParams P) {
 // GELU, the tanh form the reference uses.
 __device__ __forceinline__ float dec_gelu(float x) { return x * 0.5f * (1.0f + tanhf(x * 0.7071067811865476f)); }
 
+// max over a block of 256 threads into *slot: unsigned order is float order
+// for non-negative values.  red: 4 words nothing reads any more.
+__device__ __forceinline__ void block_amax(float m, float *red, unsigned *slot) {
+    m = wave_max(m);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        atomicMax(slot, __float_as_uint(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]))));
+}
+
 // rms_norm_f32 of each of `rows` rows of n values: one block per row.
-__global__ __launch_bounds__(256) void k_dec_rmsnorm(const float *x, const float *gamma, int n, float eps, float *out) {
+// max |out| (NaN excluded) goes into the slots of amax, as k_dec_snake's.
+__global__ __launch_bounds__(256) void k_dec_rmsnorm(const float *x, const float *gamma, int n, float eps, float *out,
+                                                     unsigned *amax) {
     __shared__ float red[4];
     const float *r = x + (size_t)blockIdx.x * n;
     float ss = 0.0f;
@@ -82,7 +95,13 @@ __global__ __launch_bounds__(256) void k_dec_rmsnorm(const float *x, const float
     __syncthreads();
     ss = (red[0] + red[1]) + (red[2] + red[3]);
     const float inv = 1.0f / sqrtf(ss / (float)n + eps);
-    for (int i = threadIdx.x; i < n; i += 256) out[(size_t)blockIdx.x * n + i] = r[i] * inv * gamma[i];
+    float m = 0.0f;
+    for (int i = threadIdx.x; i < n; i += 256) {
+        const float v = r[i] * inv * gamma[i];
+        m = fmaxf(m, fabsf(v));
+        out[(size_t)blockIdx.x * n + i] = v;
+    }
+    block_amax(m, red, &amax[blockIdx.x % kDecMaxSlots]);
 }
 
 // Split-half rotation of q and k at position = frame; no rotation past the
@@ -140,19 +159,30 @@ __global__ __launch_bounds__(256) void k_dec_attn(DecAttnParams P) {
         inv = 1.0f / wave_sum(sum);
     }
     __syncthreads();
+    float m = 0.0f;
     if (valid)
         for (int d = lane; d < P.hd; d += 64) {
             float o = 0.0f;
             for (int s = 0; s < n; s++) o += (ps[wave][s] * inv) * P.v[(size_t)(start + s) * ld + (size_t)h * P.hd + d];
             P.out[(size_t)t * ad + (size_t)h * P.hd + d] = o;
+            m = fmaxf(m, fabsf(o));
         }
+    block_amax(m, &qs[0][0], &P.amax[blockIdx.x % kDecMaxSlots]);  // qs was last read before the last barrier
 }
 
-__global__ void k_dec_swiglu(const float *g, const float *u, int rows, int width, int ld, float *out) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)rows * width) return;
-    const size_t t = i / width, j = i - t * width, a = t * ld + j;
-    out[i] = (g[a] / (1.0f + expf(-g[a]))) * u[a];
+// silu(g) * u, max |out| into the slots of amax.
+__global__ __launch_bounds__(256) void k_dec_swiglu(const float *g, const float *u, int rows, int width, int ld,
+                                                    float *out, unsigned *amax) {
+    __shared__ float red[4];
+    const size_t n = (size_t)rows * width, stride = (size_t)gridDim.x * blockDim.x;
+    float m = 0.0f;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+        const size_t t = i / width, j = i - t * width, a = t * ld + j;
+        const float v = (g[a] / (1.0f + expf(-g[a]))) * u[a];
+        m = fmaxf(m, fabsf(v));
+        out[i] = v;
+    }
+    block_amax(m, red, &amax[blockIdx.x % kDecMaxSlots]);
 }
 
 // Causal depthwise convolution (padding kernel_size - 1), channel-first.
@@ -207,17 +237,17 @@ __global__ __launch_bounds__(64) void k_dec_lnorm(const float *x, const float *g
 
 // The same LayerNorm with TS time steps per block: the block's [ch][TS]
 // input tile is loaded once into LDS (TS consecutive steps of a channel are
-// consecutive addresses, 16 loads per thread in flight), thread t < TS runs
-// step t's two channel sums in channel order from LDS -- the arithmetic of
-// k_dec_lnorm, so the output is the same bit for bit -- and every thread
-// writes the normalised tile.  One global round trip instead of one per 8
-// channels of each pass.
+// consecutive addresses, 16 loads per thread in flight), 256 / TS threads
+// share a step's channel sums (each a run of every (256 / TS)-th channel,
+// then added in a fixed order), and every thread writes the normalised tile,
+// with max |out| into the slots of amax.  With one thread per step the two
+// sums over 1024 channels were 30 of 39 us at 26 steps.
 template <int TS>
 __global__ __launch_bounds__(256) void k_dec_lnorm_tile(const float *x, const float *g, const float *b, int ch, int len,
-                                                        float eps, float *out) {
+                                                        float eps, float *out, unsigned *amax) {
     extern __shared__ float tile[];  // [ch][TS]
-    __shared__ float s_mean[TS], s_inv[TS];
-    constexpr int U = 16;
+    constexpr int U = 16, R = 256 / TS;
+    __shared__ float part[R][TS];
     const int t0 = blockIdx.x * TS, tid = threadIdx.x;
     const int n = min(TS, len - t0);
     const int total = ch * TS;
@@ -235,23 +265,33 @@ __global__ __launch_bounds__(256) void k_dec_lnorm_tile(const float *x, const fl
         }
     }
     __syncthreads();
-    if (tid < n) {
-        float mean = 0.0f;
-        for (int c = 0; c < ch; c++) mean += tile[c * TS + tid];
-        mean /= (float)ch;
-        float var = 0.0f;
-        for (int c = 0; c < ch; c++) {
-            const float d = tile[c * TS + tid] - mean;
-            var += d * d;
+    const int j = tid % TS, r = tid / TS;
+    auto sum = [&](float v) {  // over the R threads of step j
+        part[r][j] = v;
+        __syncthreads();
+        float s = 0.0f;
+#pragma unroll
+        for (int i = 0; i < R; i++) s += part[i][j];
+        __syncthreads();
+        return s;
+    };
+    float acc = 0.0f;
+    for (int c = r; c < ch; c += R) acc += tile[c * TS + j];
+    const float mean = sum(acc) / (float)ch;
+    acc = 0.0f;
+    for (int c = r; c < ch; c += R) {
+        const float d = tile[c * TS + j] - mean;
+        acc += d * d;
+    }
+    const float inv = 1.0f / sqrtf(sum(acc) / (float)ch + eps);
+    float m = 0.0f;
+    if (j < n)
+        for (int c = r; c < ch; c += R) {
+            const float v = (tile[c * TS + j] - mean) * inv * g[c] + b[c];
+            m = fmaxf(m, fabsf(v));
+            out[(size_t)c * len + t0 + j] = v;
         }
-        s_mean[tid] = mean;
-        s_inv[tid] = 1.0f / sqrtf(var / (float)ch + eps);
-    }
-    __syncthreads();
-    for (int i = tid; i < total; i += 256) {
-        const int c = i / TS, j = i - c * TS;
-        if (j < n) out[(size_t)c * len + t0 + j] = (tile[i] - s_mean[j]) * s_inv[j] * g[c] + b[c];
-    }
+    block_amax(m, &part[0][0], &amax[blockIdx.x % kDecMaxSlots]);
 }
 
 // With add set, the input is x + add, stored to sum (which may be x: each
@@ -548,90 +588,115 @@ __global__ __launch_bounds__(256) void k_dec_conv_mfma(DecConvMfmaParams P) {
 }
 
 // The same product for launches too small to fill the GPU (the transformer's
-// linears at 500 rows, the first Vocos stages): one block per (32 output
-// steps, channel tile), its 4 waves splitting the K steps four ways (each
-// wave loads its own A operands and gathers its own B), the partial sums
-// added through LDS in wave order (deterministic) by wave 0, which runs the
-// epilogue.  A quarter of the dependent step chain per wave and four times
-// the blocks of k_dec_conv_mfma<1>.
-template <bool KF>
-__global__ __launch_bounds__(256) void k_dec_conv_mfma_ks(DecConvMfmaParams P) {
+// linears, the first Vocos stages; every layer of a short decode): one block
+// per (32 output steps, channel tile), its NW waves splitting the K steps.
+// Such a launch is one chain of loads, MFMAs and the sum, so each wave has
+// the operands of U steps in flight at once, and the waves' partials go
+// through LDS to all threads, one output each, added in wave order.
+// 13 frames: the transformer's linears 18 -> 6-10 us, 768 -> 768 channels of
+// 7 taps 85 -> 70 (four waves, one step ahead, before).
+template <bool KF, int NW>
+__global__ __launch_bounds__(64 * NW) void k_dec_conv_mfma_ks(DecConvMfmaParams P) {
     static_assert(kDecMaxSlots == 64, "one max slot per lane");
-    __shared__ float red[3][16][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int U = 4;
+    __shared__ float red[NW][16][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 31, half = lane >> 5;
-    const int n = blockIdx.x * 32 + col;
-    const int tile = blockIdx.y;
+    // Blocks of one XCD (every 8th) take a contiguous run of (phase, tile,
+    // positions), positions innermost: a tile's weights then come into one
+    // XCD's L2 only.
     const int len = P.len, ksteps = P.ksteps;
+    const int nx = (len + 31) / 32, total = nx * P.mtiles * max(1, P.nphase), per = (int)(gridDim.x >> 3);
+    const int L = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if (L >= total) return;
+    const int ty = __builtin_amdgcn_readfirstlane(L / nx), n = (L - ty * nx) * 32 + col;
+    const int z = __builtin_amdgcn_readfirstlane(ty / P.mtiles), tile = ty - z * P.mtiles;
     const bool multi = P.nphase > 1;  // uniform
-    const _Float16 *wh = multi ? P.ph_wh[blockIdx.z] : P.wh, *wl = multi ? P.ph_wl[blockIdx.z] : P.wl;
-    const int phase = multi ? (int)blockIdx.z : P.phase;
-    const int q = (ksteps + 3) / 4, s0 = wave * q, s1 = min(ksteps, s0 + q);
-    const int ex = split_exponent(wave_max(__uint_as_float(P.xmax[lane])));
-    const float xs = ldexpf(1.0f, ex);
-    const int cpl = P.cin - 8 * half;
-    auto load = [&](int s, half8 &ah, half8 &al, float (&xv)[8]) {
-        const int cb = s / P.ksize, tap = s - cb * P.ksize, ci0 = 16 * cb;  // wave-uniform
-        const int p = n + (tap - (P.ksize - 1)) * P.dilation;
-        const bool ok = n < len && p >= 0 && ci0 < cpl;
-        const float *xp = P.x + (long long)(ci0 + 8 * half) * P.sxc + (long long)(ok ? p : 0) * P.sxn;
-        if constexpr (KF) {
-            const float4 a = ok ? *reinterpret_cast<const float4 *>(xp) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            const float4 b = ok ? *reinterpret_cast<const float4 *>(xp + 4) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            xv[0] = a.x, xv[1] = a.y, xv[2] = a.z, xv[3] = a.w;
-            xv[4] = b.x, xv[5] = b.y, xv[6] = b.z, xv[7] = b.w;
-        } else {
+    const _Float16 *wh = P.wh, *wl = P.wl;
 #pragma unroll
-            for (int i = 0; i < 8; i++) xv[i] = ok && ci0 + i < cpl ? xp[(long long)i * P.sxc] : 0.0f;
+    for (int i = 0; i < kDecMaxPhases; i++)  // selected one by one: indexed by z, the parameters go to scratch
+        if (multi && z == i) wh = P.ph_wh[i], wl = P.ph_wl[i];
+    const int phase = multi ? z : P.phase;
+    const int q = (ksteps + NW - 1) / NW, s0 = wave * q, s1 = min(ksteps, s0 + q);
+    const unsigned xmax = P.xmax[lane];
+    const half8 *ah0 = reinterpret_cast<const half8 *>(wh) + (size_t)tile * ksteps * 64;
+    const half8 *al0 = reinterpret_cast<const half8 *>(wl) + (size_t)tile * ksteps * 64;
+    half8 ah[U], al[U];
+    float xv[U][8];
+    int cb = s0 / P.ksize, tap = s0 - cb * P.ksize;  // of the next step to load (uniform)
+    // Steps s .. s + U - 1; one past the wave's last loads valid operands and
+    // has a zero B.  A channel's row is a uniform address, the lane's
+    // position (and upper half of the channels) a 32-bit offset.
+    auto load = [&](int s) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int ci0 = 16 * cb, p = n + (tap - (P.ksize - 1)) * P.dilation;
+            const bool ok = s + u < s1 && n < len && p >= 0;
+            const size_t o = (size_t)min(s + u, ksteps - 1) * 64;
+            ah[u] = (ah0 + o)[lane];
+            al[u] = (al0 + o)[lane];
+            if constexpr (KF) {
+                // all 8 channels exist (cin % 8 == 0): two 16-byte loads
+                const bool in = ok && ci0 + 8 * half < P.cin;
+                const float *xp = P.x + (in ? (long long)p * P.sxn + ci0 + 8 * half : 0);
+                const float4 a = *reinterpret_cast<const float4 *>(xp), b = *reinterpret_cast<const float4 *>(xp + 4);
+                xv[u][0] = a.x, xv[u][1] = a.y, xv[u][2] = a.z, xv[u][3] = a.w;
+                xv[u][4] = b.x, xv[u][5] = b.y, xv[u][6] = b.z, xv[u][7] = b.w;
+#pragma unroll
+                for (int i = 0; i < 8; i++) xv[u][i] = in ? xv[u][i] : 0.0f;
+            } else {
+                const long long lo = ok ? (long long)p * P.sxn : 0, hi = lo + 8 * half * P.sxc;
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    const float *row = P.x + (long long)min(ci0 + i, P.cin - 1) * P.sxc;  // uniform
+                    const bool in = ci0 + 8 * half + i < P.cin;
+                    xv[u][i] = row[in ? hi : lo];
+                    xv[u][i] = in && ok ? xv[u][i] : 0.0f;
+                }
+            }
+            if (++tap == P.ksize) tap = 0, cb++;
         }
-        const size_t o = ((size_t)tile * ksteps + s) * 64 + lane;
-        ah = reinterpret_cast<const half8 *>(wh)[o];
-        al = reinterpret_cast<const half8 *>(wl)[o];
     };
+    load(s0);
+    // max |x| over the producer's slots, one per lane
+    const int ex = split_exponent(wave_max(__uint_as_float(xmax)));
+    const float xs = ldexpf(1.0f, ex);
     f32x16 acc;
 #pragma unroll
     for (int r = 0; r < 16; r++) acc[r] = 0.0f;
-    if (s0 < s1) {  // uniform
-        half8 ah, al;
-        float xv[8];
-        load(s0, ah, al, xv);
-        for (int s = s0; s < s1; s++) {
-            half8 nh, nl;
-            float nx[8];
-            load(s + 1 < s1 ? s + 1 : s, nh, nl, nx);
+    for (int s = s0; s < s1; s += U) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
             half8 bh, bl;
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-                const float v = xv[i] * xs;
+                const float v = xv[u][i] * xs;
                 const _Float16 hv = (_Float16)v;
                 bh[i] = hv;
                 bl[i] = (_Float16)(v - (float)hv);
             }
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bh, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh, acc, 0, 0, 0);
-            ah = nh;
-            al = nl;
-#pragma unroll
-            for (int i = 0; i < 8; i++) xv[i] = nx[i];
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[u], bh, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[u], bl, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[u], bh, acc, 0, 0, 0);
         }
+        if (s + U < s1) load(s + U);  // uniform
     }
-    if (wave > 0) {
 #pragma unroll
-        for (int r = 0; r < 16; r++) red[wave - 1][r][lane] = acc[r];
-    }
+    for (int r = 0; r < 16; r++) red[wave][r][lane] = acc[r];
     __syncthreads();
-    if (wave > 0 || n >= len) return;
-#pragma unroll
-    for (int r = 0; r < 16; r++) acc[r] = ((acc[r] + red[0][r][lane]) + red[1][r][lane]) + red[2][r][lane];
+    if (n >= len) return;
     // D layout: lane l, register r -> row (r / 4) * 8 + (l / 32) * 4 + r % 4,
     // column l % 32
     const int sc = -(ex + P.ew);
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
+    for (int r0 = 0; r0 < 16; r0 += NW) {
+        const int r = r0 + wave;
         const int m = 32 * tile + (r >> 2) * 8 + half * 4 + (r & 3);
+        float v = red[0][r][lane];
+#pragma unroll
+        for (int w = 1; w < NW; w++) v += red[w][r][lane];
         if (m >= P.M) continue;
-        float v = ldexpf(acc[r], sc);
+        v = ldexpf(v, sc);
         if (P.bias) v += P.bias[m];
         if (P.act == DEC_ACT_GELU) v = dec_gelu(v);
         float *dst = P.c + (long long)m * P.ldc + (long long)n * P.out_stride + phase;
@@ -1173,8 +1238,9 @@ void launch_dec_gather(hipStream_t st, const DecGatherParams &p, int frames) {
     hipLaunchKernelGGL(k_dec_gather, dim3((unsigned)frames), dim3(256), 0, st, p);
 }
 
-void launch_dec_rmsnorm(hipStream_t st, const float *x, const float *gamma, int rows, int n, float eps, float *out) {
-    hipLaunchKernelGGL(k_dec_rmsnorm, dim3((unsigned)rows), dim3(256), 0, st, x, gamma, n, eps, out);
+void launch_dec_rmsnorm(hipStream_t st, const float *x, const float *gamma, int rows, int n, float eps, float *out,
+                        unsigned *amax) {
+    hipLaunchKernelGGL(k_dec_rmsnorm, dim3((unsigned)rows), dim3(256), 0, st, x, gamma, n, eps, out, amax);
 }
 
 void launch_dec_rope(hipStream_t st, float *q, float *k, int T, int heads, int hd, const float *cs, const float *sn,
@@ -1187,9 +1253,11 @@ void launch_dec_attn(hipStream_t st, const DecAttnParams &p) {
     hipLaunchKernelGGL(k_dec_attn, dim3(blocks_for((size_t)p.T * p.heads, 4)), dim3(256), 0, st, p);
 }
 
-void launch_dec_swiglu(hipStream_t st, const float *g, const float *u, int rows, int width, int ld, float *out) {
-    const size_t n = (size_t)rows * width;
-    hipLaunchKernelGGL(k_dec_swiglu, dim3(blocks_for(n, 256)), dim3(256), 0, st, g, u, rows, width, ld, out);
+void launch_dec_swiglu(hipStream_t st, const float *g, const float *u, int rows, int width, int ld, float *out,
+                       unsigned *amax) {
+    // at most 512 blocks, as launch_dec_absmax
+    const unsigned blocks = std::min<unsigned>(blocks_for((size_t)rows * width, 256), 512u);
+    hipLaunchKernelGGL(k_dec_swiglu, dim3(blocks), dim3(256), 0, st, g, u, rows, width, ld, out, amax);
 }
 
 void launch_dec_dwconv(hipStream_t st, const float *x, const float *w, const float *b, int ch, int len, int ks,
@@ -1199,17 +1267,19 @@ void launch_dec_dwconv(hipStream_t st, const float *x, const float *w, const flo
 }
 
 void launch_dec_lnorm(hipStream_t st, const float *x, const float *g, const float *b, int ch, int len, float eps,
-                      float *out) {
+                      float *out, unsigned *amax) {
     // the tiled kernel while its [ch][TS] tile fits 64 KiB of LDS
     const size_t lds16 = (size_t)ch * 16 * sizeof(float), lds8 = (size_t)ch * 8 * sizeof(float);
     if (lds16 <= 65536)
         hipLaunchKernelGGL(k_dec_lnorm_tile<16>, dim3((unsigned)((len + 15) / 16)), dim3(256), lds16, st, x, g, b, ch,
-                           len, eps, out);
+                           len, eps, out, amax);
     else if (lds8 <= 65536)
         hipLaunchKernelGGL(k_dec_lnorm_tile<8>, dim3((unsigned)((len + 7) / 8)), dim3(256), lds8, st, x, g, b, ch, len,
-                           eps, out);
-    else
+                           eps, out, amax);
+    else {
         hipLaunchKernelGGL(k_dec_lnorm, dim3(blocks_for((size_t)len, 64)), dim3(64), 0, st, x, g, b, ch, len, eps, out);
+        launch_dec_absmax(st, out, (size_t)ch * len, amax);
+    }
 }
 
 void launch_dec_snake(hipStream_t st, const float *x, const float *alpha, const float *beta, int ch, int len,
@@ -1231,6 +1301,20 @@ void launch_dec_conv_repack(hipStream_t st, const float *w, long long sm, long l
     const size_t n = (size_t)mtiles * ksteps * 64;
     hipLaunchKernelGGL(k_dec_conv_repack, dim3(blocks_for(n, 256)), dim3(256), 0, st, w, sm, sci, k0, kd, M, cin,
                        taps, cin16, mtiles, ksteps, ew, wh, wl);
+}
+
+// At least 4 steps (one batch of loads) per wave, and no more waves than the
+// chip holds: 500 frames' 1024 -> 1536 channels of 7 taps (3,024 blocks) take
+// 378 us with 4 waves a block, 507 with 16; 13 frames' 768 -> 768 (312
+// blocks) 70 with 16, 85 with 4.
+template <bool KF>
+static void launch_conv_mfma_ks(hipStream_t st, const DecConvMfmaParams &p, dim3 grid) {
+    if (p.ksteps >= 64 && grid.x <= 512)
+        hipLaunchKernelGGL((k_dec_conv_mfma_ks<KF, 16>), grid, dim3(1024), 0, st, p);
+    else if (p.ksteps >= 32 && grid.x <= 1024)
+        hipLaunchKernelGGL((k_dec_conv_mfma_ks<KF, 8>), grid, dim3(512), 0, st, p);
+    else
+        hipLaunchKernelGGL((k_dec_conv_mfma_ks<KF, 4>), grid, dim3(256), 0, st, p);
 }
 
 template <bool KF>
@@ -1258,11 +1342,11 @@ void launch_dec_conv_mfma(hipStream_t st, const DecConvMfmaParams &p) {
     const size_t nph = (size_t)std::max(1, p.nphase);  // a transposed convolution's phases in one launch
     if (force_split ||
         (!force_tiles && (size_t)blocks_for((size_t)p.len, 128) * (size_t)p.mtiles * nph < kDecFillBlocks)) {
-        const dim3 grid(blocks_for((size_t)p.len, 32), (unsigned)p.mtiles, (unsigned)nph);
+        const dim3 grid(blocks_for(blocks_for((size_t)p.len, 32) * (size_t)p.mtiles * nph, 8) * 8);
         if (kf)
-            hipLaunchKernelGGL(k_dec_conv_mfma_ks<true>, grid, dim3(256), 0, st, p);
+            launch_conv_mfma_ks<true>(st, p, grid);
         else
-            hipLaunchKernelGGL(k_dec_conv_mfma_ks<false>, grid, dim3(256), 0, st, p);
+            launch_conv_mfma_ks<false>(st, p, grid);
         return;
     }
     int mt = p.mtiles % 4 == 0 ? 4 : p.mtiles % 3 == 0 ? 3 : p.mtiles % 2 == 0 ? 2 : 1;
@@ -1291,17 +1375,19 @@ void launch_dec_absmax(hipStream_t st, const float *x, size_t n, unsigned *amax)
     hipLaunchKernelGGL(k_dec_absmax, dim3(blocks), dim3(256), 0, st, x, n, amax);
 }
 
-// 3 or 6 channel tiles (12 waves a block, conv2's operand at most 96 KiB of
-// LDS) and a window of at most 64 positions before the block's.  At 384
-// channels a block would hold 64 positions and read 4.1 MB of weights for
-// them, more than the L2 gives in the time of its MFMAs.
+// 3, 6 or 12 channel tiles (12 waves a block, conv2's operand 96 KiB of LDS)
+// and a window of at most 64 positions before the block's.  C = 384, 80,000
+// positions: 810 -> 565 us a unit, its weights read from the L2 for every 64
+// positions; 768 channels would not fit the LDS.
 bool dec_resunit_fits(int channels, int ksize1, int dilation, int ksize2) {
-    return (channels == 96 || channels == 192) && ksize1 == 7 && dilation >= 1 && dilation <= 10 && ksize2 == 1;
+    return (channels == 96 || channels == 192 || channels == 384) && ksize1 == 7 && dilation >= 1 && dilation <= 10 && ksize2 == 1;
 }
 
 void launch_dec_resunit(hipStream_t st, const DecResUnitParams &p, int channels) {
     if (channels == 96)
         hipLaunchKernelGGL((k_dec_resunit<3, 12>), dim3(blocks_for((size_t)p.len, 256)), dim3(768), 0, st, p);
+    else if (channels == 384)
+        hipLaunchKernelGGL((k_dec_resunit<12, 12>), dim3(blocks_for((size_t)p.len, 64)), dim3(768), 0, st, p);
     else
         hipLaunchKernelGGL((k_dec_resunit<6, 12>), dim3(blocks_for((size_t)p.len, 128)), dim3(768), 0, st, p);
 }

@@ -153,6 +153,7 @@ struct DecAttnParams {
     float *out;
     int T, heads, hd, window;
     float scale;
+    unsigned *amax;  // [kDecMaxSlots]: receives max |out|
 };
 
 struct GemmMfmaParams {
@@ -358,16 +359,18 @@ void launch_repack_mfma(hipStream_t st, const DevQ4 &w, uint32_t *wm, uint16_t *
 void launch_mfma_rows(hipStream_t st, const MfmaRowsParams &p);
 void launch_qkv_rows(hipStream_t st, const QkvRowsParams &p);
 void launch_dec_gather(hipStream_t st, const DecGatherParams &p, int frames);
-void launch_dec_rmsnorm(hipStream_t st, const float *x, const float *gamma, int rows, int n, float eps, float *out);
+void launch_dec_rmsnorm(hipStream_t st, const float *x, const float *gamma, int rows, int n, float eps, float *out,
+                        unsigned *amax);
 void launch_dec_rope(hipStream_t st, float *q, float *k, int T, int heads, int hd, const float *cs, const float *sn,
                      int rows, int ld);  // q, k rows ld apart
 void launch_dec_attn(hipStream_t st, const DecAttnParams &p);
 // out[t][j] = silu(g[t * ld + j]) * u[t * ld + j] for rows t < rows, j < width (out rows width apart)
-void launch_dec_swiglu(hipStream_t st, const float *g, const float *u, int rows, int width, int ld, float *out);
+void launch_dec_swiglu(hipStream_t st, const float *g, const float *u, int rows, int width, int ld, float *out,
+                       unsigned *amax);
 void launch_dec_dwconv(hipStream_t st, const float *x, const float *w, const float *b, int ch, int len, int ks,
                        float *out);
 void launch_dec_lnorm(hipStream_t st, const float *x, const float *g, const float *b, int ch, int len, float eps,
-                      float *out);
+                      float *out, unsigned *amax);
 void launch_dec_snake(hipStream_t st, const float *x, const float *alpha, const float *beta, int ch, int len,
                       float *out, unsigned *amax = nullptr, const float *add = nullptr, float *sum = nullptr);
 void launch_dec_fill_u32(hipStream_t st, unsigned *p, int n, unsigned v);

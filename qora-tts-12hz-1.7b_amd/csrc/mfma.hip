@@ -359,8 +359,8 @@ __global__ __launch_bounds__(64 * NW, 2) void k_gemm_mfma_tile(GemmMfmaParams P,
     const int total = T.mb * T.nb * T.kc, per = (int)(gridDim.x >> 3);
     const int L = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
     if (L >= total) return;
-    const int m_blk = L % T.mb, nc = L / T.mb;
-    const int ch = nc % T.kc, n_blk = nc / T.kc;
+    const int nc = __builtin_amdgcn_readfirstlane(L / T.mb), m_blk = L - nc * T.mb;
+    const int n_blk = __builtin_amdgcn_readfirstlane(nc / T.kc), ch = nc - n_blk * T.kc;
     const int K = P.w.K, N = P.w.N, Ks = K / 16, panels = N / 32;
     const int pw = NW * n_blk + wave, p = min(pw, panels - 1);
     const int sb = ch * T.cs, se = min(Ks, sb + T.cs);

@@ -1,6 +1,6 @@
-"""Residual units of 96 and 192 channels (one launch each) against the oracle
+"""Residual units of 96, 192 and 384 channels (one launch each) against the oracle
 and against the same decoder with every layer a launch of its own: lengths off
-the 128- and 256-position blocks and shorter than a window, the largest
+the 64-, 128- and 256-position blocks and shorter than a window, the largest
 dilation the unit takes and one past it, and SnakeBeta factors up to e^3."""
 import numpy as np
 import pytest
@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 def _decoder(ctx, dilations, big=False):
     cfg = qtts.DecoderConfig(hidden=32, heads=2, head_dim=16, inter=64, window=8, codebook_dim=16, codebook_size=64,
                              vq_dim=32, latent=32, num_rest=3, layers=1, upsample=(1,), vocos_channels=64,
-                             vocos=((64, 192, 6, 3), (192, 96, 4, 2)), dilations=dilations, rope_rows=64)
+                             vocos=((64, 384, 2, 1), (384, 192, 6, 3), (192, 96, 4, 2)), dilations=dilations, rope_rows=64)
     w = qtts.DecoderWeights(17, cfg)
     if big:
         # SnakeBeta at arguments of tens of periods.  Its slope 1 + exp(alpha -
