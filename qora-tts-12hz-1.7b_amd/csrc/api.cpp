@@ -418,12 +418,33 @@ size_t tile_part_floats(const GemmTilePlan &t) {
     return t.kc > 1 ? (size_t)t.mb * t.nb * t.kc * (size_t)(t.nw * t.mt * 1024) : 0;
 }
 
+// 32-row steps per wave and K chunks of the product of up to 16 rows: 8 steps
+// where that leaves no chunks to add or fills the chip (384 blocks), else 4.
+// Call with 8 / 4 / 2 steps, 16 rows: 2048 -> 12288 13.2 / 13.3 / 13.5 us,
+// 6144 -> 2048 11.6 / 13.3 / 17.3, 1024 -> 6144 6.8 / 8.4 / 8.3; 2048 -> 4096
+// 9.1 / 8.7 / 9.7, 2048 -> 1024 8.7 / 8.1 / 8.5.
+constexpr int kMfma16Rows = 16;
+
+void mfma16_plan(int K, int N, int *sw, int *kc) {
+    const int K32 = (K + 31) / 32, panels = N / 32;
+    int s = 8;
+    while (s > 1 && 2 * s >= K32) s /= 2;
+    *kc = (K32 + 4 * s - 1) / (4 * s);
+    if (*kc > 1 && panels * *kc < 384) {
+        s = 4;
+        *kc = (K32 + 15) / 16;
+    }
+    *sw = s;
+}
+
 // Grows the MFMA GEMM scratch for a K x N weight at up to M rows, so that a
 // later call allocates nothing (e.g. under stream capture).
 qtts_status mfma_reserve(qtts_ctx *c, int K, int N, int M) {
     int sw, kc;
     mfma_plan(K, &sw, &kc);
     size_t rows = 64, part = kc > 1 ? (size_t)kc * (M > 32 ? 64 : 32) * N : 0;
+    mfma16_plan(K, N, &sw, &kc);
+    if (kc > 1) part = std::max(part, (size_t)kc * kMfma16Rows * N);
     if (M > kMfmaPassRows) {
         const GemmTilePlan t = tile_plan(M < kTileMaxRows ? M : kTileMaxRows, K, N);
         rows = std::max(rows, (size_t)32 * t.mt * t.mb);
@@ -449,14 +470,16 @@ qtts_status run_gemm_mfma(qtts_ctx *c, const DevQ4Mfma &w, const float *x, int M
     if (panels > kCounters) return fail(c, QTTS_ESHAPE, "MFMA GEMM: more panels than counters");
     for (int r0 = 0; r0 < M; r0 += kTileMaxRows) {
         const int Mc = M - r0 < kTileMaxRows ? M - r0 : kTileMaxRows;
-        const bool tiled = Mc > kMfmaPassRows;
+        const bool tiled = Mc > kMfmaPassRows, m16 = Mc <= kMfma16Rows;
         GemmTilePlan t{};
         int sw = 0, kc = 0;
         if (tiled)
             t = tile_plan(Mc, K, N);
+        else if (m16)
+            mfma16_plan(K, N, &sw, &kc);
         else
             mfma_plan(K, &sw, &kc);
-        const int mt = Mc > 32 ? 2 : 1, Mpad = tiled ? 32 * t.mt * t.mb : 32 * mt;
+        const int mt = Mc > 32 ? 2 : 1, Mpad = tiled ? 32 * t.mt * t.mb : m16 ? kMfma16Rows : 32 * mt;
         QTTS_TRY(mfma_reserve(c, K, N, Mc));
         MfmaRowsParams r{};
         r.x = x + (size_t)r0 * ldx;
@@ -466,9 +489,11 @@ qtts_status run_gemm_mfma(qtts_ctx *c, const DevQ4Mfma &w, const float *x, int M
         r.Mpad = Mpad;
         r.mode = mode;
         r.gamma = gamma;
+        const size_t half = (size_t)Mpad * (m16 ? (K + 31) / 32 * 32 : K);  // 16-row operands: whole 32-row steps
+        r.m16 = m16 ? 1 : 0;
         r.xh = c->mfma_x;
-        r.xl = c->mfma_x + (size_t)Mpad * K;
-        r.rexp = reinterpret_cast<int *>(c->mfma_x + (size_t)2 * Mpad * K);
+        r.xl = c->mfma_x + half;
+        r.rexp = reinterpret_cast<int *>(c->mfma_x + 2 * half);
         r.norm_out = norm_out ? norm_out + (size_t)r0 * ldn : nullptr;
         r.ldn = ldn;
         launch_mfma_rows(c->stream, r);
@@ -488,6 +513,8 @@ qtts_status run_gemm_mfma(qtts_ctx *c, const DevQ4Mfma &w, const float *x, int M
         p.full = full ? 1 : 0;
         if (tiled)
             launch_gemm_mfma_tile(c->stream, p, t);
+        else if (m16)
+            launch_gemm_mfma16(c->stream, p, sw, kc);
         else
             launch_gemm_mfma(c->stream, p, mt, sw, kc);
         QTTS_TRY(check_launch(c, "k_gemm_mfma"));

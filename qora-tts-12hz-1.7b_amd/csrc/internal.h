@@ -49,6 +49,7 @@ struct MfmaRowsParams {
     int ldx, K, M, Mpad, mode;
     const uint16_t *gamma;  // RMSNORM weight (binary16 bits)
     _Float16 *xh, *xl;      // [Mpad / 32][K / 16][64][8], the MFMA A-operand order
+    int m16;                // 1: [ceil(K / 32)][64][8], the 16-row operand order (Mpad 16)
     int *rexp;              // [Mpad] row exponents
     float *norm_out;        // optional: the prologue's rows (f32) at norm_out[m * ldn + k]
     int ldn;
@@ -384,6 +385,8 @@ void launch_dec_resunit(hipStream_t st, const DecResUnitParams &p, int channels)
 // out[i] = exp(sign * x[i]) for i < n
 void launch_dec_exp(hipStream_t st, const float *x, float sign, int n, float *out);
 void launch_gemm_mfma(hipStream_t st, const GemmMfmaParams &p, int mt, int sw, int kc);
+// up to 16 rows, split in the 16-row operand order; part: [kc][16][N] when kc > 1
+void launch_gemm_mfma16(hipStream_t st, const GemmMfmaParams &p, int sw, int kc);
 // q, kcache, vcache, kv_cap, nq, nkv, scale and out of p; head_dim 128; M rows into an empty cache
 void launch_attn_prefill(hipStream_t st, const AttnParams &p, int M);
 // part: [mb * nb * kc][32 * mt * 32 * nw] when kc > 1; counters: mb * nb, zero between launches

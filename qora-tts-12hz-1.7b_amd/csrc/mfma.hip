@@ -79,19 +79,26 @@ __global__ void k_repack_mfma(DevQ4 w, uint32_t *wm, uint16_t *sa, uint16_t *sb,
 // block barrier, and the gammas load with the row), which can miss max|v| by
 // a few ulps: e is then one lower, putting max|v| * 2^e in [2^13, 2^15).
 // rexp[m] = e; rows >= M are zero with e = 0.  xh and xl are stored in the
-// MFMA A-operand order -- [M-tile][16-row step][lane][8] -- so that each
-// wave's operand load of a step is one contiguous KiB.
-template <int G>  // 8-value groups per thread: K <= 2048 * G
-__global__ __launch_bounds__(256) void k_mfma_rows(MfmaRowsParams P) {
-    __shared__ float red[2][4];
+// MFMA A-operand order -- [M-tile][16-row step][lane][8], or
+// [32-row step][lane][8] for k_gemm_mfma16 -- so that each wave's operand
+// load of a step is one contiguous KiB.  One 8-value group per thread (K =
+// 6144: 1024 threads a row).
+template <int NT, bool M16>  // threads (K <= 8 * NT); the 16-row operand order
+__global__ __launch_bounds__(NT) void k_mfma_rows(MfmaRowsParams P) {
+    constexpr int G = 1;  // 8-value groups per thread
+    __shared__ float red[2][NT / 64];
     const int m = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int K = P.K, Ks = K / 16, ng = K / 8;
     // 8-value group g = k / 8 of row m goes to the A-operand slot of lane
-    // (m % 32) + 32 (g % 2) in step g / 2 of M-tile m / 32
-    const size_t tile = (size_t)(m >> 5) * Ks * 64 + (m & 31);
+    // (m % 32) + 32 (g % 2) in step g / 2 of M-tile m / 32, or (16-row
+    // operands) of lane m + 16 (g % 4) in 32-row step g / 4
+    const size_t tile = M16 ? (size_t)m : (size_t)(m >> 5) * Ks * 64 + (m & 31);
+    auto slot = [&](int g) {
+        return (tile + (M16 ? (size_t)(g >> 2) * 64 + 16 * (g & 3) : (size_t)(g >> 1) * 64 + 32 * (g & 1))) * 8;
+    };
     if (m >= P.M) {
-        for (int g = tid; g < ng; g += 256) {
-            const size_t o = (tile + (size_t)(g >> 1) * 64 + 32 * (g & 1)) * 8;
+        for (int g = tid; g < ng; g += NT) {
+            const size_t o = slot(g);
             *reinterpret_cast<half8 *>(P.xh + o) = (half8){};
             *reinterpret_cast<half8 *>(P.xl + o) = (half8){};
         }
@@ -106,7 +113,7 @@ __global__ __launch_bounds__(256) void k_mfma_rows(MfmaRowsParams P) {
     //    and max|x * gamma| (RMSNorm) or max|v|
 #pragma unroll
     for (int j = 0; j < G; j++) {
-        const int g = tid + 256 * j;
+        const int g = tid + NT * j;
         if (g < ng) {
             const float4 a = *reinterpret_cast<const float4 *>(src + 8 * g);
             const float4 b = *reinterpret_cast<const float4 *>(src + 8 * g + 4);
@@ -150,9 +157,13 @@ __global__ __launch_bounds__(256) void k_mfma_rows(MfmaRowsParams P) {
         red[1][wave] = mx;
     }
     __syncthreads();
-    mx = fmaxf(fmaxf(red[1][0], red[1][1]), fmaxf(red[1][2], red[1][3]));
+    mx = red[1][0];
+#pragma unroll
+    for (int w = 1; w < NT / 64; w++) mx = fmaxf(mx, red[1][w]);
     if (norm) {
-        ss = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
+        ss = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NT / 64; w += 4) ss += (red[0][w] + red[0][w + 1]) + (red[0][w + 2] + red[0][w + 3]);
         const float inv = 1.0f / sqrtf(ss / (float)K + 1e-6f);
         mx *= inv;
 #pragma unroll
@@ -171,7 +182,7 @@ __global__ __launch_bounds__(256) void k_mfma_rows(MfmaRowsParams P) {
     if (P.norm_out) {
 #pragma unroll
         for (int j = 0; j < G; j++) {
-            const int g = tid + 256 * j;
+            const int g = tid + NT * j;
             if (g >= ng) continue;
             float *dst = P.norm_out + (size_t)m * P.ldn + 8 * g;
 #pragma unroll
@@ -179,9 +190,13 @@ __global__ __launch_bounds__(256) void k_mfma_rows(MfmaRowsParams P) {
         }
     }
     // 3. the binary16 hi + lo split
+    if (M16 && ng + tid < (ng + 3) / 4 * 4) {  // the last 32-row step's rows past K
+        *reinterpret_cast<half8 *>(P.xh + slot(ng + tid)) = (half8){};
+        *reinterpret_cast<half8 *>(P.xl + slot(ng + tid)) = (half8){};
+    }
 #pragma unroll
     for (int j = 0; j < G; j++) {
-        const int g = tid + 256 * j;
+        const int g = tid + NT * j;
         if (g >= ng) continue;
         half8 h, l;
 #pragma unroll
@@ -190,7 +205,7 @@ __global__ __launch_bounds__(256) void k_mfma_rows(MfmaRowsParams P) {
             h[i] = (_Float16)s;
             l[i] = (_Float16)(s - (float)h[i]);
         }
-        const size_t o = (tile + (size_t)(g >> 1) * 64 + 32 * (g & 1)) * 8;
+        const size_t o = slot(g);
         *reinterpret_cast<half8 *>(P.xh + o) = h;
         *reinterpret_cast<half8 *>(P.xl + o) = l;
     }
@@ -324,6 +339,127 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     }
 #pragma unroll
     for (int u = 0; u < U; u++) {
+        const int i = tid + 256 * u, m = i >> 5, n = 32 * p + (i & 31);
+        if (m >= M) continue;
+        float r = ldexpf(v[u], -P.rexp[m]);
+        if (P.bias) r += P.bias[n];
+        float *dst = P.y + (size_t)m * P.ldy + n;
+        *dst = P.accumulate ? *dst + r : r;
+    }
+}
+
+// The same for up to 16 rows: 16x16x32 MFMAs, so that no operand register or
+// L2 read goes to rows that are not there.  A block of 4 waves owns one panel
+// and 4 * SW 32-row steps; a wave holds twice the K of k_gemm_mfma's in as
+// many registers, which halves the chunks (and their partials) and puts the
+// whole weight in flight in one round of blocks.  Lane l: k rows 8 (l / 16)
+// .. + 7 of a step, A row and B column l % 16; the panel's two 16-column
+// tiles share the A operand and the scales.
+// Row split and product, 16 rows, weights from memory: 2048 -> 12288 17.9 ->
+// 13.2 us, 6144 -> 2048 15.9 -> 11.6, 1024 -> 6144 9.4 -> 6.8, 2048 -> 4096
+// 9.7 -> 8.7.  Bound by launch, load and merge latency (the weights alone
+// take 3 us of the first).
+template <int SW, bool FULL>
+__global__ __launch_bounds__(256) void k_gemm_mfma16(GemmMfmaParams P) {
+    __shared__ float red[4][512];
+    __shared__ int s_last;
+    const int p = blockIdx.x, ch = blockIdx.y, kc = gridDim.y;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: the operand addresses are scalar + lane
+    const int K = P.w.K, N = P.w.N, Ks = K / 16, K32 = (K + 31) / 32;
+    const int s0 = (ch * 4 + wave) * SW;
+    const int kg = lane >> 4, col = lane & 15;
+    // K = 16 (mod 32): the last step's upper half re-reads its lower half, q = 0 (and x = 0)
+    uint32_t wq[SW][2];
+    u32x4v sav[SW], sbv[SW];
+    half8 xh[SW], xl[SW];
+#pragma unroll
+    for (int i = 0; i < SW; i++) {
+        const int s = min(s0 + i, K32 - 1);
+        const int up = 2 * s + (kg >> 1) < Ks ? kg >> 1 : 0;  // 16-row step within the 32
+        const uint32_t *wm = P.w.wm + ((size_t)p * Ks + 2 * s) * 64;
+        wq[i][0] = wm[64 * up + 32 * (kg & 1) + col];
+        wq[i][1] = wm[64 * up + 32 * (kg & 1) + col + 16];
+        const size_t so = (size_t)p * K + 32 * s;
+        sav[i] = reinterpret_cast<const u32x4v *>(P.w.sa + so)[2 * up + (kg & 1)];
+        sbv[i] = reinterpret_cast<const u32x4v *>(P.w.sb + so)[2 * up + (kg & 1)];
+        xh[i] = reinterpret_cast<const half8 *>(P.xh + (size_t)s * 512)[lane];
+        xl[i] = reinterpret_cast<const half8 *>(P.xl + (size_t)s * 512)[lane];
+    }
+    __builtin_amdgcn_sched_barrier(0);  // keep every load ahead of the first wait
+    f32x4 acc[2];
+#pragma unroll
+    for (int t = 0; t < 2; t++) acc[t] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < SW; i++) {
+        const bool in = s0 + i < K32 && 2 * (s0 + i) + (kg >> 1) < Ks;
+        const uint32_t sap[4] = {sav[i].x, sav[i].y, sav[i].z, sav[i].w};
+        const uint32_t sbp[4] = {sbv[i].x, sbv[i].y, sbv[i].z, sbv[i].w};
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const uint32_t w = in ? wq[i][t] : 0x88888888u;
+            half8 ba, bb;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+                const uint32_t bits = ((w >> (4 * j)) & 0x000F000Fu) | 0x64006400u;
+                const half2v q = __builtin_bit_cast(half2v, bits) - (half2v){(_Float16)1032.0f, (_Float16)1032.0f};
+                const half2v a = q * __builtin_bit_cast(half2v, sap[j]);
+                const half2v b = q * __builtin_bit_cast(half2v, sbp[j]);
+                ba[2 * j] = a.x;
+                ba[2 * j + 1] = a.y;
+                bb[2 * j] = b.x;
+                bb[2 * j + 1] = b.y;
+            }
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[i], ba, acc[t], 0, 0, 0);
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh[i], bb, acc[t], 0, 0, 0);
+            acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl[i], ba, acc[t], 0, 0, 0);
+            if constexpr (FULL) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl[i], bb, acc[t], 0, 0, 0);
+        }
+    }
+    // D layout: lane l, register r -> row 4 (l / 16) + r, column l % 16
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) red[wave][(4 * kg + r) * 32 + 16 * t + col] = acc[t][r];
+    __syncthreads();
+    const int M = P.M;
+    float v[2];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int i = tid + 256 * u;
+        v[u] = (red[0][i] + red[1][i]) + (red[2][i] + red[3][i]);
+    }
+    if (kc > 1) {
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int i = tid + 256 * u;
+            if ((i >> 5) < M) st_dev(P.part + ((size_t)ch * 16 + (i >> 5)) * N + 32 * p + (i & 31), v[u]);
+        }
+        wait_stores();
+        __syncthreads();
+        if (tid == 0) s_last = arrive_dev(&P.counters[p]) == (unsigned)(kc - 1);
+        __syncthreads();
+        if (!s_last) return;
+        if (tid == 0) reset_dev(&P.counters[p]);
+        v[0] = v[1] = 0.0f;
+        for (int c0 = 0; c0 < kc; c0 += 8) {
+            float t[8][2];
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+                    t[j][u] = ld_dev(P.part + ((size_t)min(c0 + j, kc - 1) * 16 + min((tid + 256 * u) >> 5, M - 1)) * N +
+                                     32 * p + (tid & 31));
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+                    if (c0 + j < kc) v[u] += t[j][u];
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
         const int i = tid + 256 * u, m = i >> 5, n = 32 * p + (i & 31);
         if (m >= M) continue;
         float r = ldexpf(v[u], -P.rexp[m]);
@@ -743,14 +879,34 @@ void launch_repack_mfma(hipStream_t st, const DevQ4 &w, uint32_t *wm, uint16_t *
     hipLaunchKernelGGL(k_repack_mfma, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, w, wm, sa, sb, too_large);
 }
 
-void launch_mfma_rows(hipStream_t st, const MfmaRowsParams &p) {
-    const int g = (p.K / 8 + 255) / 256;
-    if (g <= 1)
-        hipLaunchKernelGGL(k_mfma_rows<1>, dim3((unsigned)p.Mpad), dim3(256), 0, st, p);
-    else if (g == 2)
-        hipLaunchKernelGGL(k_mfma_rows<2>, dim3((unsigned)p.Mpad), dim3(256), 0, st, p);
+template <bool M16>
+static void launch_mfma_rows_order(hipStream_t st, const MfmaRowsParams &p) {
+    const dim3 grid((unsigned)p.Mpad);
+    if (p.K <= 2048)
+        hipLaunchKernelGGL((k_mfma_rows<256, M16>), grid, dim3(256), 0, st, p);
+    else if (p.K <= 4096)
+        hipLaunchKernelGGL((k_mfma_rows<512, M16>), grid, dim3(512), 0, st, p);
     else
-        hipLaunchKernelGGL(k_mfma_rows<4>, dim3((unsigned)p.Mpad), dim3(256), 0, st, p);
+        hipLaunchKernelGGL((k_mfma_rows<1024, M16>), grid, dim3(1024), 0, st, p);
+}
+
+void launch_mfma_rows(hipStream_t st, const MfmaRowsParams &p) {
+    p.m16 ? launch_mfma_rows_order<true>(st, p) : launch_mfma_rows_order<false>(st, p);
+}
+
+template <bool FULL>
+static void launch_gemm_mfma16_full(hipStream_t st, const GemmMfmaParams &p, int sw, int kc) {
+    const dim3 grid((unsigned)(p.w.N / 32), (unsigned)kc);
+    switch (sw) {
+        case 8: hipLaunchKernelGGL((k_gemm_mfma16<8, FULL>), grid, dim3(256), 0, st, p); break;
+        case 4: hipLaunchKernelGGL((k_gemm_mfma16<4, FULL>), grid, dim3(256), 0, st, p); break;
+        case 2: hipLaunchKernelGGL((k_gemm_mfma16<2, FULL>), grid, dim3(256), 0, st, p); break;
+        default: hipLaunchKernelGGL((k_gemm_mfma16<1, FULL>), grid, dim3(256), 0, st, p); break;
+    }
+}
+
+void launch_gemm_mfma16(hipStream_t st, const GemmMfmaParams &p, int sw, int kc) {
+    p.full ? launch_gemm_mfma16_full<true>(st, p, sw, kc) : launch_gemm_mfma16_full<false>(st, p, sw, kc);
 }
 
 template <int MT, bool FULL>

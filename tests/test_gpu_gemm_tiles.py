@@ -1,4 +1,4 @@
-"""The Q4 product in row blocks (more than 64 rows) against float64, at the
+"""The Q4 product of 8 to 16 rows and in row blocks (more than 64 rows) against float64, at the
 edges of its tiles: one row past a pass, rows off the 32- and 128-row tiles,
 an odd number of 16-row K steps, panel counts off a block's 4 or 8, one and
 several K chunks; and the scale split's last accepted scales."""
@@ -17,7 +17,8 @@ def _bound(x, w, K):
     return (2.0 ** -19 + (3 * K / 16 + 32) * 2.0 ** -24) * (np.abs(x.astype(np.float64)) @ np.abs(w))
 
 
-@pytest.mark.parametrize("rows,K,N", [(65, 1040, 160), (96, 2048, 2048), (97, 16, 32), (128, 48, 288), (129, 6144, 96),
+@pytest.mark.parametrize("rows,K,N", [(8, 16, 32), (9, 48, 96), (15, 272, 1056), (16, 1040, 2048), (13, 2064, 64),
+                                      (16, 6144, 2048), (17, 1040, 96), (65, 1040, 160), (96, 2048, 2048), (97, 16, 32), (128, 48, 288), (129, 6144, 96),
                                       (300, 1024, 1056), (1000, 272, 2048), (1064, 2048, 4096), (4097, 32, 64)])
 def test_gemm_row_blocks(ctx, rows, K, N):
     w = qtts.Q4Weight.synthetic(21, f"tiles.{K}.{N}", K, N)
