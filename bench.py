@@ -328,7 +328,7 @@ def mfma_gemm_roofline(ctx, rows=64, iters=128, copies=32):
         "peak": MFMA_F16_PEAK_TFLOPS,
         "unit": "TFLOP/s",
         "frac": round(achieved / MFMA_F16_PEAK_TFLOPS, 4),
-        "kernel": "k_mfma_rows + k_gemm_mfma<2,8> (Q4 GEMM 64x2048 -> 12288, talker gate|up at prefill)",
+        "kernel": "k_mfma_rows + k_gemm_mfma<2> (Q4 GEMM 64x2048 -> 12288, talker gate|up at prefill)",
         "weight_GBps": round((K * N // 2 + K * (N // 32) * 4) / avg_s / 1e9, 1),
         "avg_call_us": round(avg_s * 1e6, 2),
     }

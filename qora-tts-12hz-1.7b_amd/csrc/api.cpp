@@ -362,13 +362,19 @@ qtts_status grow(qtts_ctx *c, T **buf, size_t *cap, size_t need) {
     return QTTS_OK;
 }
 
-// Steps per wave (sw) and K chunks (kc) of the MFMA GEMM for K rows.
-void mfma_plan(int K, int *sw, int *kc) {
-    const int Ks = K / 16;
-    int s = 8;
-    while (s > 1 && 4 * (s / 2) >= Ks) s /= 2;
-    *sw = s;
-    *kc = (Ks + 4 * s - 1) / (4 * s);
+// Steps per wave and K chunks of the product of 17 to 64 rows: 16 steps where
+// that still makes 192 blocks or leaves one chunk, else 8; 4 where 8 would
+// make fewer than 192 blocks.  64 rows, 16 / 8 steps: 6144 -> 2048 18.3 / 20.0
+// us, 2048 -> 4096 13.1 / 12.8; 8 / 4: 2048 -> 2048 12.3 / 11.6, 2048 -> 1024
+// 12.1 / 10.8, 32 rows 9.8 / 9.8 and 9.6 / 9.0.
+void mfma_plan(int K, int N, int *steps, int *kc) {
+    const int Ks = K / 16, panels = N / 32;
+    auto chunks = [&](int s) { return (Ks + kMfmaWaves * s - 1) / (kMfmaWaves * s); };
+    int s = panels * chunks(16) >= 192 ? 16 : 8;
+    if (chunks(s) > 1 && panels * chunks(s) < 192) s = 4;
+    while (s > 1 && kMfmaWaves * (s / 2) >= Ks) s /= 2;
+    *steps = s;
+    *kc = chunks(s);
 }
 
 // Rows past kMfmaPassRows run in row blocks (k_gemm_mfma_tile), at most
@@ -441,7 +447,7 @@ void mfma16_plan(int K, int N, int *sw, int *kc) {
 // later call allocates nothing (e.g. under stream capture).
 qtts_status mfma_reserve(qtts_ctx *c, int K, int N, int M) {
     int sw, kc;
-    mfma_plan(K, &sw, &kc);
+    mfma_plan(K, N, &sw, &kc);
     size_t rows = 64, part = kc > 1 ? (size_t)kc * (M > 32 ? 64 : 32) * N : 0;
     mfma16_plan(K, N, &sw, &kc);
     if (kc > 1) part = std::max(part, (size_t)kc * kMfma16Rows * N);
@@ -457,9 +463,7 @@ qtts_status mfma_reserve(qtts_ctx *c, int K, int N, int M) {
 // y[m] (+)= f(x[m]) . W (+ bias) for M rows on the matrix cores
 // (csrc/mfma.hip), f the row prologue (MfmaRowsMode): the prologue and
 // binary16 split, then the product.  Up to kMfmaPassRows rows: one block per
-// (panel, K chunk) of 4 * sw 16-row steps, and the last block of a panel sums
-// its chunks; sw is 8 (each wave keeps 8 steps of operand loads in flight;
-// measured fastest at every talker shape, 64 rows) unless K is short.  More
+// (panel, K chunk), and the last block of a panel sums its chunks.  More
 // rows: row blocks by tile_plan.
 qtts_status run_gemm_mfma(qtts_ctx *c, const DevQ4Mfma &w, const float *x, int M, int ldx, int mode,
                           const uint16_t *gamma, float *y, int ldy, const float *bias, bool accumulate,
@@ -478,7 +482,7 @@ qtts_status run_gemm_mfma(qtts_ctx *c, const DevQ4Mfma &w, const float *x, int M
         else if (m16)
             mfma16_plan(K, N, &sw, &kc);
         else
-            mfma_plan(K, &sw, &kc);
+            mfma_plan(K, N, &sw, &kc);
         const int mt = Mc > 32 ? 2 : 1, Mpad = tiled ? 32 * t.mt * t.mb : m16 ? kMfma16Rows : 32 * mt;
         QTTS_TRY(mfma_reserve(c, K, N, Mc));
         MfmaRowsParams r{};

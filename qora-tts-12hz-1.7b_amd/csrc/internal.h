@@ -184,6 +184,7 @@ struct GemmTilePlan {
 constexpr int kGemvThreads = 256;
 constexpr int kGemvWideThreads = 1024;  // the one-row GEMV's block for 2048 < K <= 8192
 constexpr int kMaxM = 4;          // rows per GEMV launch (prefill chunks)
+constexpr int kMfmaWaves = 8;     // waves of a k_gemm_mfma block
 constexpr int kMfmaMinRows = 8;   // GEMMs of at least this many rows run on the matrix cores
 constexpr int kMaxGroups = 15;    // predictor code groups
 constexpr int kAttnThreads = 256;
@@ -384,7 +385,8 @@ bool dec_resunit_fits(int channels, int ksize1, int dilation, int ksize2);
 void launch_dec_resunit(hipStream_t st, const DecResUnitParams &p, int channels);
 // out[i] = exp(sign * x[i]) for i < n
 void launch_dec_exp(hipStream_t st, const float *x, float sign, int n, float *out);
-void launch_gemm_mfma(hipStream_t st, const GemmMfmaParams &p, int mt, int sw, int kc);
+// kc chunks of kMfmaWaves * steps 16-row steps
+void launch_gemm_mfma(hipStream_t st, const GemmMfmaParams &p, int mt, int steps, int kc);
 // up to 16 rows, split in the 16-row operand order; part: [kc][16][N] when kc > 1
 void launch_gemm_mfma16(hipStream_t st, const GemmMfmaParams &p, int sw, int kc);
 // q, kcache, vcache, kv_cap, nq, nkv, scale and out of p; head_dim 128; M rows into an empty cache

@@ -211,139 +211,147 @@ __global__ __launch_bounds__(NT) void k_mfma_rows(MfmaRowsParams P) {
     }
 }
 
-// One 32-column panel x one K chunk of 4 * SW 16-row steps per block; wave w
-// takes steps [w * SW, (w + 1) * SW) of the chunk and issues all of their
-// operand loads before its first MFMA (a step past K re-reads the last step
-// and contributes zero: its scales are masked).  MT M-tiles of 32 rows share
-// each step's B operand.  The waves are summed through LDS; with several
-// chunks, each block stores its tile to `part` and the last block of a panel
-// to arrive (a counter per panel) adds the chunks in chunk order --
-// deterministic -- and finishes: * 2^-rexp[m], + bias, store or accumulate.
-template <int MT, int SW, bool FULL>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_gemm_mfma(GemmMfmaParams P) {
-    __shared__ float red[4][MT * 1024];
+// One 32-column panel x one K chunk per block: 8 waves of `steps` 16-row
+// steps, MT M-tiles of 32 rows sharing each step's B operand.  A wave's
+// operands are loaded R steps ahead into a ring whose registers are loaded
+// again as soon as their MFMAs are issued (a step past the end re-reads the
+// last one and contributes zero: its nibbles are masked to q = 0); four waves
+// a SIMD hide the rest.  The waves are summed through LDS in a fixed tree;
+// with several chunks, each block stores its tile to `part` and the last
+// block of a panel to arrive (a counter per panel) adds the chunks in chunk
+// order -- deterministic -- and finishes: * 2^-rexp[m], + bias, store or
+// accumulate.
+// Row split and product, 64 rows, against blocks of 4 waves with all of a
+// wave's 8 steps loaded at once (two waves a SIMD): 2048 -> 12288 27.4 ->
+// 26.0 us, 6144 -> 2048 20.9 -> 18.3, 1024 -> 6144 12.8 -> 9.6 (no chunks to
+// add).  Bound at 64 rows by the rows' operands from the L2, 512 KiB for
+// every panel; two or four panels to a block measured slower (28.6-34.9).
+template <int MT, bool FULL>
+__global__ __launch_bounds__(64 * kMfmaWaves) void k_gemm_mfma(GemmMfmaParams P, int steps) {
+    constexpr int NW = kMfmaWaves;
+    __shared__ float red[NW][MT * 1024];
     __shared__ int s_last;
     const int p = blockIdx.x, ch = blockIdx.y, kc = gridDim.y;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: the operand addresses are scalar + lane
     const int K = P.w.K, N = P.w.N, Ks = K / 16, Mpad = 32 * MT;
-    const int s0 = (ch * 4 + wave) * SW;
+    const int s0 = (ch * NW + wave) * steps, s1 = min(Ks, s0 + steps);
     const int half = lane >> 5, col = lane & 31;
-
-    // 1. every operand of this wave's steps
-    uint32_t wq[SW];
-    u32x4v sav[SW], sbv[SW];
-    half8 xh[SW][MT], xl[SW][MT];
-#pragma unroll
-    for (int i = 0; i < SW; i++) {
-        const int s = min(s0 + i, Ks - 1);
-        const int krow = 16 * s + 8 * half;
-        wq[i] = P.w.wm[((size_t)p * Ks + s) * 64 + lane];
-        sav[i] = *reinterpret_cast<const u32x4v *>(P.w.sa + (size_t)p * K + krow);
-        sbv[i] = *reinterpret_cast<const u32x4v *>(P.w.sb + (size_t)p * K + krow);
+    constexpr int R = MT == 1 ? 4 : 2;  // ring
+    uint32_t wq[R];
+    u32x4v sav[R], sbv[R];
+    half8 xh[R][MT], xl[R][MT];
+    auto load = [&](int i, int sw) {
+        const int s = min(sw, Ks - 1);
+        wq[i] = (P.w.wm + ((size_t)p * Ks + s) * 64)[lane];
+        sav[i] = reinterpret_cast<const u32x4v *>(P.w.sa + (size_t)p * K + 16 * s)[half];
+        sbv[i] = reinterpret_cast<const u32x4v *>(P.w.sb + (size_t)p * K + 16 * s)[half];
 #pragma unroll
         for (int t = 0; t < MT; t++) {
-            const size_t off = (((size_t)t * Ks + s) * 64 + lane) * 8;
-            xh[i][t] = *reinterpret_cast<const half8 *>(P.xh + off);
-            xl[i][t] = *reinterpret_cast<const half8 *>(P.xl + off);
+            const size_t off = ((size_t)t * Ks + s) * 64 * 8;
+            xh[i][t] = reinterpret_cast<const half8 *>(P.xh + off)[lane];
+            xl[i][t] = reinterpret_cast<const half8 *>(P.xl + off)[lane];
         }
-    }
-    __builtin_amdgcn_sched_barrier(0);  // keep every load ahead of the first wait
+    };
+#pragma unroll
+    for (int i = 0; i < R; i++) load(i, s0 + i);
+    __builtin_amdgcn_sched_barrier(0);
     f32x16 acc[MT];
 #pragma unroll
     for (int t = 0; t < MT; t++)
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[t][r] = 0.0f;
-    // 2. B = (sa + sb) * q as two exact binary16 operands; three MFMAs per tile
+    for (int s = s0; s < s1; s += R) {
 #pragma unroll
-    for (int i = 0; i < SW; i++) {
-        const bool in = s0 + i < Ks;
-        half8 ba, bb;
-        const uint32_t sap[4] = {sav[i].x, sav[i].y, sav[i].z, sav[i].w};
-        const uint32_t sbp[4] = {sbv[i].x, sbv[i].y, sbv[i].z, sbv[i].w};
+        for (int i = 0; i < R; i++) {
+            const uint32_t w = s + i < s1 ? wq[i] : 0x88888888u;  // past the end: nibbles of 8, q = 0
+            half8 ba, bb;
+            const uint32_t sap[4] = {sav[i].x, sav[i].y, sav[i].z, sav[i].w};
+            const uint32_t sbp[4] = {sbv[i].x, sbv[i].y, sbv[i].z, sbv[i].w};
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            // rows 2j, 2j+1 as binary16 1024 + nib (magic exponent), minus 1032
-            typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-            const uint32_t bits = ((wq[i] >> (4 * j)) & 0x000F000Fu) | 0x64006400u;
-            const half2v q = __builtin_bit_cast(half2v, bits) - (half2v){(_Float16)1032.0f, (_Float16)1032.0f};
-            const half2v a = q * __builtin_bit_cast(half2v, in ? sap[j] : 0u);
-            const half2v b = q * __builtin_bit_cast(half2v, in ? sbp[j] : 0u);
-            ba[2 * j] = a.x;
-            ba[2 * j + 1] = a.y;
-            bb[2 * j] = b.x;
-            bb[2 * j + 1] = b.y;
-        }
+            for (int j = 0; j < 4; j++) {
+                typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+                const uint32_t bits = ((w >> (4 * j)) & 0x000F000Fu) | 0x64006400u;
+                const half2v q = __builtin_bit_cast(half2v, bits) - (half2v){(_Float16)1032.0f, (_Float16)1032.0f};
+                const half2v a = q * __builtin_bit_cast(half2v, sap[j]);
+                const half2v b = q * __builtin_bit_cast(half2v, sbp[j]);
+                ba[2 * j] = a.x;
+                ba[2 * j + 1] = a.y;
+                bb[2 * j] = b.x;
+                bb[2 * j + 1] = b.y;
+            }
 #pragma unroll
-        for (int t = 0; t < MT; t++) {
-            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh[i][t], ba, acc[t], 0, 0, 0);
-            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh[i][t], bb, acc[t], 0, 0, 0);
-            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl[i][t], ba, acc[t], 0, 0, 0);
-            if constexpr (FULL) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl[i][t], bb, acc[t], 0, 0, 0);
+            for (int t = 0; t < MT; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh[i][t], ba, acc[t], 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < MT; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xh[i][t], bb, acc[t], 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < MT; t++) acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl[i][t], ba, acc[t], 0, 0, 0);
+            if constexpr (FULL) {
+#pragma unroll
+                for (int t = 0; t < MT; t++)
+                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xl[i][t], bb, acc[t], 0, 0, 0);
+            }
+            load(i, s + R + i);
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
-    // 3. the 4 waves through LDS.  D layout: lane l, register r -> row
-    //    (r/4)*8 + (l/32)*4 + r%4, column l%32
+    // the waves through LDS.  D layout: lane l, register r -> row
+    // (r/4)*8 + (l/32)*4 + r%4, column l%32
 #pragma unroll
     for (int t = 0; t < MT; t++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) red[wave][t * 1024 + ((r >> 2) * 8 + half * 4 + (r & 3)) * 32 + col] = acc[t][r];
+        for (int r = 0; r < 16; r++)
+            red[wave][t * 1024 + ((r >> 2) * 8 + half * 4 + (r & 3)) * 32 + col] = acc[t][r];
     __syncthreads();
-    const int M = P.M;
+    constexpr int U = MT * 16 / NW;  // outputs i = tid + 64 NW u: row i / 32, column i % 32
+    const int M = P.M, n = 32 * p + (tid & 31);
+    float v[U];
+    int mrow[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        const int i = tid + 64 * NW * u;
+        mrow[u] = i >> 5;
+        float t[NW];
+#pragma unroll
+        for (int w = 0; w < NW; w++) t[w] = red[w][i];
+#pragma unroll
+        for (int j = 1; j < NW; j *= 2)
+#pragma unroll
+            for (int w = 0; w < NW; w += 2 * j) t[w] += t[w + j];
+        v[u] = t[0];
+    }
     if (kc > 1) {
-        float *mine = P.part + (size_t)ch * Mpad * N;
-        for (int i = tid; i < M * 32; i += 256) {
-            const int m = i >> 5, n = 32 * p + (i & 31);
-            st_dev(&mine[(size_t)m * N + n], (red[0][i] + red[1][i]) + (red[2][i] + red[3][i]));
-        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (mrow[u] < M) st_dev(P.part + ((size_t)ch * Mpad + mrow[u]) * N + n, v[u]);
         wait_stores();
         __syncthreads();
         if (tid == 0) s_last = arrive_dev(&P.counters[p]) == (unsigned)(kc - 1);
         __syncthreads();
         if (!s_last) return;
         if (tid == 0) reset_dev(&P.counters[p]);
-    }
-    // the block's outputs i = tid + 256 u; with several chunks, the partials
-    // of 4 chunks for all of a thread's outputs are loaded before any is
-    // added (in chunk order)
-    constexpr int U = MT * 4;
-    float v[U];
-    if (kc > 1) {
 #pragma unroll
         for (int u = 0; u < U; u++) v[u] = 0.0f;
-        uint32_t off[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int i = tid + 256 * u;
-            off[u] = (uint32_t)min(i >> 5, M - 1) * (uint32_t)N + (uint32_t)(32 * p + (i & 31));
-        }
         for (int c0 = 0; c0 < kc; c0 += 4) {
             float t[4][U];
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const float *pc = P.part + (size_t)min(c0 + j, kc - 1) * Mpad * N;  // uniform
+            for (int j = 0; j < 4; j++)
 #pragma unroll
-                for (int u = 0; u < U; u++) t[j][u] = ld_dev(pc + off[u]);
-            }
+                for (int u = 0; u < U; u++)
+                    t[j][u] = ld_dev(P.part + ((size_t)min(c0 + j, kc - 1) * Mpad + min(mrow[u], M - 1)) * N + n);
 #pragma unroll
             for (int j = 0; j < 4; j++)
 #pragma unroll
                 for (int u = 0; u < U; u++)
                     if (c0 + j < kc) v[u] += t[j][u];
         }
-    } else {
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int i = tid + 256 * u;
-            v[u] = (red[0][i] + red[1][i]) + (red[2][i] + red[3][i]);
-        }
     }
 #pragma unroll
     for (int u = 0; u < U; u++) {
-        const int i = tid + 256 * u, m = i >> 5, n = 32 * p + (i & 31);
-        if (m >= M) continue;
-        float r = ldexpf(v[u], -P.rexp[m]);
+        if (mrow[u] >= M) continue;
+        float r = ldexpf(v[u], -P.rexp[mrow[u]]);
         if (P.bias) r += P.bias[n];
-        float *dst = P.y + (size_t)m * P.ldy + n;
+        float *dst = P.y + (size_t)mrow[u] * P.ldy + n;
         *dst = P.accumulate ? *dst + r : r;
     }
 }
@@ -909,22 +917,19 @@ void launch_gemm_mfma16(hipStream_t st, const GemmMfmaParams &p, int sw, int kc)
     p.full ? launch_gemm_mfma16_full<true>(st, p, sw, kc) : launch_gemm_mfma16_full<false>(st, p, sw, kc);
 }
 
-template <int MT, bool FULL>
-static void launch_gemm_mfma_mt(hipStream_t st, const GemmMfmaParams &p, int sw, int kc) {
-    const dim3 grid((unsigned)(p.w.N / 32), (unsigned)kc);
-    switch (sw) {
-        case 8: hipLaunchKernelGGL((k_gemm_mfma<MT, 8, FULL>), grid, dim3(256), 0, st, p); break;
-        case 4: hipLaunchKernelGGL((k_gemm_mfma<MT, 4, FULL>), grid, dim3(256), 0, st, p); break;
-        case 2: hipLaunchKernelGGL((k_gemm_mfma<MT, 2, FULL>), grid, dim3(256), 0, st, p); break;
-        default: hipLaunchKernelGGL((k_gemm_mfma<MT, 1, FULL>), grid, dim3(256), 0, st, p); break;
+void launch_gemm_mfma(hipStream_t st, const GemmMfmaParams &p, int mt, int steps, int kc) {
+    const dim3 grid((unsigned)(p.w.N / 32), (unsigned)kc), block(64 * kMfmaWaves);
+    if (mt == 1) {
+        if (p.full)
+            hipLaunchKernelGGL((k_gemm_mfma<1, true>), grid, block, 0, st, p, steps);
+        else
+            hipLaunchKernelGGL((k_gemm_mfma<1, false>), grid, block, 0, st, p, steps);
+    } else {
+        if (p.full)
+            hipLaunchKernelGGL((k_gemm_mfma<2, true>), grid, block, 0, st, p, steps);
+        else
+            hipLaunchKernelGGL((k_gemm_mfma<2, false>), grid, block, 0, st, p, steps);
     }
-}
-
-void launch_gemm_mfma(hipStream_t st, const GemmMfmaParams &p, int mt, int sw, int kc) {
-    if (p.full)
-        mt == 1 ? launch_gemm_mfma_mt<1, true>(st, p, sw, kc) : launch_gemm_mfma_mt<2, true>(st, p, sw, kc);
-    else
-        mt == 1 ? launch_gemm_mfma_mt<1, false>(st, p, sw, kc) : launch_gemm_mfma_mt<2, false>(st, p, sw, kc);
 }
 
 template <bool FULL>
