@@ -363,8 +363,8 @@ qtts_status grow(qtts_ctx *c, T **buf, size_t *cap, size_t need) {
 }
 
 // Steps per wave and K chunks of the product of 17 to 64 rows: 16 steps where
-// that still makes 192 blocks or leaves one chunk, else 8; 4 where 8 would
-// make fewer than 192 blocks.  64 rows, 16 / 8 steps: 6144 -> 2048 18.3 / 20.0
+// that still makes 192 blocks, else 8; 4 where 8 would make chunks and fewer
+// than 192 blocks.  64 rows, 16 / 8 steps: 6144 -> 2048 18.3 / 20.0
 // us, 2048 -> 4096 13.1 / 12.8; 8 / 4: 2048 -> 2048 12.3 / 11.6, 2048 -> 1024
 // 12.1 / 10.8, 32 rows 9.8 / 9.8 and 9.6 / 9.0.
 void mfma_plan(int K, int N, int *steps, int *kc) {
@@ -2022,8 +2022,11 @@ static qtts_status prefill_layers_mfma(qtts_talker *t, qtts_kv *kv, int seq_len)
         q.kcache = kc;
         q.vcache = vc;
         q.kv_cap = kv->cap;
-        launch_qkv_rows(c->stream, q);
-        QTTS_TRY(check_launch(c, "k_qkv_rows"));
+        const bool shortp = seq_len <= kAttnShortRows;
+        if (!shortp) {
+            launch_qkv_rows(c->stream, q);
+            QTTS_TRY(check_launch(c, "k_qkv_rows"));
+        }
         AttnParams a{};
         a.q = t->qp;
         a.ldq = qd;
@@ -2036,7 +2039,9 @@ static qtts_status prefill_layers_mfma(qtts_talker *t, qtts_kv *kv, int seq_len)
         a.scale = 1.0f / sqrtf((float)st.hd);  // src/talker.rs:305
         a.out = t->ap;
         a.ldo = qd;
-        if (seq_len > kAttnPrefillRows || seq_len * st.nkv > kAttnCounters) {
+        if (shortp) {
+            launch_attn_short(c->stream, q, a);
+        } else if (seq_len > kAttnPrefillRows || seq_len * st.nkv > kAttnCounters) {
             launch_attn_prefill(c->stream, a, seq_len);
         } else {
             a.nsplit = 1;

@@ -389,6 +389,10 @@ void launch_dec_exp(hipStream_t st, const float *x, float sign, int n, float *ou
 void launch_gemm_mfma(hipStream_t st, const GemmMfmaParams &p, int mt, int steps, int kc);
 // up to 16 rows, split in the 16-row operand order; part: [kc][16][N] when kc > 1
 void launch_gemm_mfma16(hipStream_t st, const GemmMfmaParams &p, int sw, int kc);
+// k_qkv_rows and attention in one for q.M <= kAttnShortRows rows into an empty
+// cache (scale, out and ldo of a; q.q is not written)
+constexpr int kAttnShortRows = 16;
+void launch_attn_short(hipStream_t st, const QkvRowsParams &q, const AttnParams &a);
 // q, kcache, vcache, kv_cap, nq, nkv, scale and out of p; head_dim 128; M rows into an empty cache
 void launch_attn_prefill(hipStream_t st, const AttnParams &p, int M);
 // part: [mb * nb * kc][32 * mt * 32 * nw] when kc > 1; counters: mb * nb, zero between launches

@@ -1,7 +1,8 @@
-"""The prefill's attention past 64 rows (32-row tiles, four waves over the
-keys) against the oracle: one row past the limit, whole and ragged tiles, one
-to four query heads per kv head; and a row of NaNs, which the rows before it
-must not see."""
+"""The prefill's attention up to 16 rows (one launch with QK-norm, RoPE and
+the append) and past 64 (32-row tiles, four waves over the keys) against the
+oracle: the limits and one past them, whole and ragged tiles, one to four
+query heads per kv head; and a row of NaNs, which the rows before it must not
+see."""
 import numpy as np
 import pytest
 
@@ -20,7 +21,7 @@ def _talker(ctx, heads, kv_heads, seed=31):
 
 
 @pytest.mark.parametrize("heads,kv_heads", [(4, 4), (4, 2), (4, 1), (18, 18)])
-@pytest.mark.parametrize("rows", [64, 65, 96, 129, 257])
+@pytest.mark.parametrize("rows", [8, 9, 16, 17, 64, 65, 96, 129, 257])
 def test_prefill_attention(ctx, rows, heads, kv_heads):
     cfg, tw, t = _talker(ctx, heads, kv_heads)
     ot = oracle.Talker(tw)
@@ -32,7 +33,7 @@ def test_prefill_attention(ctx, rows, heads, kv_heads):
         assert within(got, ref)
 
 
-@pytest.mark.parametrize("rows,bad", [(96, 95), (100, 70), (129, 128), (200, 3)])
+@pytest.mark.parametrize("rows,bad", [(16, 9), (96, 95), (100, 70), (129, 128), (200, 3)])
 def test_prefill_rows_before_a_nan_row_are_unchanged(ctx, rows, bad):
     cfg, tw, t = _talker(ctx, 4, 2)
     x = qtts.synth_normal_f32(32, f"nan.x.{rows}", rows * cfg.hidden).reshape(rows, -1).copy()
