@@ -3156,12 +3156,12 @@ struct qtts_decoder {
     Owner own;
     std::vector<std::vector<DecResUnit>> res_unit;  // [block][unit]
     // the Vocos convolutions on the matrix cores: [block][unit][conv1, conv2]
-    // and [block][output phase] of each block's transposed convolution
+    // and [block] of each block's transposed convolution
     std::vector<std::vector<std::array<DecConvMfma, 2>>> res_mfma;
-    std::vector<std::vector<DecConvMfma>> up_mfma;
+    std::vector<DecConvMfma> up_mfma;
     // the other matrix-core layers: codebook projections, pre-conv, the
     // transformer's input / output and per-layer q, k, v, o, gate, up, down,
-    // each ConvNeXt stage's transposed convolution (per phase) and pw1, pw2,
+    // each ConvNeXt stage's transposed convolution and pw1, pw2,
     // the Vocos input and output convolutions
     DecConvMfma proj0, proj_rest, pre_conv, tf_in, tf_out, vocos_init, out_conv;
     std::vector<std::array<DecConvMfma, 7>> layer_mfma;
@@ -3169,7 +3169,7 @@ struct qtts_decoder {
     // an input in one launch; when every part is a whole number of tiles)
     std::vector<std::array<DecConvMfma, 2>> layer_cat;
     bool cat = false;
-    std::vector<std::vector<DecConvMfma>> cnx_up_mfma;
+    std::vector<DecConvMfma> cnx_up_mfma;
     std::vector<std::array<DecConvMfma, 2>> pw_mfma;
     unsigned *amax = nullptr;  // [amax_slots][kDecMaxSlots]: max |x| of each such convolution's input, cleared per decode
     int amax_slots = 0;
@@ -3231,10 +3231,10 @@ int dec_weight_exponent(const float *w, size_t n) {
 }
 
 // A matrix-core operand copy (k_dec_conv_repack) of the device weights dw:
-// element (m, ci, tap) at dw[m * sm + ci * sci + k0 + tap * kd], scaled by
-// 2^ew and split into binary16 hi + lo.
+// element (m, ci, tap) at dw[m / up * sm + m % up + ci * sci + k0 + tap * kd],
+// scaled by 2^ew and split into binary16 hi + lo.
 qtts_status dec_mfma_copy(qtts_ctx *c, Owner &own, const float *dw, long long sm, long long sci, int k0, int kd,
-                          int M, int cin, int taps, int ew, DecConvMfma *out) {
+                          int M, int cin, int taps, int ew, DecConvMfma *out, int up = 1) {
     DecConvMfma m;
     m.ew = ew;
     m.cin16 = (cin + 15) / 16 * 16;
@@ -3243,7 +3243,8 @@ qtts_status dec_mfma_copy(qtts_ctx *c, Owner &own, const float *dw, long long sm
     const size_t n = (size_t)m.mtiles * m.ksteps * 64 * 8;
     QTTS_TRY(own.alloc(c, &m.wh, n));
     QTTS_TRY(own.alloc(c, &m.wl, n));
-    launch_dec_conv_repack(c->stream, dw, sm, sci, k0, kd, M, cin, taps, m.cin16, m.mtiles, m.ksteps, ew, m.wh, m.wl);
+    launch_dec_conv_repack(c->stream, dw, sm, sci, k0, kd, M, cin, taps, m.cin16, m.mtiles, m.ksteps, ew, up, m.wh,
+                           m.wl);
     QTTS_TRY(check_launch(c, "k_dec_conv_repack"));
     *out = m;
     return QTTS_OK;
@@ -3258,17 +3259,14 @@ qtts_status dec_conv_mfma(qtts_ctx *c, Owner &own, const qtts_conv_view &h, cons
     return dec_mfma_copy(c, own, dv.weight, (long long)ci * k, k, 0, 1, co, ci, k, ew, out);
 }
 
-// A transposed convolution's copy, one per output phase r: tap t of phase r
-// is kernel index r + (J - 1 - t) * stride (J = kernel / stride taps).
+// A transposed convolution's copy, row m = channel * stride + output phase:
+// tap t of phase r is kernel index r + (J - 1 - t) * stride (J = kernel /
+// stride taps).
 qtts_status dec_convt_mfma(qtts_ctx *c, Owner &own, const qtts_conv_view &h, const qtts_conv_view &dv,
-                           std::vector<DecConvMfma> *out) {
+                           DecConvMfma *out) {
     const int ci = h.in_channels, co = h.out_channels, k = h.kernel_size, s = h.stride, J = k / s;
     const int ew = dec_weight_exponent(h.weight, (size_t)ci * co * k);
-    out->assign((size_t)s, DecConvMfma{});
-    for (int r = 0; r < s; r++)
-        QTTS_TRY(dec_mfma_copy(c, own, dv.weight, k, (long long)co * k, r + (J - 1) * s, -s, co, ci, J, ew,
-                               &(*out)[(size_t)r]));
-    return QTTS_OK;
+    return dec_mfma_copy(c, own, dv.weight, k, (long long)co * k, (J - 1) * s, -s, co * s, ci, J, ew, out, s);
 }
 
 // A linear layer's copy: W [K][N] (in-major, as dec_linear reads it), output
@@ -3299,8 +3297,8 @@ qtts_status dec_lin_mfma_cat(qtts_ctx *c, Owner &own, const float *const *hw, co
     QTTS_TRY(own.alloc(c, &m.wh, per * parts));
     QTTS_TRY(own.alloc(c, &m.wl, per * parts));
     for (int q = 0; q < parts; q++) {
-        launch_dec_conv_repack(c->stream, dw[q], 1, N, 0, 0, N, K, 1, m.cin16, tiles, m.ksteps, ew, m.wh + per * q,
-                               m.wl + per * q);
+        launch_dec_conv_repack(c->stream, dw[q], 1, N, 0, 0, N, K, 1, m.cin16, tiles, m.ksteps, ew, 1,
+                               m.wh + per * q, m.wl + per * q);
         QTTS_TRY(check_launch(c, "k_dec_conv_repack"));
     }
     *out = m;
@@ -3368,7 +3366,7 @@ qtts_status dec_causal_mfma(qtts_decoder *d, const qtts_conv_view &v, const DecC
     p.c = c;
     p.ldc = len;
     p.out_stride = 1;
-    p.phase = 0;
+    p.up = 1;
     p.resid = resid;
     launch_dec_conv_mfma(d->ctx->stream, p);
     return check_launch(d->ctx, "k_dec_conv_mfma");
@@ -3406,7 +3404,7 @@ qtts_status dec_linear_mfma(qtts_decoder *d, const DecConvMfma &m, const float *
     p.c = c;
     p.ldc = scn;
     p.out_stride = scm;
-    p.phase = 0;
+    p.up = 1;
     p.resid = resid;
     launch_dec_conv_mfma(d->ctx->stream, p);
     return check_launch(d->ctx, "k_dec_conv_mfma");
@@ -3415,48 +3413,38 @@ qtts_status dec_linear_mfma(qtts_decoder *d, const DecConvMfma &m, const float *
 // conv_transpose1d + the causal right crop (src/conv.rs:198-268,
 // src/decoder.rs:430-444) on the matrix cores: output phase r
 // (out[q * stride + r], q < len) is a causal convolution of x with
-// J = kernel / stride taps reaching J - 1 steps back, from the phase's
-// operand copy.
-qtts_status dec_transposed_mfma(qtts_decoder *d, const qtts_conv_view &v, const std::vector<DecConvMfma> &ph,
-                                const float *x, const unsigned *xmax, int len, float *c) {
-    const int J = v.kernel_size / v.stride;
-    // up to kDecMaxPhases output phases in one launch (grid z = phase): the
-    // phases share their input, shapes and weight exponent
-    const bool one = v.stride > 1 && v.stride <= kDecMaxPhases;
-    for (int r = 0; r < v.stride; r++) {
-        const DecConvMfma &m = ph[(size_t)r];
-        DecConvMfmaParams p{};
-        if (one) {
-            p.nphase = v.stride;
-            for (int q = 0; q < v.stride; q++) {
-                p.ph_wh[q] = ph[(size_t)q].wh;
-                p.ph_wl[q] = ph[(size_t)q].wl;
-            }
-        }
-        p.wh = m.wh;
-        p.wl = m.wl;
-        p.ew = m.ew;
-        p.M = v.out_channels;
-        p.mtiles = m.mtiles;
-        p.ksteps = m.ksteps;
-        p.cin = v.in_channels;
-        p.cin16 = m.cin16;
-        p.ksize = J;
-        p.dilation = 1;
-        p.len = len;
-        p.x = x;
-        p.sxc = len;
-        p.sxn = 1;
-        p.xmax = xmax;
-        p.bias = v.bias;
-        p.epi = DEC_EPI_STORE;
-        p.c = c;
-        p.ldc = (long long)len * v.stride;
-        p.out_stride = v.stride;
-        p.phase = r;
-        launch_dec_conv_mfma(d->ctx->stream, p);
-        QTTS_TRY(check_launch(d->ctx, "k_dec_conv_mfma"));
-        if (one) break;  // the launch ran every phase
+// J = kernel / stride taps reaching J - 1 steps back; the channels' phases
+// are the rows of one convolution.  omax (or null): receives max |out|.
+qtts_status dec_transposed_mfma(qtts_decoder *d, const qtts_conv_view &v, const DecConvMfma &m, const float *x,
+                                const unsigned *xmax, int len, float *c, unsigned *omax = nullptr) {
+    DecConvMfmaParams p{};
+    p.wh = m.wh;
+    p.wl = m.wl;
+    p.ew = m.ew;
+    p.M = v.out_channels * v.stride;
+    p.mtiles = m.mtiles;
+    p.ksteps = m.ksteps;
+    p.cin = v.in_channels;
+    p.cin16 = m.cin16;
+    p.ksize = v.kernel_size / v.stride;
+    p.dilation = 1;
+    p.len = len;
+    p.x = x;
+    p.sxc = len;
+    p.sxn = 1;
+    p.xmax = xmax;
+    p.bias = v.bias;
+    p.epi = DEC_EPI_STORE;
+    p.c = c;
+    p.ldc = (long long)len * v.stride;
+    p.out_stride = v.stride;
+    p.up = v.stride;
+    p.omax = omax;
+    const bool recorded = launch_dec_conv_mfma(d->ctx->stream, p);
+    QTTS_TRY(check_launch(d->ctx, "k_dec_conv_mfma"));
+    if (omax && !recorded) {
+        launch_dec_absmax(d->ctx->stream, c, (size_t)v.out_channels * v.stride * len, omax);
+        QTTS_TRY(check_launch(d->ctx, "k_dec_absmax"));
     }
     return QTTS_OK;
 }
@@ -3653,11 +3641,12 @@ qtts_status dec_decode(qtts_decoder *d, const uint32_t *d_codes, int T, int ld, 
         launch_dec_snake(st, sig, b.pre_snake_alpha, b.pre_snake_beta, cin, L, t1, m0, pend, pend ? sig : nullptr);
         pend = nullptr;
         QTTS_TRY(check_launch(c, "k_dec_snake"));
-        QTTS_TRY(dec_transposed_mfma(d, b.upsample, d->up_mfma[bi], t1, m0, L, nxt));
+        unsigned *msig = nullptr;  // max |sig|, where a fused unit reads it
+        if (fuse && b.num_residuals > 0 && d->res_unit[bi][0].ea1) QTTS_TRY(own(&msig));
+        QTTS_TRY(dec_transposed_mfma(d, b.upsample, d->up_mfma[bi], t1, m0, L, nxt, msig));
         L *= b.upsample.stride;
         sig = nxt;
         float *t2 = other(sig, t1);
-        unsigned *msig = nullptr;  // max |sig|, where a fused unit recorded it
         for (int r = 0; r < b.num_residuals; r++) {
             const qtts_vocos_residual_view &rv = b.residuals[r];
             const std::array<DecConvMfma, 2> &mc = d->res_mfma[bi][(size_t)r];
@@ -3832,7 +3821,7 @@ qtts_status qtts_decoder_upload(qtts_ctx *c, const qtts_decoder_view *v, qtts_de
             (s = up(U.pw2_b, (size_t)ch, &D.pw2_b, "pw2_b")) != QTTS_OK ||
             (s = up(U.gamma, (size_t)ch, &D.gamma, "gamma")) != QTTS_OK)
             return bail(s);
-        std::vector<DecConvMfma> ph;
+        DecConvMfma ph;
         std::array<DecConvMfma, 2> pw{};
         if ((s = dec_convt_mfma(c, o, U.conv_t, D.conv_t, &ph)) != QTTS_OK ||
             (s = dec_lin_mfma(c, o, U.pw1_w, D.pw1_w, ch, U.inner_dim, &pw[0])) != QTTS_OK ||

@@ -15,12 +15,12 @@
 //                 max |out| for the convolution that reads it
 //  k_dec_conv_mfma  every projection and convolution on the matrix cores
 //                 (v_mfma_f32_32x32x16_f16 with binary16 hi + lo operands):
-//                 causal convolutions as implicit GEMMs, one output phase
-//                 of a transposed convolution, linear layers as one tap;
+//                 causal convolutions as implicit GEMMs, a transposed
+//                 convolution's phases as rows, linear layers as one tap;
 //                 fused epilogues; k_dec_conv_win for convolutions of 3+
 //                 taps (the input window split once into LDS; the variant
 //                 k_dec_conv_win_tw, one channel tile per wave, at 3 and 4
-//                 tiles),
+//                 tiles, for 2+ taps),
 //                 k_dec_conv_mfma_ks for launches too small to fill the GPU
 //  k_dec_resunit  a residual unit of 96 or 192 channels (both SnakeBetas,
 //                 both convolutions, the residual) in one launch
@@ -418,12 +418,14 @@ __device__ __forceinline__ int split_exponent(float m) {
 // ci = 16 cb + 8 (lane / 32) + i (zero past M or cin): the element
 // w[m * sm + ci * sci + k0 + tap * kd] -- for a causal convolution
 // W[m][ci][tap] (src/conv.rs:114-184: sm = cin * ksize, sci = ksize, k0 = 0,
-// kd = 1); for output phase r of a transposed one W[ci][m][r + (J-1-tap) s]
-// (src/conv.rs:198-268: sm = ksize, sci = M * ksize, k0 = r + (J - 1) s,
-// kd = -s), so that tap t reads the input J - 1 - t steps back.
+// kd = 1).  up > 1: row m is output phase m % up of channel m / up of a
+// transposed one, W[ci][m / up][m % up + (J-1-tap) up] (src/conv.rs:198-268:
+// sm = ksize, sci = channels * ksize, k0 = (J - 1) up, kd = -up), so that tap
+// t reads the input J - 1 - t steps back.
 // hi = f16(w'), lo = f16(w' - hi).
 __global__ void k_dec_conv_repack(const float *w, long long sm, long long sci, int k0, int kd, int M, int cin,
-                                  int taps, int cin16, int mtiles, int ksteps, int ew, _Float16 *wh, _Float16 *wl) {
+                                  int taps, int cin16, int mtiles, int ksteps, int ew, int up, _Float16 *wh,
+                                  _Float16 *wl) {
     const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= (size_t)mtiles * ksteps * 64) return;
     const int lane = (int)(idx & 63);
@@ -436,7 +438,7 @@ __global__ void k_dec_conv_repack(const float *w, long long sm, long long sci, i
     for (int i = 0; i < 8; i++) {
         const int ci = 16 * cb + (kb & 15) + i;
         const float v = (m < M && ci < cin && tap < taps)
-                            ? ldexpf(w[(long long)m * sm + (long long)ci * sci + k0 + (long long)tap * kd], ew)
+                            ? ldexpf(w[(long long)(m / up) * sm + m % up + (long long)ci * sci + k0 + (long long)tap * kd], ew)
                             : 0.0f;
         const _Float16 hv = (_Float16)v;
         h[i] = hv;
@@ -444,6 +446,26 @@ __global__ void k_dec_conv_repack(const float *w, long long sm, long long sci, i
     }
     reinterpret_cast<half8 *>(wh)[idx] = h;
     reinterpret_cast<half8 *>(wl)[idx] = l;
+}
+
+// Row m's channel and output phase (m = channel * up + phase; up_inv as
+// launch_dec_conv_mfma sets it), and the output of row m at position n.
+__device__ __forceinline__ int dec_row_channel(const DecConvMfmaParams &P, int m) {
+    return P.up_inv ? (int)__umulhi((unsigned)m, P.up_inv) : m;
+}
+__device__ __forceinline__ float dec_conv_out(const DecConvMfmaParams &P, int m, int n, float v) {
+    const int ch = dec_row_channel(P, m);
+    if (P.bias) v += P.bias[ch];
+    if (P.act == DEC_ACT_GELU) v = dec_gelu(v);
+    float *dst = P.c + (long long)ch * P.ldc + (long long)n * P.out_stride + (m - ch * P.up);
+    switch (P.epi) {
+        case DEC_EPI_STORE: *dst = v; break;
+        case DEC_EPI_ACCUM: *dst += v; break;
+        case DEC_EPI_SCALED_RESID: *dst += P.scale[m] * v; break;
+        case DEC_EPI_RESID_IN: *dst = P.resid[dst - P.c] + (P.scale ? P.scale[m] * v : v); break;
+        default: *dst = v < -1.0f ? -1.0f : (v > 1.0f ? 1.0f : v); break;  // DEC_EPI_CLAMP (NaN stays)
+    }
+    return v;
 }
 
 // A causal convolution c[m][n] = bias[m] + sum_{ci, tap} W[m][ci][tap] *
@@ -476,9 +498,7 @@ __global__ __launch_bounds__(256) void k_dec_conv_mfma(DecConvMfmaParams P) {
     const int n = (blockIdx.x * 4 + wave) * 32 + col;  // this lane's output step
     const int t0 = blockIdx.y * MT;
     const int len = P.len, cin16 = P.cin16, ksteps = P.ksteps, nstage = ksteps / G;
-    const bool multi = P.nphase > 1;  // uniform
-    const _Float16 *wh = multi ? P.ph_wh[blockIdx.z] : P.wh, *wl = multi ? P.ph_wl[blockIdx.z] : P.wl;
-    const int phase = multi ? (int)blockIdx.z : P.phase;
+    const _Float16 *wh = P.wh, *wl = P.wl;
     // max |x| over the producer's slots, one per lane
     const int ex = split_exponent(wave_max(__uint_as_float(P.xmax[lane])));
     const float xs = ldexpf(1.0f, ex);
@@ -574,16 +594,7 @@ __global__ __launch_bounds__(256) void k_dec_conv_mfma(DecConvMfmaParams P) {
             const int m = 32 * (t0 + t) + (r >> 2) * 8 + half * 4 + (r & 3);
             if (m >= P.M) continue;
             float v = ldexpf(acc[t][r], sc);
-            if (P.bias) v += P.bias[m];
-            if (P.act == DEC_ACT_GELU) v = dec_gelu(v);
-            float *dst = P.c + (long long)m * P.ldc + (long long)n * P.out_stride + phase;
-            switch (P.epi) {
-                case DEC_EPI_STORE: *dst = v; break;
-                case DEC_EPI_ACCUM: *dst += v; break;
-                case DEC_EPI_SCALED_RESID: *dst += P.scale[m] * v; break;
-                case DEC_EPI_RESID_IN: *dst = P.resid[dst - P.c] + (P.scale ? P.scale[m] * v : v); break;
-                default: *dst = v < -1.0f ? -1.0f : (v > 1.0f ? 1.0f : v); break;  // DEC_EPI_CLAMP (NaN stays)
-            }
+            dec_conv_out(P, m, n, v);
         }
 }
 
@@ -602,21 +613,15 @@ __global__ __launch_bounds__(64 * NW) void k_dec_conv_mfma_ks(DecConvMfmaParams 
     __shared__ float red[NW][16][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 31, half = lane >> 5;
-    // Blocks of one XCD (every 8th) take a contiguous run of (phase, tile,
+    // Blocks of one XCD (every 8th) take a contiguous run of (tile,
     // positions), positions innermost: a tile's weights then come into one
     // XCD's L2 only.
     const int len = P.len, ksteps = P.ksteps;
-    const int nx = (len + 31) / 32, total = nx * P.mtiles * max(1, P.nphase), per = (int)(gridDim.x >> 3);
+    const int nx = (len + 31) / 32, total = nx * P.mtiles, per = (int)(gridDim.x >> 3);
     const int L = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
     if (L >= total) return;
-    const int ty = __builtin_amdgcn_readfirstlane(L / nx), n = (L - ty * nx) * 32 + col;
-    const int z = __builtin_amdgcn_readfirstlane(ty / P.mtiles), tile = ty - z * P.mtiles;
-    const bool multi = P.nphase > 1;  // uniform
+    const int tile = __builtin_amdgcn_readfirstlane(L / nx), n = (L - tile * nx) * 32 + col;
     const _Float16 *wh = P.wh, *wl = P.wl;
-#pragma unroll
-    for (int i = 0; i < kDecMaxPhases; i++)  // selected one by one: indexed by z, the parameters go to scratch
-        if (multi && z == i) wh = P.ph_wh[i], wl = P.ph_wl[i];
-    const int phase = multi ? z : P.phase;
     const int q = (ksteps + NW - 1) / NW, s0 = wave * q, s1 = min(ksteps, s0 + q);
     const unsigned xmax = P.xmax[lane];
     const half8 *ah0 = reinterpret_cast<const half8 *>(wh) + (size_t)tile * ksteps * 64;
@@ -697,16 +702,7 @@ __global__ __launch_bounds__(64 * NW) void k_dec_conv_mfma_ks(DecConvMfmaParams 
         for (int w = 1; w < NW; w++) v += red[w][r][lane];
         if (m >= P.M) continue;
         v = ldexpf(v, sc);
-        if (P.bias) v += P.bias[m];
-        if (P.act == DEC_ACT_GELU) v = dec_gelu(v);
-        float *dst = P.c + (long long)m * P.ldc + (long long)n * P.out_stride + phase;
-        switch (P.epi) {
-            case DEC_EPI_STORE: *dst = v; break;
-            case DEC_EPI_ACCUM: *dst += v; break;
-            case DEC_EPI_SCALED_RESID: *dst += P.scale[m] * v; break;
-            case DEC_EPI_RESID_IN: *dst = P.resid[dst - P.c] + (P.scale ? P.scale[m] * v : v); break;
-            default: *dst = v < -1.0f ? -1.0f : (v > 1.0f ? 1.0f : v); break;  // DEC_EPI_CLAMP (NaN stays)
-        }
+        dec_conv_out(P, m, n, v);
     }
 }
 
@@ -733,9 +729,7 @@ __global__ __launch_bounds__(256) void k_dec_conv_win(DecConvMfmaParams P) {
     const int n0 = blockIdx.x * 128, n = n0 + wave * 32 + col;
     const int t0 = blockIdx.y * MT;
     const int len = P.len, ks = P.ksize, dil = P.dilation, ksteps = P.ksteps;
-    const bool multi = P.nphase > 1;  // uniform
-    const _Float16 *wh = multi ? P.ph_wh[blockIdx.z] : P.wh, *wl = multi ? P.ph_wl[blockIdx.z] : P.wl;
-    const int phase = multi ? (int)blockIdx.z : P.phase;
+    const _Float16 *wh = P.wh, *wl = P.wl;
     const int W = 128 + (ks - 1) * dil, wpos = n0 - (ks - 1) * dil + tid;  // this thread's window position
     const bool wok = tid < W && wpos >= 0 && wpos < len;
     const int ncb = P.cin16 / 16;
@@ -819,16 +813,7 @@ __global__ __launch_bounds__(256) void k_dec_conv_win(DecConvMfmaParams P) {
             const int m = 32 * (t0 + t) + (r >> 2) * 8 + half * 4 + (r & 3);
             if (m >= P.M) continue;
             float v = ldexpf(acc[t][r], sc);
-            if (P.bias) v += P.bias[m];
-            if (P.act == DEC_ACT_GELU) v = dec_gelu(v);
-            float *dst = P.c + (long long)m * P.ldc + (long long)n * P.out_stride + phase;
-            switch (P.epi) {
-                case DEC_EPI_STORE: *dst = v; break;
-                case DEC_EPI_ACCUM: *dst += v; break;
-                case DEC_EPI_SCALED_RESID: *dst += P.scale[m] * v; break;
-                case DEC_EPI_RESID_IN: *dst = P.resid[dst - P.c] + (P.scale ? P.scale[m] * v : v); break;
-                default: *dst = v < -1.0f ? -1.0f : (v > 1.0f ? 1.0f : v); break;  // DEC_EPI_CLAMP (NaN stays)
-            }
+            dec_conv_out(P, m, n, v);
         }
 }
 
@@ -842,20 +827,32 @@ __global__ __launch_bounds__(256) void k_dec_conv_win(DecConvMfmaParams P) {
 // is staged by the block's 64 * NW threads, position t + 64 * NW * q by
 // thread t in pass q.  Same window, operands and product order per output
 // as k_dec_conv_win: the same bits.
+// The transposed convolutions (2 taps) come here with their phases as rows:
+// the input is read for all of them at once and each stretch of the output
+// is written whole, 16 bytes at a time where 4 rows are 4 phases of one
+// channel.  As one launch row per phase (k_dec_conv_mfma, each gathering the
+// input and writing every stride-th float) 768 -> 384 channels by 5 to
+// 80,000 positions took 437 us, 384 -> 192 by 4 to 320,000 563, 192 -> 96 by
+// 3 to 960,000 601 and 67 more for max |out|; here 424, 375 and 486.
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void k_dec_conv_win_tw(DecConvMfmaParams P) {
     static_assert(kDecMaxSlots == 64, "one max slot per lane");
     constexpr int WMAX = 256, PT = 4;  // window positions; 32-position tiles per block
     constexpr int NT = 64 * NW, NP = (WMAX + NT - 1) / NT;  // threads; staging passes
     __shared__ __align__(16) _Float16 wh_s[2][2][WMAX][8], wl_s[2][2][WMAX][8];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, half = lane >> 5;
-    const int n0 = blockIdx.x * 128;
-    const int tile = blockIdx.y * NW + wave;  // < mtiles (the grid has mtiles / NW rows)
+    // Blocks of one XCD (every 8th) take a contiguous run of (positions, tile
+    // group), the tile groups innermost where the input is the larger operand
+    // (it then comes into one XCD's L2 once), else the positions.
+    const int nx = (P.len + 127) / 128, ny = P.mtiles / NW, per = (int)(gridDim.x >> 3);
+    const int L = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if (L >= nx * ny) return;
+    const bool inner = (long long)P.mtiles * 32 * P.ksize < P.len;  // weights: 4 bytes per value, as the input
+    const int bx = inner ? L / ny : L % nx, by = inner ? L % ny : L / nx;
+    const int n0 = bx * 128, tile = by * NW + wave;
     const int len = P.len, ks = P.ksize, dil = P.dilation, ksteps = P.ksteps;
-    const bool multi = P.nphase > 1;  // uniform
-    const _Float16 *wh = multi ? P.ph_wh[blockIdx.z] : P.wh, *wl = multi ? P.ph_wl[blockIdx.z] : P.wl;
-    const int phase = multi ? (int)blockIdx.z : P.phase;
+    const _Float16 *wh = P.wh, *wl = P.wl;
     const int W = 128 + (ks - 1) * dil;  // window positions n0 - (ks - 1) * dil .. n0 + 127
     const int ncb = P.cin16 / 16;
     const int ex = split_exponent(wave_max(__uint_as_float(P.xmax[lane])));
@@ -933,26 +930,36 @@ __global__ __launch_bounds__(64 * NW) void k_dec_conv_win_tw(DecConvMfmaParams P
     // D layout: lane l, register r -> row (r / 4) * 8 + (l / 32) * 4 + r % 4,
     // column l % 32
     const int sc = -(ex + P.ew);
+    float mx = 0.0f;
 #pragma unroll
     for (int t = 0; t < PT; t++) {
         const int n = n0 + t * 32 + col;
         if (n >= len) continue;
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int m = 32 * tile + (r >> 2) * 8 + half * 4 + (r & 3);
-            if (m >= P.M) continue;
-            float v = ldexpf(acc[t][r], sc);
-            if (P.bias) v += P.bias[m];
-            if (P.act == DEC_ACT_GELU) v = dec_gelu(v);
-            float *dst = P.c + (long long)m * P.ldc + (long long)n * P.out_stride + phase;
-            switch (P.epi) {
-                case DEC_EPI_STORE: *dst = v; break;
-                case DEC_EPI_ACCUM: *dst += v; break;
-                case DEC_EPI_SCALED_RESID: *dst += P.scale[m] * v; break;
-                case DEC_EPI_RESID_IN: *dst = P.resid[dst - P.c] + (P.scale ? P.scale[m] * v : v); break;
-                default: *dst = v < -1.0f ? -1.0f : (v > 1.0f ? 1.0f : v); break;  // DEC_EPI_CLAMP (NaN stays)
+        for (int r = 0; r < 16; r += 4) {
+            const int m = 32 * tile + (r >> 2) * 8 + half * 4;
+            if (P.quad) {  // 4 phases of one channel: one 16-byte store
+                if (m >= P.M) continue;
+                const int ch = dec_row_channel(P, m);
+                const float b = P.bias ? P.bias[ch] : 0.0f;
+                float4 v;
+                v.x = ldexpf(acc[t][r], sc) + b;
+                v.y = ldexpf(acc[t][r + 1], sc) + b;
+                v.z = ldexpf(acc[t][r + 2], sc) + b;
+                v.w = ldexpf(acc[t][r + 3], sc) + b;
+                mx = fmaxf(fmaxf(mx, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+                *reinterpret_cast<float4 *>(P.c + (long long)ch * P.ldc + (long long)n * P.out_stride +
+                                            (m - ch * P.up)) = v;
+                continue;
             }
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (m + j < P.M) mx = fmaxf(mx, fabsf(dec_conv_out(P, m + j, n, ldexpf(acc[t][r + j], sc))));
         }
+    }
+    if (P.omax) {  // uniform
+        mx = wave_max(mx);
+        if (lane == 0) atomicMax(&P.omax[(blockIdx.x * NW + wave) % kDecMaxSlots], __float_as_uint(mx));
     }
 }
 
@@ -1297,10 +1304,10 @@ void launch_dec_fill_u32(hipStream_t st, unsigned *p, int n, unsigned v) {
 }
 
 void launch_dec_conv_repack(hipStream_t st, const float *w, long long sm, long long sci, int k0, int kd, int M, int cin,
-                            int taps, int cin16, int mtiles, int ksteps, int ew, _Float16 *wh, _Float16 *wl) {
+                            int taps, int cin16, int mtiles, int ksteps, int ew, int up, _Float16 *wh, _Float16 *wl) {
     const size_t n = (size_t)mtiles * ksteps * 64;
     hipLaunchKernelGGL(k_dec_conv_repack, dim3(blocks_for(n, 256)), dim3(256), 0, st, w, sm, sci, k0, kd, M, cin,
-                       taps, cin16, mtiles, ksteps, ew, wh, wl);
+                       taps, cin16, mtiles, ksteps, ew, up, wh, wl);
 }
 
 // At least 4 steps (one batch of loads) per wave, and no more waves than the
@@ -1319,7 +1326,7 @@ static void launch_conv_mfma_ks(hipStream_t st, const DecConvMfmaParams &p, dim3
 
 template <bool KF>
 static void launch_conv_mfma_kf(hipStream_t st, const DecConvMfmaParams &p, int mt) {
-    const dim3 grid(blocks_for((size_t)p.len, 128), (unsigned)(p.mtiles / mt), (unsigned)std::max(1, p.nphase));
+    const dim3 grid(blocks_for((size_t)p.len, 128), (unsigned)(p.mtiles / mt));
     switch (mt) {
         case 4: hipLaunchKernelGGL((k_dec_conv_mfma<4, KF>), grid, dim3(256), 0, st, p); break;
         case 3: hipLaunchKernelGGL((k_dec_conv_mfma<3, KF>), grid, dim3(256), 0, st, p); break;
@@ -1332,40 +1339,46 @@ static void launch_conv_mfma_kf(hipStream_t st, const DecConvMfmaParams &p, int 
 // tiles share each gathered B operand); a launch that would leave CUs idle
 // even at MT = 1 (fewer than kDecFillBlocks blocks) splits K over the
 // block's waves instead (k_dec_conv_mfma_ks); channel-first convolutions of
-// 3 or more taps take k_dec_conv_win.  QTTS_DEC_CONV=tiles or =split forces
+// 3 or more taps take k_dec_conv_win, of 2 where k_dec_conv_win_tw takes
+// them.  QTTS_DEC_CONV=tiles or =split forces
 // the long-decode kernels (MT by divisibility alone) or the K split for
 // every launch, so that short decodes can check both against a reference.
-void launch_dec_conv_mfma(hipStream_t st, const DecConvMfmaParams &p) {
+bool launch_dec_conv_mfma(hipStream_t st, DecConvMfmaParams p) {
     const char *plan = std::getenv("QTTS_DEC_CONV");
     const bool force_tiles = plan && std::strcmp(plan, "tiles") == 0, force_split = plan && std::strcmp(plan, "split") == 0;
     const bool kf = p.sxc == 1 && p.cin % 8 == 0 && p.sxn % 4 == 0 && ((uintptr_t)p.x & 15) == 0;
-    const size_t nph = (size_t)std::max(1, p.nphase);  // a transposed convolution's phases in one launch
+    // m / up = umulhi(m, up_inv) while m * up < 2^32
+    p.up_inv = p.up > 1 ? (unsigned)((1ull << 32) / (unsigned)p.up + 1) : 0;
     if (force_split ||
-        (!force_tiles && (size_t)blocks_for((size_t)p.len, 128) * (size_t)p.mtiles * nph < kDecFillBlocks)) {
-        const dim3 grid(blocks_for(blocks_for((size_t)p.len, 32) * (size_t)p.mtiles * nph, 8) * 8);
+        (!force_tiles && (size_t)blocks_for((size_t)p.len, 128) * (size_t)p.mtiles < kDecFillBlocks)) {
+        const dim3 grid(blocks_for(blocks_for((size_t)p.len, 32) * (size_t)p.mtiles, 8) * 8);
         if (kf)
             launch_conv_mfma_ks<true>(st, p, grid);
         else
             launch_conv_mfma_ks<false>(st, p, grid);
-        return;
+        return false;
     }
     int mt = p.mtiles % 4 == 0 ? 4 : p.mtiles % 3 == 0 ? 3 : p.mtiles % 2 == 0 ? 2 : 1;
-    if (!force_tiles && (size_t)blocks_for((size_t)p.len, 128) * (size_t)(p.mtiles / mt) * nph < 256) mt = 1;
-    if (p.ksize >= 3 && p.sxn == 1 && p.sxc == p.len && 128 + (p.ksize - 1) * p.dilation <= 256) {
-        // a channel-first convolution with 3 or more taps whose window fits the block's threads
-        const dim3 grid(blocks_for((size_t)p.len, 128), (unsigned)(p.mtiles / mt), (unsigned)nph);
+    if (!force_tiles && (size_t)blocks_for((size_t)p.len, 128) * (size_t)(p.mtiles / mt) < 256) mt = 1;
+    if (p.ksize >= (mt >= 3 ? 2 : 3) && p.sxn == 1 && p.sxc == p.len && 128 + (p.ksize - 1) * p.dilation <= 256) {
+        // a channel-first convolution whose window fits the block's threads
+        const dim3 grid(blocks_for((size_t)p.len, 128), (unsigned)(p.mtiles / mt));
+        const dim3 flat(blocks_for((size_t)grid.x * grid.y, 8) * 8);
+        p.quad = p.up > 1 && p.up % 4 == 0 && p.out_stride == p.up && p.ldc % 4 == 0 && p.epi == DEC_EPI_STORE &&
+                 p.act == DEC_ACT_NONE && ((uintptr_t)p.c & 15) == 0;
         switch (mt) {
-            case 4: hipLaunchKernelGGL(k_dec_conv_win_tw<4>, grid, dim3(256), 0, st, p); break;
-            case 3: hipLaunchKernelGGL(k_dec_conv_win_tw<3>, grid, dim3(192), 0, st, p); break;
+            case 4: hipLaunchKernelGGL(k_dec_conv_win_tw<4>, flat, dim3(256), 0, st, p); return true;
+            case 3: hipLaunchKernelGGL(k_dec_conv_win_tw<3>, flat, dim3(192), 0, st, p); return true;
             case 2: hipLaunchKernelGGL(k_dec_conv_win<2>, grid, dim3(256), 0, st, p); break;
             default: hipLaunchKernelGGL(k_dec_conv_win<1>, grid, dim3(256), 0, st, p); break;
         }
-        return;
+        return false;
     }
     if (kf)
         launch_conv_mfma_kf<true>(st, p, mt);
     else
         launch_conv_mfma_kf<false>(st, p, mt);
+    return false;
 }
 
 void launch_dec_absmax(hipStream_t st, const float *x, size_t n, unsigned *amax) {

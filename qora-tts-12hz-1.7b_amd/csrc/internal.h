@@ -107,30 +107,29 @@ enum DecEpi { DEC_EPI_STORE = 0, DEC_EPI_ACCUM = 1, DEC_EPI_SCALED_RESID = 2, DE
 // multiple of 16 with zero weights); x(ci, p) = x[ci * sxc + p * sxn],
 // split on the fly.  A linear
 // layer is the case ksize = 1 with m the output feature and n the row.
-constexpr int kDecMaxPhases = 8;  // output phases of one transposed-convolution launch
-
+// A transposed convolution of stride up is one whose rows are its channels'
+// output phases, m = channel * up + phase: one launch reads the input for all
+// of them and writes each stretch of the output whole.
 struct DecConvMfmaParams {
     const _Float16 *wh, *wl;  // [mtiles][ksteps][64][8]; row m = 32 * tile + lane % 32
     int ew;                   // the weights were scaled by 2^ew
-    int M, mtiles, ksteps;    // output channels, 32-row tiles, 16-row K steps (ksize * cin16 / 16,
+    int M, mtiles, ksteps;    // output rows (channels * up), 32-row tiles, 16-row K steps (ksize * cin16 / 16,
                               // rounded up to a multiple of kConvStage with zero weights)
     int cin, cin16, ksize, dilation, len;  // len: output positions n
     const float *x;
     long long sxc, sxn;       // x strides of a channel and a position
     const unsigned *xmax;     // [kDecMaxSlots]: bits of max |x| over the slots
-    const float *bias;        // [M] or null
+    const float *bias;        // [M / up] or null
     const float *scale;       // [M]: DEC_EPI_SCALED_RESID / DEC_EPI_RESID_IN (null: 1)
     int act, epi;             // DecAct, DecEpi
-    float *c;                 // output (m, n) at c[m * ldc + n * out_stride + phase]
+    float *c;                 // output (m, n) at c[m / up * ldc + n * out_stride + m % up]
     long long ldc;
     long long out_stride;
-    int phase;
+    int up;                   // >= 1
     const float *resid;       // DEC_EPI_RESID_IN: at the output's index (may be c)
-    // nphase > 1: one launch runs the output phases 0 .. nphase-1 of a
-    // transposed convolution (grid z = phase); phase p's weights are
-    // ph_wh[p] / ph_wl[p] (wh, wl and phase are then unused)
-    int nphase;
-    const _Float16 *ph_wh[kDecMaxPhases], *ph_wl[kDecMaxPhases];
+    unsigned *omax;           // null, or [kDecMaxSlots]: receives max |out| where the launch says so
+    unsigned up_inv;          // set by the launch: 0 (up = 1) or the multiplier that divides by up
+    bool quad;                // set by the launch: 4 rows are 4 neighbouring outputs, 16-byte aligned
 };
 
 // One residual unit (k_dec_resunit): x, out [C][len], distinct buffers; the
@@ -378,8 +377,9 @@ void launch_dec_snake(hipStream_t st, const float *x, const float *alpha, const 
 void launch_dec_fill_u32(hipStream_t st, unsigned *p, int n, unsigned v);
 void launch_dec_absmax(hipStream_t st, const float *x, size_t n, unsigned *amax);
 void launch_dec_conv_repack(hipStream_t st, const float *w, long long sm, long long sci, int k0, int kd, int M, int cin,
-                            int taps, int cin16, int mtiles, int ksteps, int ew, _Float16 *wh, _Float16 *wl);
-void launch_dec_conv_mfma(hipStream_t st, const DecConvMfmaParams &p);
+                            int taps, int cin16, int mtiles, int ksteps, int ew, int up, _Float16 *wh,
+                            _Float16 *wl);
+bool launch_dec_conv_mfma(hipStream_t st, DecConvMfmaParams p);  // true: max |out| is in p.omax
 // Whether k_dec_resunit takes a residual unit of these shapes.
 bool dec_resunit_fits(int channels, int ksize1, int dilation, int ksize2);
 void launch_dec_resunit(hipStream_t st, const DecResUnitParams &p, int channels);
