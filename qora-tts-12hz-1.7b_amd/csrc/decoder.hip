@@ -22,7 +22,7 @@
 //                 k_dec_conv_win_tw, one channel tile per wave, at 3 and 4
 //                 tiles, for 2+ taps),
 //                 k_dec_conv_mfma_ks for launches too small to fill the GPU
-//  k_dec_resunit  a residual unit of 96 or 192 channels (both SnakeBetas,
+//  k_dec_resunit  a residual unit of 96, 192 or 384 channels (both SnakeBetas,
 //                 both convolutions, the residual) in one launch
 //  k_dec_absmax   max |x| of a layer input (the operand scale)
 #include <hip/hip_runtime.h>
@@ -497,7 +497,7 @@ __global__ __launch_bounds__(256) void k_dec_conv_mfma(DecConvMfmaParams P) {
     const int col = lane & 31, half = lane >> 5;
     const int n = (blockIdx.x * 4 + wave) * 32 + col;  // this lane's output step
     const int t0 = blockIdx.y * MT;
-    const int len = P.len, cin16 = P.cin16, ksteps = P.ksteps, nstage = ksteps / G;
+    const int len = P.len, ksteps = P.ksteps, nstage = ksteps / G;
     const _Float16 *wh = P.wh, *wl = P.wl;
     // max |x| over the producer's slots, one per lane
     const int ex = split_exponent(wave_max(__uint_as_float(P.xmax[lane])));
@@ -997,8 +997,8 @@ __device__ __forceinline__ float dec_sin2(float t) {
 // through L1 by the 12 / CT waves of its tile; A operands are loaded three
 // to four taps ahead.  conv1's operand scale bounds SnakeBeta by max |x| +
 // max exp(-beta), and max |out| is recorded for the next unit.
-// C = 96, 960,000 positions: 1130 us as five launches, 624 here; C = 192,
-// 240,000 positions: 1060, 665.  Matrix cores a third busy, vector ALU (the
+// C = 96, 960,000 positions: 1130 us as five launches, 590 here; C = 192,
+// 320,000 positions: 1060, 650; C = 384, 80,000: 810, 565.  Matrix cores a third busy, vector ALU (the
 // sines and splits) a third, the rest latency: one block a CU.  Blocks of 6
 // waves and half the positions measured slower (C = 96, 805 us: twice the A
 // operands through the L2).
