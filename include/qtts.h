@@ -178,7 +178,13 @@ qtts_status qtts_gemv(qtts_ctx *ctx, const qtts_q4 *w, const float *input, float
 qtts_status qtts_gemm(qtts_ctx *ctx, const qtts_q4 *w, const float *x, int32_t seq_len, float *output);
 /* embed_lookup(weight, token_id, n) -> [n]; src/gemv.rs:164-176 -> embed_lookup_q4 377-400. */
 qtts_status qtts_embed_lookup(qtts_ctx *ctx, const qtts_q4 *w, int32_t token_id, float *output);
-/* Same operators on device buffers, enqueued on the context stream. */
+/* Same operators on device buffers, enqueued on the context stream.  The first
+ * call of 8 or more rows with a weight allocates its operand copy, and the
+ * first on a context its scratch for that shape at any number of rows; later
+ * calls of the shape allocate nothing and do not synchronise, so they can be
+ * captured into a graph.  Scratch that a larger weight outgrows is kept until
+ * the context goes: captured calls stay valid.  The scratch is shared by the
+ * context's calls: replay a graph in order with them (on the context stream). */
 qtts_status qtts_gemv_device(qtts_ctx *ctx, const qtts_q4 *w, const float *d_input, float *d_output);
 qtts_status qtts_gemm_device(qtts_ctx *ctx, const qtts_q4 *w, const float *d_x, int32_t seq_len, float *d_output);
 /* No counterpart in the reference: qtts_gemm_device for 1..4 rows that

@@ -63,6 +63,7 @@ struct qtts_ctx {
     size_t mfma_x_cap = 0;
     float *mfma_part = nullptr;
     size_t mfma_part_cap = 0;
+    std::vector<void *> mfma_old;  // outgrown scratch: a graph captured on the stream may still name it
     // The context and every object made from it hold one reference each, so
     // objects may be freed after qtts_ctx_destroy (e.g. in any order at
     // interpreter shutdown).
@@ -92,6 +93,7 @@ void ctx_release(qtts_ctx *c) {
     (void)hipFree(c->eng_trace);
     (void)hipFree(c->mfma_x);
     (void)hipFree(c->mfma_part);
+    for (void *p : c->mfma_old) (void)hipFree(p);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }
@@ -317,51 +319,6 @@ qtts_status run_gemv(qtts_ctx *c, const GemvParams &p) {
     return check_launch(c, "k_gemv");
 }
 
-// The MFMA operand copy of a panel-major weight (one allocation at *mem).
-// *ok is false (and *mem null) for a weight the matrix-core path cannot take
-// exactly: a shape off the 16 x 32 grid, K above the row prologue's limit,
-// or a scale above 8188 in magnitude.  Synchronises the stream.
-qtts_status make_mfma_copy(qtts_ctx *c, const DevQ4 &w, void **mem, DevQ4Mfma *m, bool *ok) {
-    *mem = nullptr;
-    *ok = false;
-    if (w.K % 16 != 0 || w.N % 32 != 0 || w.K > kMfmaRowsMaxK) return QTTS_OK;
-    const size_t nw = (size_t)(w.N / 32) * (w.K / 16) * 64, ns = (size_t)(w.N / 32) * w.K;
-    const size_t flag_off = (nw * 4 + 2 * ns * 2 + 255) / 256 * 256;
-    HIP_TRY(c, hipMalloc(mem, flag_off + 256));
-    m->wm = reinterpret_cast<uint32_t *>(*mem);
-    m->sa = reinterpret_cast<uint16_t *>((uint8_t *)*mem + nw * 4);
-    m->sb = m->sa + ns;
-    m->K = w.K;
-    m->N = w.N;
-    int *flag = reinterpret_cast<int *>((uint8_t *)*mem + flag_off);
-    HIP_TRY(c, hipMemsetAsync(flag, 0, sizeof(int), c->stream));
-    launch_repack_mfma(c->stream, w, const_cast<uint32_t *>(m->wm), const_cast<uint16_t *>(m->sa),
-                       const_cast<uint16_t *>(m->sb), flag);
-    QTTS_TRY(check_launch(c, "k_repack_mfma"));
-    int too_large = 0;
-    HIP_TRY(c, hipMemcpyAsync(&too_large, flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-    if (too_large) {
-        (void)hipFree(*mem);
-        *mem = nullptr;
-        return QTTS_OK;
-    }
-    *ok = true;
-    return QTTS_OK;
-}
-
-template <class T>
-qtts_status grow(qtts_ctx *c, T **buf, size_t *cap, size_t need) {
-    if (*cap >= need) return QTTS_OK;
-    HIP_TRY(c, hipStreamSynchronize(c->stream));
-    (void)hipFree(*buf);
-    *buf = nullptr;
-    *cap = 0;
-    HIP_TRY(c, hipMalloc(buf, need * sizeof(T)));
-    *cap = need;
-    return QTTS_OK;
-}
-
 // Steps per wave and K chunks of the product of 17 to 64 rows: 16 steps where
 // that still makes 192 blocks, else 8; 4 where 8 would make chunks and fewer
 // than 192 blocks.  64 rows, 16 / 8 steps: 6144 -> 2048 18.3 / 20.0
@@ -443,21 +400,83 @@ void mfma16_plan(int K, int N, int *sw, int *kc) {
     *sw = s;
 }
 
-// Grows the MFMA GEMM scratch for a K x N weight at up to M rows, so that a
-// later call allocates nothing (e.g. under stream capture).
-qtts_status mfma_reserve(qtts_ctx *c, int K, int N, int M) {
+// The GEMM scratch of a K x N weight at any number of rows: binary16 values
+// of the split rows and floats of the partials.  The plans are not monotonic
+// in the rows (fewer may take more K chunks), so every number of row tiles is
+// looked at, 126 of them, once per operand copy (20 us).  6144 -> 2048: 101
+// MB and 71 MB; launches of at most 2048 rows would halve the first, but 4096
+// rows of that weight take 298 us in one launch and 326 in two, of 2048 ->
+// 2048 108 and 139.
+void mfma_scratch(int K, int N, size_t *x, size_t *part) {
     int sw, kc;
+    size_t rows = 64;
     mfma_plan(K, N, &sw, &kc);
-    size_t rows = 64, part = kc > 1 ? (size_t)kc * (M > 32 ? 64 : 32) * N : 0;
+    *part = kc > 1 ? (size_t)kc * 64 * N : 0;
     mfma16_plan(K, N, &sw, &kc);
-    if (kc > 1) part = std::max(part, (size_t)kc * kMfma16Rows * N);
-    if (M > kMfmaPassRows) {
-        const GemmTilePlan t = tile_plan(M < kTileMaxRows ? M : kTileMaxRows, K, N);
+    if (kc > 1) *part = std::max(*part, (size_t)kc * kMfma16Rows * N);
+    for (int M = kMfmaPassRows + 32; M <= kTileMaxRows; M += 32) {
+        const GemmTilePlan t = tile_plan(M, K, N);
         rows = std::max(rows, (size_t)32 * t.mt * t.mb);
-        part = std::max(part, tile_part_floats(t));
+        *part = std::max(*part, tile_part_floats(t));
     }
-    QTTS_TRY(grow(c, &c->mfma_x, &c->mfma_x_cap, 2 * rows * K + 2 * rows));
-    return grow(c, &c->mfma_part, &c->mfma_part_cap, part);
+    *x = 2 * rows * K + 2 * rows;  // 16-row operands of whole 32-row steps included: 2 * 16 * (K + 16) + 32
+}
+
+// The MFMA operand copy of a panel-major weight (one allocation at *mem).
+// *ok is false (and *mem null) for a weight the matrix-core path cannot take
+// exactly: a shape off the 16 x 32 grid, K above the row prologue's limit,
+// or a scale above 8188 in magnitude.  Synchronises the stream.
+qtts_status make_mfma_copy(qtts_ctx *c, const DevQ4 &w, void **mem, DevQ4Mfma *m, bool *ok) {
+    *mem = nullptr;
+    *ok = false;
+    if (w.K % 16 != 0 || w.N % 32 != 0 || w.K > kMfmaRowsMaxK) return QTTS_OK;
+    const size_t nw = (size_t)(w.N / 32) * (w.K / 16) * 64, ns = (size_t)(w.N / 32) * w.K;
+    const size_t flag_off = (nw * 4 + 2 * ns * 2 + 255) / 256 * 256;
+    HIP_TRY(c, hipMalloc(mem, flag_off + 256));
+    m->wm = reinterpret_cast<uint32_t *>(*mem);
+    m->sa = reinterpret_cast<uint16_t *>((uint8_t *)*mem + nw * 4);
+    m->sb = m->sa + ns;
+    m->K = w.K;
+    m->N = w.N;
+    mfma_scratch(w.K, w.N, &m->scratch_x, &m->scratch_part);
+    int *flag = reinterpret_cast<int *>((uint8_t *)*mem + flag_off);
+    HIP_TRY(c, hipMemsetAsync(flag, 0, sizeof(int), c->stream));
+    launch_repack_mfma(c->stream, w, const_cast<uint32_t *>(m->wm), const_cast<uint16_t *>(m->sa),
+                       const_cast<uint16_t *>(m->sb), flag);
+    QTTS_TRY(check_launch(c, "k_repack_mfma"));
+    int too_large = 0;
+    HIP_TRY(c, hipMemcpyAsync(&too_large, flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    if (too_large) {
+        (void)hipFree(*mem);
+        *mem = nullptr;
+        return QTTS_OK;
+    }
+    *ok = true;
+    return QTTS_OK;
+}
+
+// The context's scratch for a weight, sized by the first product with it for
+// any number of rows: no later product of that shape allocates (e.g. under
+// stream capture).  A block that a larger weight outgrows is kept until the
+// context goes, since work in flight and graphs captured on the stream use
+// it; each is at least twice the one before, so all of them together are
+// smaller than the current one.
+template <class T>
+qtts_status grow_kept(qtts_ctx *c, T **buf, size_t *cap, size_t need) {
+    if (*cap >= need) return QTTS_OK;
+    need = std::max(need, 2 * *cap);
+    T *p = nullptr;
+    HIP_TRY(c, hipMalloc(&p, need * sizeof(T)));
+    if (*buf) c->mfma_old.push_back(*buf);
+    *buf = p;
+    *cap = need;
+    return QTTS_OK;
+}
+
+qtts_status mfma_reserve(qtts_ctx *c, const DevQ4Mfma &w) {
+    QTTS_TRY(grow_kept(c, &c->mfma_x, &c->mfma_x_cap, w.scratch_x));
+    return grow_kept(c, &c->mfma_part, &c->mfma_part_cap, w.scratch_part);
 }
 
 // y[m] (+)= f(x[m]) . W (+ bias) for M rows on the matrix cores
@@ -472,6 +491,7 @@ qtts_status run_gemm_mfma(qtts_ctx *c, const DevQ4Mfma &w, const float *x, int M
     if (K % 16 || N % 32 || K > kMfmaRowsMaxK || ldx % 4 || ((uintptr_t)x & 15))
         return fail(c, QTTS_ESHAPE, "MFMA GEMM: unsupported shape or unaligned rows");
     if (panels > kCounters) return fail(c, QTTS_ESHAPE, "MFMA GEMM: more panels than counters");
+    QTTS_TRY(mfma_reserve(c, w));
     for (int r0 = 0; r0 < M; r0 += kTileMaxRows) {
         const int Mc = M - r0 < kTileMaxRows ? M - r0 : kTileMaxRows;
         const bool tiled = Mc > kMfmaPassRows, m16 = Mc <= kMfma16Rows;
@@ -484,7 +504,6 @@ qtts_status run_gemm_mfma(qtts_ctx *c, const DevQ4Mfma &w, const float *x, int M
         else
             mfma_plan(K, N, &sw, &kc);
         const int mt = Mc > 32 ? 2 : 1, Mpad = tiled ? 32 * t.mt * t.mb : m16 ? kMfma16Rows : 32 * mt;
-        QTTS_TRY(mfma_reserve(c, K, N, Mc));
         MfmaRowsParams r{};
         r.x = x + (size_t)r0 * ldx;
         r.ldx = ldx;
@@ -4432,18 +4451,12 @@ qtts_status qtts_generate_codes_batch(qtts_talker *t, qtts_predictor *p, int32_t
             return QTTS_OK;
     };
     // every GEMM's scratch, reserved before capture
-    QTTS_TRY(mfma_reserve(c, H, ts.nq * ts.hd + 2 * ts.nkv * ts.hd, B));
-    QTTS_TRY(mfma_reserve(c, ts.nq * ts.hd, H, B));
-    QTTS_TRY(mfma_reserve(c, H, 2 * ts.inter, B));
-    QTTS_TRY(mfma_reserve(c, ts.inter, H, B));
-    QTTS_TRY(mfma_reserve(c, H, V, B));
+    for (const DevQ4Mfma &w : t->mfma) QTTS_TRY(mfma_reserve(c, w));
+    QTTS_TRY(mfma_reserve(c, t->head_mfma));
     if (!talker_only) {
-        if (!p->identity_proj) QTTS_TRY(mfma_reserve(c, H, hp, 2 * B));
-        QTTS_TRY(mfma_reserve(c, hp, ps->nq * ps->hd + 2 * ps->nkv * ps->hd, 2 * B));
-        QTTS_TRY(mfma_reserve(c, ps->nq * ps->hd, hp, 2 * B));
-        QTTS_TRY(mfma_reserve(c, hp, 2 * ps->inter, 2 * B));
-        QTTS_TRY(mfma_reserve(c, ps->inter, hp, 2 * B));
-        QTTS_TRY(mfma_reserve(c, hp, p->vocab, B));
+        if (!p->identity_proj) QTTS_TRY(mfma_reserve(c, p->mfma_in));
+        for (const DevQ4Mfma &w : p->mfma) QTTS_TRY(mfma_reserve(c, w));
+        for (const DevQ4Mfma &w : p->mfma_heads) QTTS_TRY(mfma_reserve(c, w));
     }
     const bool use_graph = std::getenv("QTTS_NO_GRAPH") == nullptr;
     hipGraph_t graph = nullptr;
