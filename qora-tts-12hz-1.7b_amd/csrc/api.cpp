@@ -2008,7 +2008,7 @@ static qtts_status make_talker_mfma(qtts_talker *t) {
 // prologue) -> down (SiLU*up prologue, +residual); src/talker.rs:364-462.
 // Up to kAttnPrefillRows rows, one block per row and kv head (k_attn: 6.8 us
 // at 10 rows, 8.0 at 64, 12.7 at 96) has the shorter chain; past them the
-// row-tiled kernel (k_attn_prefill: 9.4, 10.0 and 9.7 us) wins, 78 against
+// row-tiled kernel (k_attn_prefill: 9.4, 10.0 and 10.1 us) wins, 73 against
 // 620 us at 1064.
 constexpr int kAttnPrefillRows = 64;
 static_assert(kAttnPrefillRows <= kAttnMaxChunk, "one split holds every row's cache");

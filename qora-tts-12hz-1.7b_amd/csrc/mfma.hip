@@ -733,8 +733,8 @@ __global__ __launch_bounds__(64 * NW, 2) void k_gemm_mfma_tile(GemmMfmaParams P,
 // MFMA takes 64 cycles, 32 keys 8192, and their 32 KiB come from the L2
 // meanwhile.  Longest rows first; the query heads of one kv head (and so its
 // K and V) fall on one XCD where there are 8 kv heads.
-// 1064 rows, 16 heads: 78 us per layer (the f32 MFMAs alone 37), where k_attn
-// (one row per block) took 620.
+// 1064 rows, 16 heads: 73 us per layer (the f32 MFMAs alone 37), where k_attn
+// (one row per block) took 620; 300 rows 19.9, 96 rows 10.1.
 __global__ __launch_bounds__(256, 2) void k_attn_prefill(AttnParams P, int M) {
     constexpr int HD = 128;
     __shared__ float part[4][16][4][64];  // [wave][register][t][lane]
@@ -770,6 +770,10 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill(AttnParams P, int M) {
             vb[to][r] = *reinterpret_cast<const f32x4 *>(
                 V + (size_t)min(32 * kt + 8 * c + 4 * half + r, M - 1) * HD + 4 * col);
     };
+    // In the last run (the rows' own keys) an infinite or NaN V meets the
+    // queries that do not see its key with weight 0, which makes them NaN too.
+    // z, the largest |V| of that run or NaN, finds such a V.
+    float z = 0.0f;
     load_k(min(wave, qt), 0, 0);
     for (int kt = wave; kt <= qt; kt += 4) {
         const bool diag = kt == qt;
@@ -811,6 +815,7 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill(AttnParams P, int M) {
         for (int t = 0; t < 4; t++)
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[t][r] *= alpha;
+        z = diag ? 0.0f : z;
 #pragma unroll
         for (int c = 0; c < 4; c++) {
             if (c < 3)
@@ -823,8 +828,43 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill(AttnParams P, int M) {
 #pragma unroll
                 for (int t = 0; t < 4; t++)
                     acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(vb[c & 1][r][t], s[4 * c + r], acc[t], 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int t = 0; t < 4; t++) z = __builtin_elementwise_maximum(z, fabsf(vb[c & 1][r][t]));
             __builtin_amdgcn_sched_barrier(0);
         }
+    }
+    if (wave == (qt & 3) && __any(!(z < INFINITY))) {  // uniform
+        // the wave's keys again, one at a time for all 32 queries without the
+        // matrix cores, a lane skipping those it does not see: for 1500 rows
+        // 90 to 190 us more in a layer, however many rows are NaN (row by row
+        // over all keys, for every tile after the bad row, it was 4 ms)
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[t][r] = 0.0f;
+        for (int kt = wave; kt <= qt; kt += 4)
+#pragma unroll 1
+            for (int key = 32 * kt; key < min(32 * kt + 32, M); key++) {
+                const float *kr = K + (size_t)key * HD + 4 * half, *vr = V + (size_t)key * HD + 16 * half;
+                float d = 0.0f;
+#pragma unroll
+                for (int g = 0; g < 16; g++) {
+                    const f32x4 k = *reinterpret_cast<const f32x4 *>(kr + 8 * g);
+#pragma unroll
+                    for (int j = 0; j < 4; j++) d = fmaf(k[j], qv[g][j], d);
+                }
+                d = halves_sum(d);
+                if (key > q) continue;
+                const float p = expf(d * P.scale - mx);
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const f32x4 v = *reinterpret_cast<const f32x4 *>(vr + 4 * (8 * (r >> 2) + (r & 3)));
+#pragma unroll
+                    for (int t = 0; t < 4; t++) acc[t][r] = fmaf(p, v[t], acc[t][r]);
+                }
+            }
     }
     // merge: weights exp(max of the wave - max of all), sums in wave order
     if (half == 0) {
@@ -846,39 +886,14 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill(AttnParams P, int M) {
         for (int t = 0; t < 4; t++) part[wave][r][t][lane] = acc[t][r] * f;
     __syncthreads();
     float *o = P.out + (size_t)q * P.ldo + (size_t)head * HD;
-    bool odd = false;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const int r = 4 * wave + i;
         f32x4 v;
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
+        for (int t = 0; t < 4; t++)
             v[t] = ((part[0][r][t][lane] + part[1][r][t][lane]) + (part[2][r][t][lane] + part[3][r][t][lane])) / l;
-            odd |= !(fabsf(v[t]) < INFINITY);
-        }
         if (q < M) *reinterpret_cast<f32x4 *>(o + 4 * (8 * (r >> 2) + 4 * half + (r & 3))) = v;
-    }
-    if (!__syncthreads_or(odd)) return;
-    // An infinity or NaN: a key that a row does not see meets it with weight
-    // 0 in the last run's MFMAs.  The block's rows again, one at a time over
-    // the keys each sees, lane d holding dims d and d + 64.
-    for (int i = wave; i < 32 && 32 * qt + i < M; i += 4) {
-        const int row = 32 * qt + i;
-        const float *qq = P.q + (size_t)row * P.ldq + (size_t)head * HD;
-        const float q0 = qq[lane], q1 = qq[lane + 64];
-        float top = -INFINITY, den = 0.0f, o0 = 0.0f, o1 = 0.0f;
-        for (int k = 0; k <= row; k++)
-            top = fmaxf(top, wave_sum(q0 * K[(size_t)k * HD + lane] + q1 * K[(size_t)k * HD + lane + 64]) * P.scale);
-        for (int k = 0; k <= row; k++) {
-            const float sc = wave_sum(q0 * K[(size_t)k * HD + lane] + q1 * K[(size_t)k * HD + lane + 64]) * P.scale;
-            const float p = expf(sc - top);
-            den += p;
-            o0 += p * V[(size_t)k * HD + lane];
-            o1 += p * V[(size_t)k * HD + lane + 64];
-        }
-        float *dst = P.out + (size_t)row * P.ldo + (size_t)head * HD;
-        dst[lane] = o0 / den;
-        dst[lane + 64] = o1 / den;
     }
 }
 

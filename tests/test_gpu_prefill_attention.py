@@ -2,7 +2,9 @@
 the append) and past 64 (32-row tiles, four waves over the keys) against the
 oracle: the limits and one past them, whole and ragged tiles, one to four
 query heads per kv head; and a row of NaNs, which the rows before it must not
-see."""
+see and which must not cost the rows after it anything."""
+import time
+
 import numpy as np
 import pytest
 
@@ -46,3 +48,29 @@ def test_prefill_rows_before_a_nan_row_are_unchanged(ctx, rows, bad):
     for got, ref in zip(kv.store(), clean):
         assert np.all(np.isfinite(got[:, :bad])) and within(got[:, :bad], ref[:, :bad])
         assert np.all(np.isnan(got[1, bad:]).any(axis=(1, 2)))
+
+
+@pytest.mark.parametrize("bad", [slice(3, 4), slice(1499, 1500), slice(0, 1500, 32)])
+def test_prefill_time_with_nan_rows(ctx, bad):
+    """Where a tile's own rows hold a NaN its wave goes over its keys once more
+    on the vector units: 1.5 to 1.95 times the whole call here (20 times when
+    every tile after the bad row did it row by row)."""
+    rows = 1500
+    cfg, tw, t = _talker(ctx, 4, 2)
+    x = qtts.synth_normal_f32(33, "nan.t", rows * cfg.hidden).reshape(rows, -1).copy()
+    kv = t.new_kv(rows)
+
+    def best():
+        times = []
+        for _ in range(5):
+            kv.clear()
+            t0 = time.perf_counter()
+            t.prefill_talker_raw(x, rows, kv)
+            times.append(time.perf_counter() - t0)
+        return min(times)
+
+    clean = best()
+    x[bad, 7] = np.inf
+    slow = best()
+    print(f"{rows} rows: {clean * 1e6:.0f} us, with NaN rows {slow * 1e6:.0f}")
+    assert slow < 3.0 * clean
