@@ -797,8 +797,8 @@ struct qtts_talker {
     DevQ4 text_emb{}, fc1{}, fc2{};
     float *fc1_b = nullptr, *fc2_b = nullptr;
     int text_hidden = 0, has_text = 0;
-    DevQ4Mfma text_mfma[2] = {};  // operand copies of fc1 and fc2, made by the first projection of kTextMfmaRows rows
-    int text_mfma_state = 0;      // 0 not tried, 1 made, -1 a weight cannot use the matrix cores
+    DevQ4Mfma text_mfma[2] = {};  // operand copies of fc1 and fc2
+    bool text_mfma_ok = false;    // both are there
     float *tx_raw = nullptr, *tx_h = nullptr, *tx_rows = nullptr;
     float *pr_codec = nullptr;  // [8][hidden]: the prompt's codec rows and the voice row
     uint32_t *tx_tok = nullptr;
@@ -2235,7 +2235,7 @@ constexpr int kTextMfmaRows = 5;
 
 qtts_status text_layer(qtts_talker *t, int layer, float *x, int n, int mode, const float *bias, float *y) {
     const DevQ4 &w = layer == 0 ? t->fc1 : t->fc2;
-    if (n >= kTextMfmaRows && t->text_mfma_state == 1)
+    if (n >= kTextMfmaRows && t->text_mfma_ok)
         return run_gemm_mfma(t->ctx, t->text_mfma[layer], x, n, w.K, mode, nullptr, y, w.N, bias, false, nullptr, 0,
                              true);
     if (mode == MFMA_ROWS_SILU) {
@@ -2257,21 +2257,23 @@ qtts_status text_layer(qtts_talker *t, int layer, float *x, int n, int mode, con
     return QTTS_OK;
 }
 
-// The operand copies of both layers, or neither.
-qtts_status make_text_mfma(qtts_talker *t) {
-    bool all = true;
+// The operand copies of both layers and the scratch of their products, or
+// none of it: where a weight cannot use the matrix cores, or the device has no
+// room, the projection stays with the GEMV.
+void make_text_mfma(qtts_talker *t) {
+    qtts_ctx *c = t->ctx;
     void *mem[2] = {nullptr, nullptr};
-    for (int i = 0; i < 2 && all; i++) {
-        const qtts_status s = make_mfma_copy(t->ctx, i == 0 ? t->fc1 : t->fc2, &mem[i], &t->text_mfma[i], &all);
-        if (s != QTTS_OK || !all) {
-            for (void *p : mem) (void)hipFree(p);
-            if (s != QTTS_OK) return s;
-        }
+    bool ok = true;
+    for (int i = 0; i < 2 && ok; i++)
+        ok = make_mfma_copy(c, i == 0 ? t->fc1 : t->fc2, &mem[i], &t->text_mfma[i], &ok) == QTTS_OK && ok &&
+             mfma_reserve(c, t->text_mfma[i]) == QTTS_OK;
+    if (!ok) {
+        (void)hipGetLastError();
+        for (void *p : mem) (void)hipFree(p);
+        return;
     }
-    if (all)
-        for (void *p : mem) t->own.ptrs.push_back(p);
-    t->text_mfma_state = all ? 1 : -1;
-    return QTTS_OK;
+    for (void *p : mem) t->own.ptrs.push_back(p);
+    t->text_mfma_ok = true;
 }
 
 // embed_text_token of the n host tokens, rows [n][hidden] to `out` (device).
@@ -2284,7 +2286,6 @@ qtts_status text_project(qtts_talker *t, const uint32_t *tokens, int n, float *o
     HIP_TRY(c, hipMemcpyAsync(t->tx_tok, tokens, sizeof(uint32_t) * n, hipMemcpyHostToDevice, c->stream));
     launch_embed_rows(c->stream, t->text_emb, t->tx_tok, 1, n, t->tx_raw, t->text_hidden);
     QTTS_TRY(check_launch(c, "k_embed_rows"));
-    if (n >= kTextMfmaRows && t->text_mfma_state == 0) QTTS_TRY(make_text_mfma(t));
     QTTS_TRY(text_layer(t, 0, t->tx_raw, n, MFMA_ROWS_PLAIN, t->fc1_b, t->tx_h));
     return text_layer(t, 1, t->tx_h, n, MFMA_ROWS_SILU, t->fc2_b, out);
 }
@@ -2382,6 +2383,7 @@ qtts_status qtts_talker_text_upload(qtts_talker *t, const qtts_text_view *v) {
     QTTS_TRY(upload_array(c, t->own, v->text_proj_fc1_bias, (size_t)v->text_proj_fc1.n, &t->fc1_b, "text_proj_fc1_bias"));
     QTTS_TRY(upload_array(c, t->own, v->text_proj_fc2_bias, (size_t)H, &t->fc2_b, "text_proj_fc2_bias"));
     QTTS_TRY(t->own.alloc(c, &t->pr_codec, (size_t)8 * H));
+    make_text_mfma(t);
     t->text_hidden = th;
     t->has_text = 1;
     return QTTS_OK;

@@ -3,6 +3,7 @@ cores with all four partial products) against float64 at the edges of both,
 and the rows of one call against the same tokens one at a time."""
 import numpy as np
 import pytest
+import torch
 
 import qtts
 
@@ -43,3 +44,20 @@ def test_text_projection_rows(text, rows):
     assert np.linalg.norm(err) <= 4e-7 * np.linalg.norm(got)
     one = np.stack([t.embed_text_token(int(v)) for v in tok[:3]])
     assert np.allclose(got[:3], one, rtol=0, atol=1e-6 * np.abs(one).max())
+
+
+def test_first_projection_makes_no_operand_copies():
+    """The matrix cores' copies and scratch come with the text weights: the
+    first projection allocates its rows and no more (three buffers of 96 x
+    2048 floats and the tokens, each at most rounded up to 2 MiB)."""
+    ctx = qtts.Context(0)
+    cfg = qtts.StackConfig(layers=1, hidden=2048, heads=2, kv_heads=1, head_dim=128, inter=256, vocab=320,
+                           max_position=64)
+    t = qtts.Talker(ctx, qtts.TalkerWeights(43, cfg))
+    t.attach_text(qtts.TextWeights(43, qtts.TEXT_VOCAB_1P7B, 2048, 2048))
+    t.embed_text_token(5)
+    free = torch.cuda.mem_get_info()[0]
+    first = t.build_trailing_text(np.arange(97, dtype=np.uint32))
+    assert free - torch.cuda.mem_get_info()[0] <= 4 * 2 ** 21
+    assert np.array_equal(first, t.build_trailing_text(np.arange(97, dtype=np.uint32)))
+    ctx.close()
