@@ -963,22 +963,26 @@ __global__ __launch_bounds__(64 * NW) void k_dec_conv_win_tw(DecConvMfmaParams P
     }
 }
 
-// sin(t)^2 of SnakeBeta: t less the nearest multiple of pi (whose sine has
-// the same square), then sin r = r + r^3 p(r^2) on [-pi/2, pi/2], p fitted
-// for the least relative error (6e-9).  rms error 3.7e-8 over N(0, 6)
-// arguments, a correctly rounded sine's square 2.9e-8.  Past |t| = 8192,
-// where k * (pi - float(pi)) loses bits, the library's sinf.
+// sin(t)^2 of SnakeBeta.  r + e is t less the nearest multiple k of pi/2 (in
+// three parts: the first subtraction is exact, e what the second rounds off),
+// sin(r + e) = r + (e + r^3 p(r^2)) on [-pi/4, pi/4], p the least maximum
+// relative error (Lawson's reweighted least squares; 8.3e-9 as rounded), and
+// an odd k takes 1 - sin^2.  Error over 2^24 arguments N(0, 6) rms 1.85e-8,
+// largest 9.8e-8; the square of sinf 3.13e-8 and 1.29e-7.  A polynomial over
+// [-pi/2, pi/2] without e (3.7e-8, 2.5e-7) was 1 % of a decode faster.  Past
+// |t| = 8192 the library's.
 __device__ __forceinline__ float dec_sin2(float t) {
-    const float k = rintf(t * 0.318309886f);
-    float r = fmaf(-k, 3.14159274f, t);
-    r = fmaf(-k, -8.74227766e-8f, r);
+    const float k = rintf(t * 0.636619747f);
+    const float r1 = fmaf(-k, 1.57079637f, t);
+    const float r = fmaf(-k, -4.37113883e-8f, r1);
+    const float e = fmaf(-k, -1.71509942e-15f, fmaf(-k, -4.37113883e-8f, r1 - r));
     const float z = r * r;
-    float p = fmaf(z, 2.60575049e-6f, -1.980959e-4f);
-    p = fmaf(z, p, 8.33306648e-3f);
-    p = fmaf(z, p, -0.166666597f);
-    float s = fmaf(r * z, p, r);
-    if (!(fabsf(t) <= 8192.0f)) s = sinf(t);
-    return s * s;
+    float p = fmaf(z, -1.95149580e-4f, 8.33215844e-3f);
+    p = fmaf(z, p, -0.166666552f);
+    float s = r + fmaf(r * z, p, e);
+    s = (int)k & 1 ? fmaf(-s, s, 1.0f) : s * s;
+    if (!(fabsf(t) <= 8192.0f)) s = sinf(t), s *= s;
+    return s;
 }
 
 // A residual unit (src/decoder.rs:462-480) in one launch: out = x + conv2(
