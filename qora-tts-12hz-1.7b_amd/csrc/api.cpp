@@ -3169,7 +3169,6 @@ struct DecConvMfma {
 // k_dec_resunit takes the unit (ea1 null otherwise).
 struct DecResUnit {
     float *ea1 = nullptr, *eb1 = nullptr, *ea2 = nullptr, *eb2 = nullptr;
-    float ebmax = 0.0f;
 };
 
 struct qtts_decoder {
@@ -3435,9 +3434,11 @@ qtts_status dec_linear_mfma(qtts_decoder *d, const DecConvMfma &m, const float *
 // src/decoder.rs:430-444) on the matrix cores: output phase r
 // (out[q * stride + r], q < len) is a causal convolution of x with
 // J = kernel / stride taps reaching J - 1 steps back; the channels' phases
-// are the rows of one convolution.  omax (or null): receives max |out|.
+// are the rows of one convolution.  omax (or null): receives the bound of
+// DecConvMfmaParams::omax for the residual unit next.
 qtts_status dec_transposed_mfma(qtts_decoder *d, const qtts_conv_view &v, const DecConvMfma &m, const float *x,
-                                const unsigned *xmax, int len, float *c, unsigned *omax = nullptr) {
+                                const unsigned *xmax, int len, float *c, unsigned *omax = nullptr,
+                                const DecResUnit *next = nullptr) {
     DecConvMfmaParams p{};
     p.wh = m.wh;
     p.wl = m.wl;
@@ -3461,11 +3462,12 @@ qtts_status dec_transposed_mfma(qtts_decoder *d, const qtts_conv_view &v, const 
     p.out_stride = v.stride;
     p.up = v.stride;
     p.omax = omax;
+    if (omax) p.oea = next->ea1, p.oeb = next->eb1;
     const bool recorded = launch_dec_conv_mfma(d->ctx->stream, p);
     QTTS_TRY(check_launch(d->ctx, "k_dec_conv_mfma"));
     if (omax && !recorded) {
-        launch_dec_absmax(d->ctx->stream, c, (size_t)v.out_channels * v.stride * len, omax);
-        QTTS_TRY(check_launch(d->ctx, "k_dec_absmax"));
+        launch_dec_snake_bound(d->ctx->stream, c, next->ea1, next->eb1, v.out_channels, len * v.stride, omax);
+        QTTS_TRY(check_launch(d->ctx, "k_dec_snake_bound"));
     }
     return QTTS_OK;
 }
@@ -3662,31 +3664,36 @@ qtts_status dec_decode(qtts_decoder *d, const uint32_t *d_codes, int T, int ld, 
         launch_dec_snake(st, sig, b.pre_snake_alpha, b.pre_snake_beta, cin, L, t1, m0, pend, pend ? sig : nullptr);
         pend = nullptr;
         QTTS_TRY(check_launch(c, "k_dec_snake"));
-        unsigned *msig = nullptr;  // max |sig|, where a fused unit reads it
-        if (fuse && b.num_residuals > 0 && d->res_unit[bi][0].ea1) QTTS_TRY(own(&msig));
-        QTTS_TRY(dec_transposed_mfma(d, b.upsample, d->up_mfma[bi], t1, m0, L, nxt, msig));
+        // unit r, where it runs fused (null otherwise); msig: a bound on its first SnakeBeta
+        auto fused = [&](int r) -> const DecResUnit * {
+            return fuse && r < b.num_residuals && d->res_unit[bi][(size_t)r].ea1 ? &d->res_unit[bi][(size_t)r] : nullptr;
+        };
+        unsigned *msig = nullptr;
+        if (fused(0)) QTTS_TRY(own(&msig));
+        QTTS_TRY(dec_transposed_mfma(d, b.upsample, d->up_mfma[bi], t1, m0, L, nxt, msig, fused(0)));
         L *= b.upsample.stride;
         sig = nxt;
         float *t2 = other(sig, t1);
         for (int r = 0; r < b.num_residuals; r++) {
             const qtts_vocos_residual_view &rv = b.residuals[r];
             const std::array<DecConvMfma, 2> &mc = d->res_mfma[bi][(size_t)r];
-            const DecResUnit &ru = d->res_unit[bi][(size_t)r];
-            if (ru.ea1 && !pend && fuse) {
-                if (!msig) QTTS_TRY(maxof(sig, (size_t)cout * L, &msig));
+            if (msig) {  // fused
+                const DecResUnit &ru = d->res_unit[bi][(size_t)r], *next = fused(r + 1);
                 DecResUnitParams p{};
                 p.x = sig;
                 p.out = t1;
                 p.len = L;
                 p.dilation = rv.conv1.dilation;
                 p.xmax = msig;
-                p.omax = take();
-                if (!p.omax) return fail(c, QTTS_EDEVICE, "decoder: more matrix-core inputs than max slots");
+                if (next) {
+                    QTTS_TRY(own(&p.omax));
+                    p.oea = next->ea1;
+                    p.oeb = next->eb1;
+                }
                 p.ea1 = ru.ea1;
                 p.eb1 = ru.eb1;
                 p.ea2 = ru.ea2;
                 p.eb2 = ru.eb2;
-                p.ebmax = ru.ebmax;
                 p.w1h = mc[0].wh;
                 p.w1l = mc[0].wl;
                 p.ew1 = mc[0].ew;
@@ -3703,7 +3710,6 @@ qtts_status dec_decode(qtts_decoder *d, const uint32_t *d_codes, int T, int ld, 
                 std::swap(sig, t1);
                 continue;
             }
-            msig = nullptr;
             unsigned *m1 = take(), *m2 = take();
             if (!m1 || !m2) return fail(c, QTTS_EDEVICE, "decoder: more matrix-core inputs than max slots");
             launch_dec_snake(st, sig, rv.act1_alpha, rv.act1_beta, cout, L, t1, m1, pend, pend ? sig : nullptr);
@@ -3902,8 +3908,6 @@ qtts_status qtts_decoder_upload(qtts_ctx *c, const qtts_decoder_view *v, qtts_de
                     launch_dec_exp(c->stream, src[i], i & 1 ? -1.0f : 1.0f, ch, *dst[i]);
                     if ((s = check_launch(c, "k_dec_exp")) != QTTS_OK) return bail(s);
                 }
-                for (int i = 0; i < ch; i++)  // a few ulps over the device's exp
-                    ru.ebmax = std::max(ru.ebmax, std::exp(-R.act1_beta[i]) * 1.0001f);
             }
             d->res_unit[b].push_back(ru);
             d->amax_slots += 2;

@@ -398,6 +398,25 @@ __global__ __launch_bounds__(256) void k_dec_absmax(const float *x, size_t n, un
     }
 }
 
+// A bound on |v + eb sin(ea v)^2| that no sine is needed for, from sin(t)^2 <=
+// min(1, t^2).  NaN, which a maximum leaves out, for a v that is not finite,
+// whose SnakeBeta is NaN.
+__device__ __forceinline__ float dec_snake_bound(float v, float ea, float eb) {
+    const float t = ea * v;
+    return fmaf(v, 0.0f, fmaf(eb, fminf(1.0f, t * t), fabsf(v)));
+}
+
+// Its maximum over x [ch][len] into the slots of amax; block row y is channel y.
+__global__ __launch_bounds__(256) void k_dec_snake_bound(const float *x, const float *ea, const float *eb, int len,
+                                                         unsigned *amax) {
+    __shared__ float red[4];
+    const int c = blockIdx.y, stride = gridDim.x * blockDim.x;
+    const float a = ea[c], b = eb[c], *row = x + (size_t)c * len;
+    float m = 0.0f;
+    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < len; t += stride) m = fmaxf(m, dec_snake_bound(row[t], a, b));
+    block_amax(m, red, &amax[(blockIdx.y * gridDim.x + blockIdx.x) % kDecMaxSlots]);
+}
+
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -947,14 +966,24 @@ __global__ __launch_bounds__(64 * NW) void k_dec_conv_win_tw(DecConvMfmaParams P
                 v.y = ldexpf(acc[t][r + 1], sc) + b;
                 v.z = ldexpf(acc[t][r + 2], sc) + b;
                 v.w = ldexpf(acc[t][r + 3], sc) + b;
-                mx = fmaxf(fmaxf(mx, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+                if (P.omax) {  // uniform
+                    const float ea = P.oea[ch], eb = P.oeb[ch];
+                    mx = fmaxf(mx, fmaxf(dec_snake_bound(v.x, ea, eb), dec_snake_bound(v.y, ea, eb)));
+                    mx = fmaxf(mx, fmaxf(dec_snake_bound(v.z, ea, eb), dec_snake_bound(v.w, ea, eb)));
+                }
                 *reinterpret_cast<float4 *>(P.c + (long long)ch * P.ldc + (long long)n * P.out_stride +
                                             (m - ch * P.up)) = v;
                 continue;
             }
 #pragma unroll
-            for (int j = 0; j < 4; j++)
-                if (m + j < P.M) mx = fmaxf(mx, fabsf(dec_conv_out(P, m + j, n, ldexpf(acc[t][r + j], sc))));
+            for (int j = 0; j < 4; j++) {
+                if (m + j >= P.M) continue;
+                const float v = dec_conv_out(P, m + j, n, ldexpf(acc[t][r + j], sc));
+                if (P.omax) {  // uniform
+                    const int ch = dec_row_channel(P, m + j);
+                    mx = fmaxf(mx, dec_snake_bound(v, P.oea[ch], P.oeb[ch]));
+                }
+            }
         }
     }
     if (P.omax) {  // uniform
@@ -999,8 +1028,9 @@ __device__ __forceinline__ float dec_sin2(float t) {
 // 12 waves, wave w on channel tile w % CT and positions 64 (w / CT) ..: three
 // waves a SIMD, each A operand used for two 32-position tiles and shared
 // through L1 by the 12 / CT waves of its tile; A operands are loaded three
-// to four taps ahead.  conv1's operand scale bounds SnakeBeta by max |x| +
-// max exp(-beta), and max |out| is recorded for the next unit.
+// to four taps ahead.  conv1's operand scale is a bound on SnakeBeta (per
+// element, dec_snake_bound) that x's producer recorded, as this unit records
+// the next one's.
 // C = 96, 960,000 positions: 1130 us as five launches, 590 here; C = 192,
 // 320,000 positions: 1060, 650; C = 384, 80,000: 810, 565.  Matrix cores a third busy, vector ALU (the
 // sines and splits) a third, the rest latency: one block a CU.  Blocks of 6
@@ -1024,12 +1054,17 @@ __global__ __launch_bounds__(64 * NWV, 3) void k_dec_resunit(DecResUnitParams P)
     };
     __shared__ __align__(16) Lds sm;
     __shared__ float red[NWV];
+    __shared__ __align__(16) float next[2][C];  // oea, oeb: read in the epilogue, where nothing hides a load
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 31, half = lane >> 5;
+    if (P.omax && threadIdx.x < C) {
+        next[0][threadIdx.x] = P.oea[threadIdx.x];
+        next[1][threadIdx.x] = P.oeb[threadIdx.x];
+    }
     const int tile = wave % CT, p0 = 64 * (wave / CT);  // this wave's channels and positions of the block
     const int n0 = blockIdx.x * NP, len = P.len, dil = P.dilation;
     const int w0 = n0 - (TAPS - 1) * dil, W = NP + (TAPS - 1) * dil;
-    const int ex = split_exponent(wave_max(__uint_as_float(P.xmax[lane])) + P.ebmax);
+    const int ex = split_exponent(wave_max(__uint_as_float(P.xmax[lane])));
     const float xs = ldexpf(1.0f, ex);
 
     float v[PASSES][4];
@@ -1214,6 +1249,8 @@ __global__ __launch_bounds__(64 * NWV, 3) void k_dec_resunit(DecResUnitParams P)
         const int c = 32 * tile + 8 * j + 4 * half;
         const float4 b = *reinterpret_cast<const float4 *>(P.b2 + c);
         const float bv[4] = {b.x, b.y, b.z, b.w};
+        const float4 a = *reinterpret_cast<const float4 *>(&next[0][c]), e = *reinterpret_cast<const float4 *>(&next[1][c]);
+        const float av[4] = {a.x, a.y, a.z, a.w}, ev[4] = {e.x, e.y, e.z, e.w};
 #pragma unroll
         for (int t = 0; t < 2; t++) {
             const int n = n0 + p0 + 32 * t + col;
@@ -1221,13 +1258,14 @@ __global__ __launch_bounds__(64 * NWV, 3) void k_dec_resunit(DecResUnitParams P)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const float o = x[t][4 * j + i] + (ldexpf(acc[t][4 * j + i], sc2) + bv[i]);
-                m = fmaxf(m, fabsf(o));
+                m = fmaxf(m, dec_snake_bound(o, av[i], ev[i]));
                 P.out[(size_t)(c + i) * len + n] = o;
             }
         }
     }
+    if (!P.omax) return;
     m = wave_max(m);
-    if (lane == 0) red[wave] = m;  // last read two barriers ago
+    if (lane == 0) red[wave] = m;  // last read before the barrier ahead of conv2
     __syncthreads();
     if (threadIdx.x == 0) {
         for (int w = 1; w < NWV; w++) m = fmaxf(m, red[w]);
@@ -1301,6 +1339,13 @@ void launch_dec_snake(hipStream_t st, const float *x, const float *alpha, const 
     const unsigned per_row = std::max(1u, std::min<unsigned>(blocks_for(items, 256), kSnakeBlocks / (unsigned)ch));
     hipLaunchKernelGGL(k_dec_snake, dim3(per_row, (unsigned)ch), dim3(256), 0, st, x, alpha, beta, ch, len, out, amax,
                        add, sum);
+}
+
+void launch_dec_snake_bound(hipStream_t st, const float *x, const float *ea, const float *eb, int ch, int len,
+                            unsigned *amax) {
+    // at most 512 blocks where that leaves one per channel, as launch_dec_absmax
+    const unsigned per_row = std::max(1u, std::min<unsigned>(blocks_for((size_t)len, 1024), 512u / (unsigned)ch));
+    hipLaunchKernelGGL(k_dec_snake_bound, dim3(per_row, (unsigned)ch), dim3(256), 0, st, x, ea, eb, len, amax);
 }
 
 void launch_dec_fill_u32(hipStream_t st, unsigned *p, int n, unsigned v) {

@@ -128,7 +128,10 @@ struct DecConvMfmaParams {
     long long out_stride;
     int up;                   // >= 1
     const float *resid;       // DEC_EPI_RESID_IN: at the output's index (may be c)
-    unsigned *omax;           // null, or [kDecMaxSlots]: receives max |out| where the launch says so
+    // null, or [kDecMaxSlots], where the launch says so: receives a bound on max
+    // |out + oeb[c] sin(oea[c] out)^2|, the SnakeBeta that reads the output
+    unsigned *omax;
+    const float *oea, *oeb;   // [M / up]
     unsigned up_inv;          // set by the launch: 0 (up = 1) or the multiplier that divides by up
     bool quad;                // set by the launch: 4 rows are 4 neighbouring outputs, 16-byte aligned
 };
@@ -139,10 +142,10 @@ struct DecResUnitParams {
     const float *x;
     float *out;
     int len, dilation;
-    const unsigned *xmax;  // [kDecMaxSlots]: max |x|
-    unsigned *omax;        // [kDecMaxSlots]: receives max |out|
+    const unsigned *xmax;  // [kDecMaxSlots]: a bound on max |SnakeBeta(x)|
+    unsigned *omax;        // null, or [kDecMaxSlots]: receives the same of the unit that reads out,
+    const float *oea, *oeb;              // whose factors these are
     const float *ea1, *eb1, *ea2, *eb2;  // exp(alpha), exp(-beta) of both SnakeBetas
-    float ebmax;                         // at least max eb1
     const _Float16 *w1h, *w1l, *w2h, *w2l;
     int ew1, ew2, ksteps1, ksteps2;
     const float *b1, *b2;
@@ -380,7 +383,10 @@ void launch_dec_absmax(hipStream_t st, const float *x, size_t n, unsigned *amax)
 void launch_dec_conv_repack(hipStream_t st, const float *w, long long sm, long long sci, int k0, int kd, int M, int cin,
                             int taps, int cin16, int mtiles, int ksteps, int ew, int up, _Float16 *wh,
                             _Float16 *wl);
-bool launch_dec_conv_mfma(hipStream_t st, DecConvMfmaParams p);  // true: max |out| is in p.omax
+bool launch_dec_conv_mfma(hipStream_t st, DecConvMfmaParams p);  // true: p.omax is recorded
+// the bound of DecConvMfmaParams::omax for x [ch][len]
+void launch_dec_snake_bound(hipStream_t st, const float *x, const float *ea, const float *eb, int ch, int len,
+                            unsigned *amax);
 // Whether k_dec_resunit takes a residual unit of these shapes.
 bool dec_resunit_fits(int channels, int ksize1, int dilation, int ksize2);
 void launch_dec_resunit(hipStream_t st, const DecResUnitParams &p, int channels);
