@@ -377,6 +377,21 @@ GemmTilePlan tile_plan(int M, int K, int N) {
     return best;
 }
 
+// 65 to 96 rows of a wide weight take 64 rows and then the rest: where the
+// 64-row product has K whole in a block and 256 to 512 panels to spread, a row
+// block's 192 to 256 blocks of four panels leave its weights' loads alone on a
+// CU.  Row blocks / two passes / two passes before k_gemm_mfma16 and the ring,
+// 65 rows (96): 2048 -> 12288 42.4 / 31.6 / 38.4 us (42.7 / 34.7 / 40.5), 2048
+// -> 16384 49.9 / 36.2 / 48.1 (50.5 / 39.2 / 52.2), 1024 -> 8192 20.9 / 17.6 /
+// 21.6 (21.1 / 18.7 / 22.8); outside it 2048 -> 32768 57.7 / 63.7 / 91.4, 2048
+// -> 6144 22.9 / 23.5 / 27.0, 768 -> 12288 20.5 / 20.7 / 25.3, 3072 -> 12288
+// 50.1 / 46.5 / 57.6 (51.0 / 53.3 / 61.1).
+bool two_passes(int M, int K, int N) {
+    int steps, kc;
+    mfma_plan(K, N, &steps, &kc);
+    return M > kMfmaPassRows && M <= 96 && K >= 1024 && kc == 1 && N / 32 >= 256 && N / 32 <= 512;
+}
+
 size_t tile_part_floats(const GemmTilePlan &t) {
     return t.kc > 1 ? (size_t)t.mb * t.nb * t.kc * (size_t)(t.nw * t.mt * 1024) : 0;
 }
@@ -483,7 +498,7 @@ qtts_status mfma_reserve(qtts_ctx *c, const DevQ4Mfma &w) {
 // (csrc/mfma.hip), f the row prologue (MfmaRowsMode): the prologue and
 // binary16 split, then the product.  Up to kMfmaPassRows rows: one block per
 // (panel, K chunk), and the last block of a panel sums its chunks.  More
-// rows: row blocks by tile_plan.
+// rows: row blocks by tile_plan, or two such passes.
 qtts_status run_gemm_mfma(qtts_ctx *c, const DevQ4Mfma &w, const float *x, int M, int ldx, int mode,
                           const uint16_t *gamma, float *y, int ldy, const float *bias, bool accumulate,
                           float *norm_out = nullptr, int ldn = 0, bool full = false) {
@@ -492,8 +507,9 @@ qtts_status run_gemm_mfma(qtts_ctx *c, const DevQ4Mfma &w, const float *x, int M
         return fail(c, QTTS_ESHAPE, "MFMA GEMM: unsupported shape or unaligned rows");
     if (panels > kCounters) return fail(c, QTTS_ESHAPE, "MFMA GEMM: more panels than counters");
     QTTS_TRY(mfma_reserve(c, w));
-    for (int r0 = 0; r0 < M; r0 += kTileMaxRows) {
-        const int Mc = M - r0 < kTileMaxRows ? M - r0 : kTileMaxRows;
+    for (int r0 = 0, Mc = 0; r0 < M; r0 += Mc) {
+        Mc = M - r0 < kTileMaxRows ? M - r0 : kTileMaxRows;
+        if (two_passes(Mc, K, N)) Mc = kMfmaPassRows;
         const bool tiled = Mc > kMfmaPassRows, m16 = Mc <= kMfma16Rows;
         GemmTilePlan t{};
         int sw = 0, kc = 0;

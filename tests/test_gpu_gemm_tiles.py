@@ -2,8 +2,11 @@
 edges of its tiles: one row past a pass, rows off the 32- and 128-row tiles,
 an odd number of 16-row K steps, panel counts off a block's 4 or 8, one and
 several K chunks; and the scale split's last accepted scales."""
+import time
+
 import numpy as np
 import pytest
+import torch
 
 import qtts
 
@@ -19,7 +22,8 @@ def _bound(x, w, K):
 
 @pytest.mark.parametrize("rows,K,N", [(8, 16, 32), (9, 48, 96), (15, 272, 1056), (16, 1040, 2048), (13, 2064, 64),
                                       (16, 6144, 2048), (17, 1040, 96), (65, 1040, 160), (96, 2048, 2048), (97, 16, 32), (128, 48, 288), (129, 6144, 96),
-                                      (300, 1024, 1056), (1000, 272, 2048), (1064, 2048, 4096), (4097, 32, 64)])
+                                      (300, 1024, 1056), (1000, 272, 2048), (1064, 2048, 4096), (4097, 32, 64),
+                                      (65, 2048, 8192), (80, 1040, 16384), (96, 1024, 8224)])
 def test_gemm_row_blocks(ctx, rows, K, N):
     w = qtts.Q4Weight.synthetic(21, f"tiles.{K}.{N}", K, N)
     x = qtts.synth_normal_f32(21, f"tiles.x.{rows}.{K}", rows * K).reshape(rows, K)
@@ -46,3 +50,30 @@ def test_gemm_scale_split_is_exact(ctx, rows, scale):
     x[np.arange(rows), np.arange(rows) * 7 % K] = 1.0
     y = qtts.DeviceQ4(ctx, w).gemm(x, rows).reshape(rows, N)
     assert np.array_equal(y, w.dequantize()[np.arange(rows) * 7 % K])
+
+
+@pytest.mark.parametrize("rows", [65, 96])
+def test_rows_past_a_pass_cost_no_more_than_two(ctx, rows):
+    """Wide weights, read from memory: one call of 65 to 96 rows against one of
+    64 and one of 32 (row blocks took 1.2 times as long)."""
+    K, N = 2048, 12288
+    ws = [qtts.DeviceQ4(ctx, qtts.Q4Weight.synthetic(23, f"wide.{i}", K, N)) for i in range(8)]
+    x = torch.from_numpy(qtts.synth_normal_f32(23, "wide.x", rows * K)).cuda()
+    y = torch.empty(rows * N, device="cuda")
+    torch.cuda.synchronize()
+
+    def best(parts):
+        times = []
+        for _ in range(12):
+            t0 = time.perf_counter()
+            for _ in range(4):
+                for w in ws:
+                    for m in parts:
+                        w.gemm_device(x.data_ptr(), m, y.data_ptr())
+            ctx.synchronize()
+            times.append(time.perf_counter() - t0)
+        return min(times)
+
+    one, two = best([rows]), best([64, 32])
+    print(f"{rows} rows: {one / 32 * 1e6:.1f} us, in two calls {two / 32 * 1e6:.1f}")
+    assert one < 1.08 * two
