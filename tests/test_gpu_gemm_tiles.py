@@ -1,7 +1,7 @@
-"""The Q4 product of 8 to 16 rows and in row blocks (more than 64 rows) against float64, at the
-edges of its tiles: one row past a pass, rows off the 32- and 128-row tiles,
-an odd number of 16-row K steps, panel counts off a block's 4 or 8, one and
-several K chunks; and the scale split's last accepted scales."""
+"""The Q4 product of 8 and more rows against float64, on every kernel variant and
+at the edges of its tiles: one row past a pass, rows off the 16-, 32- and
+128-row tiles, an odd number of 16-row K steps, panel counts off a block's 4 or
+8, one and several K chunks; and the scale split's last accepted scales."""
 import time
 
 import numpy as np
@@ -20,10 +20,28 @@ def _bound(x, w, K):
     return (2.0 ** -19 + (3 * K / 16 + 32) * 2.0 ** -24) * (np.abs(x.astype(np.float64)) @ np.abs(w))
 
 
-@pytest.mark.parametrize("rows,K,N", [(8, 16, 32), (9, 48, 96), (15, 272, 1056), (16, 1040, 2048), (13, 2064, 64),
-                                      (16, 6144, 2048), (17, 1040, 96), (65, 1040, 160), (96, 2048, 2048), (97, 16, 32), (128, 48, 288), (129, 6144, 96),
-                                      (300, 1024, 1056), (1000, 272, 2048), (1064, 2048, 4096), (4097, 32, 64),
-                                      (65, 2048, 8192), (80, 1040, 16384), (96, 1024, 8224)])
+# tests/test_gemm_plans.py holds these to every kernel variant that a product
+# can take, with one chunk of K and with several.
+SHAPES = [
+    # up to 16 rows
+    (8, 16, 32), (9, 48, 96), (15, 272, 1056), (16, 1040, 2048), (13, 2064, 64), (16, 6144, 2048), (12, 512, 64),
+    (11, 144, 96), (10, 1024, 96),
+    # 17 to 64: one and two 32-row tiles, 1 to 16 steps a wave
+    (17, 1040, 96), (18, 2048, 2048), (31, 2048, 4096), (32, 16, 6144), (33, 6144, 2048), (40, 272, 96), (48, 1040, 12288),
+    (20, 1040, 12288), (24, 6144, 2048), (63, 2048, 2048), (64, 2064, 4096), (50, 48, 6176),
+    (30, 144, 96), (55, 256, 64), (48, 2048, 4096), (20, 272, 64), (20, 1024, 64), (40, 1024, 64),
+    # more, in row blocks: 1 to 4 tiles of 4 panels
+    (65, 1040, 160), (96, 2048, 2048), (97, 16, 32), (128, 48, 288), (129, 6144, 96), (300, 1024, 1056),
+    (1000, 272, 2048), (1064, 2048, 4096), (4097, 32, 64), (1064, 2048, 2048), (500, 2048, 6144), (1000, 1024, 6176),
+    (160, 6144, 2048), (400, 272, 6176), (70, 2048, 4096), (200, 272, 12288), (1000, 3072, 1056),
+    # 4 tiles of 8 panels, whole and with a part of a block past the last panel
+    (1064, 2048, 12288), (1000, 6144, 2048), (1030, 2064, 12320), (200, 6144, 4128),
+    # two passes
+    (65, 2048, 8192), (80, 1040, 16384), (96, 1024, 8224),
+]
+
+
+@pytest.mark.parametrize("rows,K,N", SHAPES)
 def test_gemm_row_blocks(ctx, rows, K, N):
     w = qtts.Q4Weight.synthetic(21, f"tiles.{K}.{N}", K, N)
     x = qtts.synth_normal_f32(21, f"tiles.x.{rows}.{K}", rows * K).reshape(rows, K)
