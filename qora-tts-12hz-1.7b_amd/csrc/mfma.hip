@@ -85,14 +85,13 @@ __global__ void k_repack_mfma(DevQ4 w, uint32_t *wm, uint16_t *sa, uint16_t *sb,
 // 6144: 1024 threads a row).
 template <int NT, bool M16>  // threads (K <= 8 * NT); the 16-row operand order
 __global__ __launch_bounds__(NT) void k_mfma_rows(MfmaRowsParams P) {
-    constexpr int G = 1;  // 8-value groups per thread
     __shared__ float red[2][NT / 64];
     // Blocks of one XCD (every 8th) take neighbouring rows (Mpad is a multiple
     // of 16): 8 rows' 16-byte slots make up each 128-byte line of xh and xl,
     // which then leaves one L2 whole (1000 rows of 6144: 23.3 -> 15.0 us).
     const int m = (int)((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3));
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int K = P.K, Ks = K / 16, ng = K / 8;
+    const int K = P.K, Ks = K / 16, ng = K / 8, g = tid;
     // 8-value group g = k / 8 of row m goes to the A-operand slot of lane
     // (m % 32) + 32 (g % 2) in step g / 2 of M-tile m / 32, or (16-row
     // operands) of lane m + 16 (g % 4) in 32-row step g / 4
@@ -101,59 +100,52 @@ __global__ __launch_bounds__(NT) void k_mfma_rows(MfmaRowsParams P) {
         return (tile + (M16 ? (size_t)(g >> 2) * 64 + 16 * (g & 3) : (size_t)(g >> 1) * 64 + 32 * (g & 1))) * 8;
     };
     if (m >= P.M) {
-        for (int g = tid; g < ng; g += NT) {
-            const size_t o = slot(g);
-            *reinterpret_cast<half8 *>(P.xh + o) = (half8){};
-            *reinterpret_cast<half8 *>(P.xl + o) = (half8){};
+        if (g < ng) {
+            *reinterpret_cast<half8 *>(P.xh + slot(g)) = (half8){};
+            *reinterpret_cast<half8 *>(P.xl + slot(g)) = (half8){};
         }
         if (tid == 0) P.rexp[m] = 0;
         return;
     }
     const float *src = P.x + (size_t)m * P.ldx;
     const bool norm = P.mode == MFMA_ROWS_RMSNORM;
-    float v[G][8];
-    uint32_t gw[G][4];
+    float v[8];
+    uint32_t gw[4];
     // 1. the row's values and gammas (all loads first); the sum of squares
     //    and max|x * gamma| (RMSNorm) or max|v|
-#pragma unroll
-    for (int j = 0; j < G; j++) {
-        const int g = tid + NT * j;
-        if (g < ng) {
-            const float4 a = *reinterpret_cast<const float4 *>(src + 8 * g);
-            const float4 b = *reinterpret_cast<const float4 *>(src + 8 * g + 4);
-            v[j][0] = a.x, v[j][1] = a.y, v[j][2] = a.z, v[j][3] = a.w;
-            v[j][4] = b.x, v[j][5] = b.y, v[j][6] = b.z, v[j][7] = b.w;
-            if (norm) {
-                const uint4 q = *reinterpret_cast<const uint4 *>(P.gamma + 8 * g);
-                gw[j][0] = q.x, gw[j][1] = q.y, gw[j][2] = q.z, gw[j][3] = q.w;
-            }
-            if (P.mode == MFMA_ROWS_SILU) {
-#pragma unroll
-                for (int i = 0; i < 8; i++) v[j][i] = v[j][i] / (1.0f + expf(-v[j][i]));
-            }
-            if (P.mode == MFMA_ROWS_SWIGLU) {
-                const float4 c = *reinterpret_cast<const float4 *>(src + K + 8 * g);
-                const float4 d = *reinterpret_cast<const float4 *>(src + K + 8 * g + 4);
-                const float u[8] = {c.x, c.y, c.z, c.w, d.x, d.y, d.z, d.w};
-#pragma unroll
-                for (int i = 0; i < 8; i++) v[j][i] = (v[j][i] / (1.0f + expf(-v[j][i]))) * u[i];
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; i++) v[j][i] = 0.0f;
-#pragma unroll
-            for (int q = 0; q < 4; q++) gw[j][q] = 0u;
+    if (g < ng) {
+        const float4 a = *reinterpret_cast<const float4 *>(src + 8 * g);
+        const float4 b = *reinterpret_cast<const float4 *>(src + 8 * g + 4);
+        v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w;
+        v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+        if (norm) {
+            const uint4 q = *reinterpret_cast<const uint4 *>(P.gamma + 8 * g);
+            gw[0] = q.x, gw[1] = q.y, gw[2] = q.z, gw[3] = q.w;
         }
+        if (P.mode == MFMA_ROWS_SILU) {
+#pragma unroll
+            for (int i = 0; i < 8; i++) v[i] = v[i] / (1.0f + expf(-v[i]));
+        }
+        if (P.mode == MFMA_ROWS_SWIGLU) {
+            const float4 c = *reinterpret_cast<const float4 *>(src + K + 8 * g);
+            const float4 d = *reinterpret_cast<const float4 *>(src + K + 8 * g + 4);
+            const float u[8] = {c.x, c.y, c.z, c.w, d.x, d.y, d.z, d.w};
+#pragma unroll
+            for (int i = 0; i < 8; i++) v[i] = (v[i] / (1.0f + expf(-v[i]))) * u[i];
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 4; q++) gw[q] = 0u;
     }
     float ss = 0.0f, mx = 0.0f;
 #pragma unroll
-    for (int j = 0; j < G; j++)
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            ss += v[j][i] * v[j][i];
-            // NaN entries drop out of the max here and stay NaN below
-            mx = fmaxf(mx, fabsf(norm ? v[j][i] * f16_to_f32((uint16_t)(gw[j][i / 2] >> (16 * (i & 1)))) : v[j][i]));
-        }
+    for (int i = 0; i < 8; i++) {
+        ss += v[i] * v[i];
+        // NaN entries drop out of the max here and stay NaN below
+        mx = fmaxf(mx, fabsf(norm ? v[i] * f16_to_f32((uint16_t)(gw[i / 2] >> (16 * (i & 1)))) : v[i]));
+    }
     ss = wave_sum(ss);
     mx = wave_max(mx);
     if (lane == 0) {
@@ -171,9 +163,7 @@ __global__ __launch_bounds__(NT) void k_mfma_rows(MfmaRowsParams P) {
         const float inv = 1.0f / sqrtf(ss / (float)K + 1e-6f);
         mx *= inv;
 #pragma unroll
-        for (int j = 0; j < G; j++)
-#pragma unroll
-            for (int i = 0; i < 8; i++) v[j][i] = v[j][i] * inv * f16_to_f32((uint16_t)(gw[j][i / 2] >> (16 * (i & 1))));
+        for (int i = 0; i < 8; i++) v[i] = v[i] * inv * f16_to_f32((uint16_t)(gw[i / 2] >> (16 * (i & 1))));
     }
     // 2. the row exponent
     int e = 0;
@@ -183,36 +173,26 @@ __global__ __launch_bounds__(NT) void k_mfma_rows(MfmaRowsParams P) {
         e = min((norm ? 14 : 15) - E, 126);
     }
     if (tid == 0) P.rexp[m] = e;
-    if (P.norm_out) {
+    if (P.norm_out && g < ng) {
+        float *dst = P.norm_out + (size_t)m * P.ldn + 8 * g;
 #pragma unroll
-        for (int j = 0; j < G; j++) {
-            const int g = tid + NT * j;
-            if (g >= ng) continue;
-            float *dst = P.norm_out + (size_t)m * P.ldn + 8 * g;
-#pragma unroll
-            for (int i = 0; i < 8; i++) dst[i] = v[j][i];
-        }
+        for (int i = 0; i < 8; i++) dst[i] = v[i];
     }
     // 3. the binary16 hi + lo split
     if (M16 && ng + tid < (ng + 3) / 4 * 4) {  // the last 32-row step's rows past K
         *reinterpret_cast<half8 *>(P.xh + slot(ng + tid)) = (half8){};
         *reinterpret_cast<half8 *>(P.xl + slot(ng + tid)) = (half8){};
     }
+    if (g >= ng) return;
+    half8 h, l;
 #pragma unroll
-    for (int j = 0; j < G; j++) {
-        const int g = tid + NT * j;
-        if (g >= ng) continue;
-        half8 h, l;
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const float s = ldexpf(v[j][i], e);
-            h[i] = (_Float16)s;
-            l[i] = (_Float16)(s - (float)h[i]);
-        }
-        const size_t o = slot(g);
-        *reinterpret_cast<half8 *>(P.xh + o) = h;
-        *reinterpret_cast<half8 *>(P.xl + o) = l;
+    for (int i = 0; i < 8; i++) {
+        const float s = ldexpf(v[i], e);
+        h[i] = (_Float16)s;
+        l[i] = (_Float16)(s - (float)h[i]);
     }
+    *reinterpret_cast<half8 *>(P.xh + slot(g)) = h;
+    *reinterpret_cast<half8 *>(P.xl + slot(g)) = l;
 }
 
 // One 32-column panel x one K chunk per block: 8 waves of `steps` 16-row
