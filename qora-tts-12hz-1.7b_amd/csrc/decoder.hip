@@ -398,13 +398,16 @@ __global__ __launch_bounds__(256) void k_dec_absmax(const float *x, size_t n, un
     }
 }
 
-// A bound on |v + eb sin(ea v)^2| that no sine is needed for, from sin(t)^2 <=
-// min(1, t^2).  NaN, which a maximum leaves out, for a v that is not finite,
-// whose SnakeBeta is NaN.
-__device__ __forceinline__ float dec_snake_bound(float v, float ea, float eb) {
-    const float t = ea * v;
-    return fmaf(v, 0.0f, fmaf(eb, fminf(1.0f, t * t), fabsf(v)));
+// A bound on |v + eb sin(ea v)^2| over |v| <= m that no sine is needed for,
+// from sin(t)^2 <= min(1, t^2).
+__device__ __forceinline__ float dec_snake_bound(float m, float ea, float eb) {
+    const float t = ea * m;
+    return fmaf(eb, fminf(1.0f, t * t), m);
 }
+
+// |v|, or for a v that is not finite, whose SnakeBeta is NaN, NaN: a maximum
+// leaves it out.
+__device__ __forceinline__ float finite_abs(float v) { return fmaf(v, 0.0f, fabsf(v)); }
 
 // Its maximum over x [ch][len] into the slots of amax; block row y is channel y.
 __global__ __launch_bounds__(256) void k_dec_snake_bound(const float *x, const float *ea, const float *eb, int len,
@@ -413,8 +416,8 @@ __global__ __launch_bounds__(256) void k_dec_snake_bound(const float *x, const f
     const int c = blockIdx.y, stride = gridDim.x * blockDim.x;
     const float a = ea[c], b = eb[c], *row = x + (size_t)c * len;
     float m = 0.0f;
-    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < len; t += stride) m = fmaxf(m, dec_snake_bound(row[t], a, b));
-    block_amax(m, red, &amax[(blockIdx.y * gridDim.x + blockIdx.x) % kDecMaxSlots]);
+    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < len; t += stride) m = fmaxf(m, finite_abs(row[t]));
+    block_amax(fmaxf(0.0f, dec_snake_bound(m, a, b)), red, &amax[(blockIdx.y * gridDim.x + blockIdx.x) % kDecMaxSlots]);
 }
 
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
@@ -852,7 +855,10 @@ __global__ __launch_bounds__(256) void k_dec_conv_win(DecConvMfmaParams P) {
 // channel.  As one launch row per phase (k_dec_conv_mfma, each gathering the
 // input and writing every stride-th float) 768 -> 384 channels by 5 to
 // 80,000 positions took 437 us, 384 -> 192 by 4 to 320,000 563, 192 -> 96 by
-// 3 to 960,000 601 and 67 more for max |out|; here 424, 375 and 486.
+// 3 to 960,000 601 and 67 more for max |out|; here 424, 375 and 486 to 516,
+// and 548 with the next unit's bound taken per channel (604 per element, whose
+// two factors were then loaded for each; 16 maxima kept over the position
+// tiles cost a wave a SIMD, 820).
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void k_dec_conv_win_tw(DecConvMfmaParams P) {
     static_assert(kDecMaxSlots == 64, "one max slot per lane");
@@ -951,39 +957,42 @@ __global__ __launch_bounds__(64 * NW) void k_dec_conv_win_tw(DecConvMfmaParams P
     const int sc = -(ex + P.ew);
     float mx = 0.0f;
 #pragma unroll
-    for (int t = 0; t < PT; t++) {
-        const int n = n0 + t * 32 + col;
-        if (n >= len) continue;
+    for (int r = 0; r < 16; r += 4) {
+        const int m = 32 * tile + (r >> 2) * 8 + half * 4;
+        if (P.quad) {  // 4 phases of one channel: one 16-byte store
+            if (m >= P.M) continue;
+            const int ch = dec_row_channel(P, m);
+            const float b = P.bias ? P.bias[ch] : 0.0f;
+            const float ea = P.omax ? P.oea[ch] : 0.0f, eb = P.omax ? P.oeb[ch] : 0.0f;
+            float cm = 0.0f;  // the channel's largest |out|
 #pragma unroll
-        for (int r = 0; r < 16; r += 4) {
-            const int m = 32 * tile + (r >> 2) * 8 + half * 4;
-            if (P.quad) {  // 4 phases of one channel: one 16-byte store
-                if (m >= P.M) continue;
-                const int ch = dec_row_channel(P, m);
-                const float b = P.bias ? P.bias[ch] : 0.0f;
+            for (int t = 0; t < PT; t++) {
+                const int n = n0 + t * 32 + col;
+                if (n >= len) continue;
                 float4 v;
                 v.x = ldexpf(acc[t][r], sc) + b;
                 v.y = ldexpf(acc[t][r + 1], sc) + b;
                 v.z = ldexpf(acc[t][r + 2], sc) + b;
                 v.w = ldexpf(acc[t][r + 3], sc) + b;
-                if (P.omax) {  // uniform
-                    const float ea = P.oea[ch], eb = P.oeb[ch];
-                    mx = fmaxf(mx, fmaxf(dec_snake_bound(v.x, ea, eb), dec_snake_bound(v.y, ea, eb)));
-                    mx = fmaxf(mx, fmaxf(dec_snake_bound(v.z, ea, eb), dec_snake_bound(v.w, ea, eb)));
-                }
+                cm = fmaxf(cm, fmaxf(fmaxf(finite_abs(v.x), finite_abs(v.y)), fmaxf(finite_abs(v.z), finite_abs(v.w))));
                 *reinterpret_cast<float4 *>(P.c + (long long)ch * P.ldc + (long long)n * P.out_stride +
                                             (m - ch * P.up)) = v;
-                continue;
             }
+            mx = fmaxf(mx, dec_snake_bound(cm, ea, eb));
+            continue;
+        }
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                if (m + j >= P.M) continue;
-                const float v = dec_conv_out(P, m + j, n, ldexpf(acc[t][r + j], sc));
-                if (P.omax) {  // uniform
-                    const int ch = dec_row_channel(P, m + j);
-                    mx = fmaxf(mx, dec_snake_bound(v, P.oea[ch], P.oeb[ch]));
-                }
+        for (int j = 0; j < 4; j++) {
+            if (m + j >= P.M) continue;
+            const int ch = P.omax ? dec_row_channel(P, m + j) : 0;
+            const float ea = P.omax ? P.oea[ch] : 0.0f, eb = P.omax ? P.oeb[ch] : 0.0f;
+            float cm = 0.0f;
+#pragma unroll
+            for (int t = 0; t < PT; t++) {
+                const int n = n0 + t * 32 + col;
+                if (n < len) cm = fmaxf(cm, finite_abs(dec_conv_out(P, m + j, n, ldexpf(acc[t][r + j], sc))));
             }
+            mx = fmaxf(mx, dec_snake_bound(cm, ea, eb));
         }
     }
     if (P.omax) {  // uniform
@@ -1031,11 +1040,13 @@ __device__ __forceinline__ float dec_sin2(float t) {
 // to four taps ahead.  conv1's operand scale is a bound on SnakeBeta (per
 // element, dec_snake_bound) that x's producer recorded, as this unit records
 // the next one's.
-// C = 96, 960,000 positions: 1130 us as five launches, 590 here; C = 192,
-// 320,000 positions: 1060, 650; C = 384, 80,000: 810, 565.  Matrix cores a third busy, vector ALU (the
-// sines and splits) a third, the rest latency: one block a CU.  Blocks of 6
-// waves and half the positions measured slower (C = 96, 805 us: twice the A
-// operands through the L2).
+// C = 96, 960,000 positions: 1130 us as five launches, 607 to 636 here; C =
+// 192, 320,000 positions: 1060, 667 to 705; C = 384, 80,000: 810, 564 to 586.
+// Matrix cores a third busy, vector ALU (the sines and splits) a third, the
+// rest latency: one block a CU, and of the 168 registers that 12 waves leave
+// 3, 7 and 10 spill (96, 192 and 384 channels).  Blocks of 6 waves and half the
+// positions measured slower (C = 96, 805 us: twice the A operands through the
+// L2).
 template <int CT, int NWV>
 __global__ __launch_bounds__(64 * NWV, 3) void k_dec_resunit(DecResUnitParams P) {
     static_assert(kDecMaxSlots == 64, "one max slot per lane");
@@ -1251,6 +1262,7 @@ __global__ __launch_bounds__(64 * NWV, 3) void k_dec_resunit(DecResUnitParams P)
         const float bv[4] = {b.x, b.y, b.z, b.w};
         const float4 a = *reinterpret_cast<const float4 *>(&next[0][c]), e = *reinterpret_cast<const float4 *>(&next[1][c]);
         const float av[4] = {a.x, a.y, a.z, a.w}, ev[4] = {e.x, e.y, e.z, e.w};
+        float cm[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // the channels' largest |out|
 #pragma unroll
         for (int t = 0; t < 2; t++) {
             const int n = n0 + p0 + 32 * t + col;
@@ -1258,10 +1270,12 @@ __global__ __launch_bounds__(64 * NWV, 3) void k_dec_resunit(DecResUnitParams P)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const float o = x[t][4 * j + i] + (ldexpf(acc[t][4 * j + i], sc2) + bv[i]);
-                m = fmaxf(m, dec_snake_bound(o, av[i], ev[i]));
+                cm[i] = fmaxf(cm[i], finite_abs(o));
                 P.out[(size_t)(c + i) * len + n] = o;
             }
         }
+#pragma unroll
+        for (int i = 0; i < 4; i++) m = fmaxf(m, dec_snake_bound(cm[i], av[i], ev[i]));
     }
     if (!P.omax) return;
     m = wave_max(m);
