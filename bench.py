@@ -389,7 +389,7 @@ def decoder_measure(ctx, frames, cpu_frames=2, reps=3):
                      "unit": "TFLOP/s", "frac": round(achieved / MFMA_F16_PEAK_TFLOPS, 4), "algorithmic_flops": flops,
                      "issued_f16_TFLOPs": round(3 * achieved, 1),
                      "frac_of_f32_peak": round(achieved / FP32_PEAK_TFLOPS, 4),
-                     "kernel": "whole decode (k_dec_conv_mfma dominant: every projection and convolution as "
+                     "kernel": "whole decode (k_dec_resunit dominant: every projection and convolution as "
                                "three binary16 MFMAs per f32 product term)"},
     }
     if cpu_frames:

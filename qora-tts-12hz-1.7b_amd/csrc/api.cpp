@@ -100,12 +100,19 @@ void ctx_release(qtts_ctx *c) {
 
 }  // namespace
 
+// A weight's operand copy and its product's scratch at any number of rows
+// (binary16 values, floats).  The sizes stay out of the kernels' arguments:
+// with them 16 streams measured 1.2 to 2 % slower.
+struct Q4Mfma : DevQ4Mfma {
+    size_t scratch_x = 0, scratch_part = 0;
+};
+
 struct qtts_q4 {
     qtts_ctx *ctx = nullptr;
     DevQ4 d{};
     void *mem = nullptr;
     size_t bytes = 0;
-    DevQ4Mfma m{};  // MFMA operand copy, made by the first GEMM of >= 8 rows
+    Q4Mfma m{};  // MFMA operand copy, made by the first GEMM of >= 8 rows
     void *mfma_mem = nullptr;
     int mfma_state = 0;  // 0 not tried, 1 made, -1 the weight stays on the VALU path
 };
@@ -344,9 +351,9 @@ constexpr int kTileMaxRows = 4096;
 // per 32-row K stage: `alone`, one block on a CU (issue and latency), and
 // `loaded`, each block of a CU that has several (operand reads through the
 // L2).  A block of 4 x 8 reads the rows half as often as 4 x 4: 1064 rows,
-// 2048 -> 12288, 180 against 192 us.  Few row and column blocks take K
-// chunks, each a partial written and read once: 1000 rows, 6144 -> 2048,
-// 161 us with one chunk, 113 with four.
+// 2048 -> 12288, 159 against 174 us with the row split.  Few row and column
+// blocks take K chunks, each a partial written and read once: 1000 rows,
+// 6144 -> 2048, 203 us with one chunk, 120 with two, 89 with four.
 GemmTilePlan tile_plan(int M, int K, int N) {
     struct Shape {
         int mt, nw;
@@ -441,7 +448,7 @@ void mfma_scratch(int K, int N, size_t *x, size_t *part) {
 // *ok is false (and *mem null) for a weight the matrix-core path cannot take
 // exactly: a shape off the 16 x 32 grid, K above the row prologue's limit,
 // or a scale above 8188 in magnitude.  Synchronises the stream.
-qtts_status make_mfma_copy(qtts_ctx *c, const DevQ4 &w, void **mem, DevQ4Mfma *m, bool *ok) {
+qtts_status make_mfma_copy(qtts_ctx *c, const DevQ4 &w, void **mem, Q4Mfma *m, bool *ok) {
     *mem = nullptr;
     *ok = false;
     if (w.K % 16 != 0 || w.N % 32 != 0 || w.K > kMfmaRowsMaxK) return QTTS_OK;
@@ -489,7 +496,7 @@ qtts_status grow_kept(qtts_ctx *c, T **buf, size_t *cap, size_t need) {
     return QTTS_OK;
 }
 
-qtts_status mfma_reserve(qtts_ctx *c, const DevQ4Mfma &w) {
+qtts_status mfma_reserve(qtts_ctx *c, const Q4Mfma &w) {
     QTTS_TRY(grow_kept(c, &c->mfma_x, &c->mfma_x_cap, w.scratch_x));
     return grow_kept(c, &c->mfma_part, &c->mfma_part_cap, w.scratch_part);
 }
@@ -499,7 +506,7 @@ qtts_status mfma_reserve(qtts_ctx *c, const DevQ4Mfma &w) {
 // binary16 split, then the product.  Up to kMfmaPassRows rows: one block per
 // (panel, K chunk), and the last block of a panel sums its chunks.  More
 // rows: row blocks by tile_plan, or two such passes.
-qtts_status run_gemm_mfma(qtts_ctx *c, const DevQ4Mfma &w, const float *x, int M, int ldx, int mode,
+qtts_status run_gemm_mfma(qtts_ctx *c, const Q4Mfma &w, const float *x, int M, int ldx, int mode,
                           const uint16_t *gamma, float *y, int ldy, const float *bias, bool accumulate,
                           float *norm_out = nullptr, int ldn = 0, bool full = false) {
     const int K = w.K, N = w.N, panels = N / 32;
@@ -798,9 +805,9 @@ struct qtts_talker {
     std::vector<void *> prefill_bufs;
     // MFMA operand copies of the layer weights (qkv, o, gu, down per layer),
     // made by the first prefill of >= kMfmaMinRows rows
-    std::vector<DevQ4Mfma> mfma;
+    std::vector<Q4Mfma> mfma;
     int mfma_state = 0;  // 0 not tried, 1 made, -1 some weight cannot use the matrix cores
-    DevQ4Mfma head_mfma{};  // codec head, for the batched loop
+    Q4Mfma head_mfma{};  // codec head, for the batched loop
     int head_mfma_state = 0;
     // loop buffers
     uint32_t *codes = nullptr;
@@ -813,7 +820,7 @@ struct qtts_talker {
     DevQ4 text_emb{}, fc1{}, fc2{};
     float *fc1_b = nullptr, *fc2_b = nullptr;
     int text_hidden = 0, has_text = 0;
-    DevQ4Mfma text_mfma[2] = {};  // operand copies of fc1 and fc2
+    Q4Mfma text_mfma[2] = {};  // operand copies of fc1 and fc2
     bool text_mfma_ok = false;    // both are there
     float *tx_raw = nullptr, *tx_h = nullptr, *tx_rows = nullptr;
     float *pr_codec = nullptr;  // [8][hidden]: the prompt's codec rows and the voice row
@@ -854,9 +861,9 @@ struct qtts_predictor {
     uint64_t prog_kv = 0;  // serial of the cache prog was built for
     // MFMA operand copies for the batched loop: 4 per layer, the input
     // projection, the heads (made by the first batched call)
-    std::vector<DevQ4Mfma> mfma;
-    DevQ4Mfma mfma_in{};
-    std::vector<DevQ4Mfma> mfma_heads;
+    std::vector<Q4Mfma> mfma;
+    Q4Mfma mfma_in{};
+    std::vector<Q4Mfma> mfma_heads;
     int mfma_state = 0;  // 0 not tried, 1 made, -1 a weight cannot use the matrix cores
     // in_proj(emb[g][code]) + bias for every code of emb[0 .. groups-2]:
     // [groups-1][tab_rows][hidden], the engine's pass inputs by code
@@ -1393,7 +1400,7 @@ qtts_status make_predictor_tables(qtts_predictor *p) {
     // launches of kMaxM rows.
     const Stack &st = p->st;
     const int nqkv = st.nq * st.hd + 2 * st.nkv * st.hd;
-    DevQ4Mfma m_in{}, m_qkv{};
+    Q4Mfma m_in{}, m_qkv{};
     bool ok_in = false, ok_qkv = false;
     void *mem = nullptr;
     if (rows >= kMfmaMinRows) {
@@ -1988,12 +1995,12 @@ static qtts_status prefill_layers_rows(qtts_talker *t, qtts_kv *kv, int seq_len)
 // copies kept) when any weight cannot take the matrix-core path.
 static qtts_status make_talker_mfma(qtts_talker *t) {
     qtts_ctx *c = t->ctx;
-    std::vector<DevQ4Mfma> copies;
+    std::vector<Q4Mfma> copies;
     std::vector<void *> mems;
     bool all = true;
     for (const DevLayer &Ly : t->st.L) {
         for (const DevQ4 *w : {&Ly.qkv, &Ly.o, &Ly.gu, &Ly.down}) {
-            DevQ4Mfma m{};
+            Q4Mfma m{};
             void *mem = nullptr;
             bool ok = false;
             const qtts_status s = make_mfma_copy(c, *w, &mem, &m, &ok);
@@ -2035,7 +2042,7 @@ static qtts_status prefill_layers_mfma(qtts_talker *t, qtts_kv *kv, int seq_len)
     const int hidden = st.hidden, qd = st.nq * st.hd, nqkv = qd + 2 * st.nkv * st.hd;
     for (int l = 0; l < st.layers; l++) {
         const DevLayer &Ly = st.L[l];
-        const DevQ4Mfma *W = &t->mfma[(size_t)4 * l];
+        const Q4Mfma *W = &t->mfma[(size_t)4 * l];
         float *kc = kv->layer_k(l), *vc = kv->layer_v(l);
         QTTS_TRY(run_gemm_mfma(c, W[0], t->xp, seq_len, hidden, MFMA_ROWS_RMSNORM, Ly.in_g, t->rawp, nqkv, nullptr,
                                false));
@@ -4076,12 +4083,12 @@ struct RowTab {
     int stride = 1, pos0 = 0, kv0 = 0, cap = 0;
 };
 
-qtts_status make_stack_mfma(qtts_ctx *c, Owner &own, const Stack &st, std::vector<DevQ4Mfma> *out, bool *ok) {
+qtts_status make_stack_mfma(qtts_ctx *c, Owner &own, const Stack &st, std::vector<Q4Mfma> *out, bool *ok) {
     std::vector<void *> mems;
     *ok = true;
     for (const DevLayer &Ly : st.L)
         for (const DevQ4 *w : {&Ly.qkv, &Ly.o, &Ly.gu, &Ly.down}) {
-            DevQ4Mfma m{};
+            Q4Mfma m{};
             void *mem = nullptr;
             bool one = false;
             const qtts_status s = make_mfma_copy(c, *w, &mem, &m, &one);
@@ -4113,7 +4120,7 @@ qtts_status make_predictor_mfma(qtts_predictor *p) {
     bool ok = false;
     QTTS_TRY(make_stack_mfma(c, p->own, p->st, &p->mfma, &ok));
     std::vector<void *> mems;
-    auto one = [&](const DevQ4 &w, DevQ4Mfma *m) -> qtts_status {
+    auto one = [&](const DevQ4 &w, Q4Mfma *m) -> qtts_status {
         void *mem = nullptr;
         bool good = false;
         QTTS_TRY(make_mfma_copy(c, w, &mem, m, &good));
@@ -4122,7 +4129,7 @@ qtts_status make_predictor_mfma(qtts_predictor *p) {
         return QTTS_OK;
     };
     if (ok && !p->identity_proj) QTTS_TRY(one(p->in_proj, &p->mfma_in));
-    p->mfma_heads.assign((size_t)p->groups, DevQ4Mfma{});
+    p->mfma_heads.assign((size_t)p->groups, Q4Mfma{});
     for (int g = 0; ok && g < p->groups; g++) QTTS_TRY(one(p->heads[g], &p->mfma_heads[(size_t)g]));
     for (void *m : mems) p->own.ptrs.push_back(m);
     p->mfma_state = ok ? 1 : -1;
@@ -4132,7 +4139,7 @@ qtts_status make_predictor_mfma(qtts_predictor *p) {
 // One layer stack over M independent rows (per-row caches from R).
 // fused: every row is its stream's only new row, so the attention kernel
 // does k_qkv_rows' work itself (no row attends to another row's new K/V).
-qtts_status layers_batched(qtts_ctx *c, const Stack &st, const DevQ4Mfma *W, const RowTab &R, float *x, int M,
+qtts_status layers_batched(qtts_ctx *c, const Stack &st, const Q4Mfma *W, const RowTab &R, float *x, int M,
                            float *raw, float *q, float *a, int nsplit, bool fused) {
     const int hidden = st.hidden, qd = st.nq * st.hd, nqkv = qd + 2 * st.nkv * st.hd;
     if ((size_t)M * st.nq * nsplit * (st.hd + 2) > kAttnPartFloats || M * st.nkv > kAttnCounters)
@@ -4140,7 +4147,7 @@ qtts_status layers_batched(qtts_ctx *c, const Stack &st, const DevQ4Mfma *W, con
     if (!attn_split_fits(R.cap, nsplit)) return fail(c, QTTS_ESHAPE, "batched attention: a split exceeds the score buffer");
     for (int l = 0; l < st.layers; l++) {
         const DevLayer &Ly = st.L[l];
-        const DevQ4Mfma *Wl = W + (size_t)4 * l;
+        const Q4Mfma *Wl = W + (size_t)4 * l;
         const long long layer_off = (long long)l * st.nkv * R.cap * st.hd;
         QTTS_TRY(run_gemm_mfma(c, Wl[0], x, M, hidden, MFMA_ROWS_RMSNORM, Ly.in_g, raw, nqkv, nullptr, false));
         QkvRowsParams qp{};
@@ -4473,12 +4480,12 @@ qtts_status qtts_generate_codes_batch(qtts_talker *t, qtts_predictor *p, int32_t
             return QTTS_OK;
     };
     // every GEMM's scratch, reserved before capture
-    for (const DevQ4Mfma &w : t->mfma) QTTS_TRY(mfma_reserve(c, w));
+    for (const Q4Mfma &w : t->mfma) QTTS_TRY(mfma_reserve(c, w));
     QTTS_TRY(mfma_reserve(c, t->head_mfma));
     if (!talker_only) {
         if (!p->identity_proj) QTTS_TRY(mfma_reserve(c, p->mfma_in));
-        for (const DevQ4Mfma &w : p->mfma) QTTS_TRY(mfma_reserve(c, w));
-        for (const DevQ4Mfma &w : p->mfma_heads) QTTS_TRY(mfma_reserve(c, w));
+        for (const Q4Mfma &w : p->mfma) QTTS_TRY(mfma_reserve(c, w));
+        for (const Q4Mfma &w : p->mfma_heads) QTTS_TRY(mfma_reserve(c, w));
     }
     const bool use_graph = std::getenv("QTTS_NO_GRAPH") == nullptr;
     hipGraph_t graph = nullptr;

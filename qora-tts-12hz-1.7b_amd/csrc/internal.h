@@ -38,7 +38,6 @@ struct DevQ4Mfma {
     const uint32_t *wm;
     const uint16_t *sa, *sb;
     int K, N;
-    size_t scratch_x, scratch_part;  // the product's scratch at any number of rows (binary16 values, floats)
 };
 
 // Row prologues of the MFMA GEMM's input split.

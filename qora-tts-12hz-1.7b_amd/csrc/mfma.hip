@@ -467,10 +467,10 @@ __global__ __launch_bounds__(256) void k_gemm_mfma16(GemmMfmaParams P) {
 // block's A operands go through LDS once for its NW panels (two 16-row steps
 // per stage, double buffered).  Loads run two stages ahead, and everything
 // that is not an MFMA is issued between MFMAs.  Bound by the rows' operands
-// from the L2: 1064 rows, 2048 -> 12288, take 180 us, 297 TFLOP/s (892 of
-// binary16 MFMAs issued; a library binary16 product with as many MFMAs takes
-// 181), where 17 passes of k_gemm_mfma took 410; 1000 rows, 6144 -> 2048, 342
-// -> 113 us.
+// from the L2: 1064 rows, 2048 -> 12288, take 159 us with the row split, 337
+// TFLOP/s (1010 of binary16 MFMAs issued; a library binary16 product with as
+// many MFMAs takes 149), where 17 passes of k_gemm_mfma took 410; 1000 rows,
+// 6144 -> 2048, 342 -> 89 us (the library 189).
 template <int MT, int NW, bool FULL>
 __global__ __launch_bounds__(64 * NW, 2) void k_gemm_mfma_tile(GemmMfmaParams P, GemmTilePlan T) {
     constexpr int SS = 2;  // 16-row steps per stage
