@@ -1040,11 +1040,12 @@ __device__ __forceinline__ float dec_sin2(float t) {
 // to four taps ahead.  conv1's operand scale is a bound on SnakeBeta (per
 // element, dec_snake_bound) that x's producer recorded, as this unit records
 // the next one's.
-// C = 96, 960,000 positions: 1130 us as five launches, 607 to 636 here; C =
-// 192, 320,000 positions: 1060, 667 to 705; C = 384, 80,000: 810, 564 to 586.
+// C = 96, 960,000 positions: 1130 us as five launches, 622 here; C = 192,
+// 320,000 positions: 1060, 709; C = 384, 80,000: 810, 570 (averages of a
+// trace whose fastest launches take 592, 666 and 548).
 // Matrix cores a third busy, vector ALU (the sines and splits) a third, the
 // rest latency: one block a CU, and of the 168 registers that 12 waves leave
-// 3, 7 and 10 spill (96, 192 and 384 channels).  Blocks of 6 waves and half the
+// 0, 4 and 6 spill (96, 192 and 384 channels).  Blocks of 6 waves and half the
 // positions measured slower (C = 96, 805 us: twice the A operands through the
 // L2).
 template <int CT, int NWV>
@@ -1065,12 +1066,13 @@ __global__ __launch_bounds__(64 * NWV, 3) void k_dec_resunit(DecResUnitParams P)
     };
     __shared__ __align__(16) Lds sm;
     __shared__ float red[NWV];
-    __shared__ __align__(16) float next[2][C];  // oea, oeb: read in the epilogue, where nothing hides a load
+    __shared__ __align__(16) float last[3][C];  // b2, oea, oeb: read in the epilogue, where nothing hides a load (1 % of a decode)
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 31, half = lane >> 5;
-    if (P.omax && threadIdx.x < C) {
-        next[0][threadIdx.x] = P.oea[threadIdx.x];
-        next[1][threadIdx.x] = P.oeb[threadIdx.x];
+    if (threadIdx.x < C) {
+        last[0][threadIdx.x] = P.b2[threadIdx.x];
+        last[1][threadIdx.x] = P.omax ? P.oea[threadIdx.x] : 0.0f;
+        last[2][threadIdx.x] = P.omax ? P.oeb[threadIdx.x] : 0.0f;
     }
     const int tile = wave % CT, p0 = 64 * (wave / CT);  // this wave's channels and positions of the block
     const int n0 = blockIdx.x * NP, len = P.len, dil = P.dilation;
@@ -1258,9 +1260,9 @@ __global__ __launch_bounds__(64 * NWV, 3) void k_dec_resunit(DecResUnitParams P)
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const int c = 32 * tile + 8 * j + 4 * half;
-        const float4 b = *reinterpret_cast<const float4 *>(P.b2 + c);
+        const float4 b = *reinterpret_cast<const float4 *>(&last[0][c]);
         const float bv[4] = {b.x, b.y, b.z, b.w};
-        const float4 a = *reinterpret_cast<const float4 *>(&next[0][c]), e = *reinterpret_cast<const float4 *>(&next[1][c]);
+        const float4 a = *reinterpret_cast<const float4 *>(&last[1][c]), e = *reinterpret_cast<const float4 *>(&last[2][c]);
         const float av[4] = {a.x, a.y, a.z, a.w}, ev[4] = {e.x, e.y, e.z, e.w};
         float cm[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // the channels' largest |out|
 #pragma unroll
