@@ -31,7 +31,7 @@ def test_row_counts_allocate_nothing(K, N):
     for rows, x in xs.items():
         w.gemm_device(x.data_ptr(), rows, ys[rows].data_ptr())
     ctx.synchronize()
-    assert torch.cuda.mem_get_info()[0] == free
+    assert free - torch.cuda.mem_get_info()[0] < 2 ** 21  # 25 and 122 MB when each row count had its own
     w.gemm_device(xs[64].data_ptr(), 64, ys[64].data_ptr())
     ctx.synchronize()
     assert torch.equal(ys[64], first)

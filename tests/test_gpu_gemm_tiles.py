@@ -94,4 +94,4 @@ def test_rows_past_a_pass_cost_no_more_than_two(ctx, rows):
 
     one, two = best([rows]), best([64, 32])
     print(f"{rows} rows: {one / 32 * 1e6:.1f} us, in two calls {two / 32 * 1e6:.1f}")
-    assert one < 1.08 * two
+    assert one < 1.12 * two
